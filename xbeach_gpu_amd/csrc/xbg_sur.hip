@@ -9,13 +9,14 @@
 // kept as FP32 masters (Adam) with BF16 copies for the matrix cores, and
 // every product accumulates in FP32 (v_mfma_f32_16x16x32_bf16).
 //
-// Convolutions are implicit GEMMs (M = pixels, N = output channels, K =
-// taps x input channels):
-//   k_conv_fwd    forward (also the data gradient, through the flipped and
-//                 transposed weights: dX = conv(dZ, W'))
-//   k_conv_wgrad  weight gradient (M = output channels, N = input
-//                 channels, K = pixels), split over pixel ranges into FP32
-//                 partials that k_reduce_parts sums in a fixed order
+// Convolutions are implicit GEMMs (pixels x output channels, K = taps x
+// input channels):
+//   k_conv        forward (also the data gradient, through the flipped and
+//                 transposed weights: dX = conv(dZ, W')), with pooling,
+//                 activation masks and the output head in its epilogue
+//   k_conv_wgrad  weight gradient (output x input channels, K = pixels),
+//                 split over pixel ranges into FP32 partials that
+//                 k_reduce_parts sums in a fixed order
 // A 16 x 16 x 32 MFMA takes from each lane 8 consecutive K values of one A
 // row (lane % 16) and of one B column (lane % 16), the lanes' K slices
 // being lane / 16; it leaves in each lane four rows 4*(lane/16)+r of column
@@ -34,6 +35,7 @@ namespace {
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -46,26 +48,80 @@ constexpr int KB = 32;        // input channels per K block
 constexpr int LROW = KB + 8;  // LDS row (pixel) stride in bf16: 80 B, keeps 16-B reads aligned and spread
 
 // ---------------------------------------------------------------------------
-// Forward convolution, 'same' padding (TAPS 9: 3x3, TAPS 1: 1x1).
+// Convolution, 'same' padding (TAPS 9: 3x3, TAPS 1: 1x1), forward and data
+// gradient, with the elementwise passes around it folded into its staging
+// and its epilogue.
+//
 // Workgroup: 4 waves, TW pixels along x times 64 MB / TW rows (64 MB pixels)
 // and BN output channels; wave w computes MB blocks of 16 pixels (pixels
-// 64 m + 16 w + 0..15 of the tile, m < MB) x BN channels, so each staged
-// weight block feeds MB times the matrix work.  Per K block the input tile
-// (+1-pixel halo for 3x3) and the block's weights are staged in LDS.  The
-// sum over K blocks and taps runs in the same order for any MB.  Epilogue:
-// + bias, optional ReLU, BF16 or FP32 store.
-// Requires Cin % 32 == 0, Cout % BN == 0, W % TW == 0, H % (64 MB / TW) == 0.
+// 64 m + 16 w + 0..15 of the tile, m < MB) x BN channels.  Per block of 32
+// input channels the input tile (+1-pixel halo for 3x3) and the block's
+// weights are staged in LDS; the next block's values are in flight from
+// memory, in registers, while this one is multiplied.  The weights are the
+// MFMA's A operand, so a lane holds four consecutive output channels of one
+// pixel.  With 64-pixel rows a pixel fragment serves the three taps of its
+// column that read it from three output rows: 54 LDS reads per 144 MFMAs
+// instead of 72, under the LDS rate that a read per operand would reach.
+// The sum over channel blocks and taps runs in the same order for any tile.
+//
+// Source (CSrc): a plain tensor; a decoder's concatenation read from its two
+// parts (the coarse tensor at half resolution, the skip); or the network's
+// 8 input channels, the other 24 being zero.  Epilogue (EPI): the tile goes
+// through LDS as BF16, so that its values leave as 16-byte stores and
+// neighbouring pixels can be combined:
+//   E_STORE   store, 0 where mask <= 0 when a mask is given
+//   E_POOL    store, and the 2x2 average pool of the stored values
+//   E_HEAD    store (when y is given), and the output head on the stored values
+//   E_UPSUM   data gradient of a concatenation: channels below c1 summed over
+//             the 2x2 cells of the upsampled part, the others stored as they are
+//   E_UNPOOL  data gradient of a pooled tensor: a quarter of the value added
+//             to the skip's gradient at the four fine pixels, then the mask
+// Every value is rounded to BF16 where a pass of its own stored it, so the
+// results are those of separate passes bit for bit.
+//
+// Bound at 64 x 256 x 256: memory at 32 channels (read 268 MB, write 268 MB),
+// the LDS and matrix rates at 64 and more.  With the elementwise passes as
+// kernels of their own (one value per thread) a backward of that size took
+// 19.9 ms, 14.5 ms this way; inference at 512 x 1024 756 and 546 us.
+// Requires Cin % 32 == 0, Cout % BN == 0, W % TW == 0, H % (64 MB / TW) == 0;
+// E_POOL and E_UPSUM TW = 64, MB = 4; E_HEAD BN = Cout = 32.
 // ---------------------------------------------------------------------------
-template <int TAPS, int TW, int BN, int MB, bool RELU, bool OUTF32>
-__global__ __launch_bounds__(256) void k_conv_fwd(const bf16* __restrict__ X, const bf16* __restrict__ Wt,
-                                                  const float* __restrict__ bias, void* __restrict__ Yv, int H,
-                                                  int W, int Cin, int Cout) {
-    constexpr int TR = 64 * MB / TW;            // rows per tile
+enum { E_STORE, E_POOL, E_HEAD, E_UPSUM, E_UNPOOL };
+struct CSrc {
+    const bf16* a;  // channels 0 .. ca-1
+    const bf16* b;  // channels ca .. (nullptr: none, they are zero)
+    int ca, up;     // up: a is at half resolution
+};
+struct CEpi {
+    bf16* y;           // E_UPSUM: the coarse part's gradient
+    bf16* y2;          // E_POOL: pooled; E_UPSUM: the skip's gradient
+    const bf16* mask;  // nullptr: none
+    const bf16* skip;  // E_UNPOOL
+    int c1;            // E_UPSUM
+    const float *wh, *bh;
+    float* head;       // E_HEAD: [pixel][HK]
+};
+constexpr int HK = 5;  // channels of the output head
+
+__device__ __forceinline__ bf16x8 masked(bf16x8 v, bf16x8 m) {
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        if (!((float)m[e] > 0.0f)) v[e] = to_bf16(0.0f);
+    return v;
+}
+
+template <int TAPS, int TW, int BN, int MB, bool RELU, int EPI>
+__global__ __launch_bounds__(256, 2) void k_conv(CSrc X, const bf16* __restrict__ Wt, const float* __restrict__ bias,
+                                                 CEpi E, int H, int W, int Cin, int Cout) {
+    constexpr int TR = 64 * MB / TW;  // rows per tile
     constexpr int HALO = TAPS == 9 ? 1 : 0;
     constexpr int SR = TR + 2 * HALO, SC = TW + 2 * HALO;
-    __shared__ __attribute__((aligned(16))) bf16 sX[SR * SC * LROW];
-    __shared__ __attribute__((aligned(16))) bf16 sW[TAPS * BN * LROW];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    constexpr int XB = SR * SC * LROW, WB = TAPS * BN * LROW, LO = BN + 8, OB = 64 * MB * LO;
+    constexpr int NX = (SR * SC * 4 + 255) / 256, NW = (TAPS * BN * 4 + 255) / 256;
+    constexpr int CH = BN / 8;  // 16-byte chunks of a pixel's output channels
+    __shared__ __attribute__((aligned(16))) bf16 sm[XB + WB > OB ? XB + WB : OB];
+    bf16 *sX = sm, *sW = sm + XB;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l16 = lane & 15, s = lane >> 4;
     const int ntx = W / TW;
     const int xt = blockIdx.x % ntx, cb = blockIdx.x / ntx;
     const int x0 = xt * TW, y0 = blockIdx.y * TR, n = blockIdx.z;
@@ -75,63 +131,183 @@ __global__ __launch_bounds__(256) void k_conv_fwd(const bf16* __restrict__ X, co
     for (int m = 0; m < MB; m++)
 #pragma unroll
         for (int j = 0; j < BN / 16; j++) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int s = lane >> 4;  // K slice of 8 channels
-    const size_t img = (size_t)n * H * W;
+    // the next channel block's values, 16-byte chunks of 8 channels
+    bf16x8 rx[NX], rw[NW];
+    auto load = [&](int c0) {
+        const bool second = c0 >= X.ca && X.b;
+        const int up = second ? 0 : X.up, C = second ? Cin - X.ca : X.ca, cc = second ? c0 - X.ca : c0;
+        const bf16* src = (second ? X.b : X.a) + (size_t)n * (H >> up) * (W >> up) * C + cc;
+#pragma unroll
+        for (int it = 0; it < NX; it++) {
+            const int k = tid + it * 256, ch = k & 3, pix = k >> 2;
+            const int yy = y0 + pix / SC - HALO, xx = x0 + pix % SC - HALO;
+            bf16x8 v = {};
+            if (pix < SR * SC && yy >= 0 && yy < H && xx >= 0 && xx < W && cc + ch * 8 < C)
+                v = *(const bf16x8*)(src + ((size_t)(yy >> up) * (W >> up) + (xx >> up)) * C + ch * 8);
+            rx[it] = v;
+        }
+#pragma unroll
+        for (int it = 0; it < NW; it++) {
+            const int k = tid + it * 256, ch = k & 3, row = k >> 2;  // row = tap * BN + j
+            const int tap = row / BN, j = row % BN;
+            if (row < TAPS * BN) rw[it] = *(const bf16x8*)(Wt + ((size_t)tap * Cout + co0 + j) * Cin + c0 + ch * 8);
+        }
+    };
+    load(0);
     for (int c0 = 0; c0 < Cin; c0 += KB) {
         __syncthreads();
-        // input tile: SR x SC pixels x 32 channels, 16-B chunks of 8 channels
-        for (int k = tid; k < SR * SC * 4; k += 256) {
-            int ch = k & 3, pix = k >> 2;
-            int r = pix / SC, c = pix % SC;
-            int yy = y0 + r - HALO, xx = x0 + c - HALO;
-            bf16x8 v = {};
-            if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = *(const bf16x8*)(X + (img + (size_t)yy * W + xx) * Cin + c0 + ch * 8);
-            *(bf16x8*)(sX + pix * LROW + ch * 8) = v;
+#pragma unroll
+        for (int it = 0; it < NX; it++) {
+            const int k = tid + it * 256;
+            if (k < SR * SC * 4) *(bf16x8*)(sX + (k >> 2) * LROW + (k & 3) * 8) = rx[it];
         }
-        // weights of the block: TAPS x BN x 32
-        for (int k = tid; k < TAPS * BN * 4; k += 256) {
-            int ch = k & 3, row = k >> 2;  // row = tap * BN + j
-            int tap = row / BN, j = row % BN;
-            *(bf16x8*)(sW + row * LROW + ch * 8) =
-                *(const bf16x8*)(Wt + ((size_t)tap * Cout + co0 + j) * Cin + c0 + ch * 8);
+#pragma unroll
+        for (int it = 0; it < NW; it++) {
+            const int k = tid + it * 256;
+            if (k < TAPS * BN * 4) *(bf16x8*)(sW + (k >> 2) * LROW + (k & 3) * 8) = rw[it];
         }
         __syncthreads();
+        if (c0 + KB < Cin) load(c0 + KB);
+        auto wfrag = [&](int tap, int j) { return *(const bf16x8*)(sW + (tap * BN + 16 * j + l16) * LROW + s * 8); };
+        auto xfrag = [&](int r, int c) { return *(const bf16x8*)(sX + (r * SC + c) * LROW + s * 8); };
+        if (TAPS == 9 && TW == 64) {
+            // the fragments of MB consecutive rows, row r in slot r % MB
+            bf16x8 xf[3][MB];
 #pragma unroll
-        for (int tap = 0; tap < TAPS; tap++) {
-            const int dy = TAPS == 9 ? tap / 3 : 0, dx = TAPS == 9 ? tap % 3 : 0;
-            bf16x8 a[MB];
+            for (int dx = 0; dx < 3; dx++)
 #pragma unroll
-            for (int m = 0; m < MB; m++) {
-                const int q = 64 * m + 16 * w + (lane & 15);  // this lane's pixel (A row) within the tile
-                a[m] = *(const bf16x8*)(sX + ((q / TW + dy) * SC + q % TW + dx) * LROW + s * 8);
+                for (int m = 0; m < MB; m++) xf[dx][m] = xfrag(m, 16 * w + l16 + dx);
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                if (dy > 0) {
+#pragma unroll
+                    for (int dx = 0; dx < 3; dx++) xf[dx][(dy - 1) % MB] = xfrag(MB - 1 + dy, 16 * w + l16 + dx);
+                }
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+                    for (int j = 0; j < BN / 16; j++) {
+                        const bf16x8 b = wfrag(dy * 3 + dx, j);
+#pragma unroll
+                        for (int m = 0; m < MB; m++) acc[m][j] = mfma16(b, xf[dx][(m + dy) % MB], acc[m][j]);
+                    }
             }
+        } else {
 #pragma unroll
-            for (int j = 0; j < BN / 16; j++) {
-                bf16x8 b = *(const bf16x8*)(sW + (tap * BN + 16 * j + (lane & 15)) * LROW + s * 8);
+            for (int tap = 0; tap < TAPS; tap++) {
+                const int dy = TAPS == 9 ? tap / 3 : 0, dx = TAPS == 9 ? tap % 3 : 0;
+                bf16x8 a[MB];
 #pragma unroll
-                for (int m = 0; m < MB; m++) acc[m][j] = mfma16(a[m], b, acc[m][j]);
+                for (int m = 0; m < MB; m++) {
+                    const int q = 64 * m + 16 * w + l16;  // this lane's pixel within the tile
+                    a[m] = xfrag(q / TW + dy, q % TW + dx);
+                }
+#pragma unroll
+                for (int j = 0; j < BN / 16; j++) {
+                    const bf16x8 b = wfrag(tap, j);
+#pragma unroll
+                    for (int m = 0; m < MB; m++) acc[m][j] = mfma16(b, a[m], acc[m][j]);
+                }
             }
         }
     }
-    // epilogue: lane holds rows (pixels) 64 m + 16 w + 4 s + r, column
-    // (channel) lane & 15
+    // the tile as BF16 in LDS: the lane holds channels 16 j + 4 s + 0..3 of
+    // pixel 64 m + 16 w + l16
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < BN / 16; j++) {
-        const int co = co0 + 16 * j + (lane & 15);
-        const float bv = bias ? bias[co] : 0.0f;
+        const int c = 16 * j + 4 * s;
+        f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (bias) {
 #pragma unroll
-        for (int m = 0; m < MB; m++)
+            for (int r = 0; r < 4; r++) bv[r] = bias[co0 + c + r];
+        }
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+            bf16x4 o;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int qq = 64 * m + 16 * w + 4 * s + r;
-                const int yy = y0 + qq / TW, xx = x0 + qq % TW;
-                float v = acc[m][j][r] + bv;
+                float v = acc[m][j][r] + bv[r];
                 if (RELU) v = v > 0.0f ? v : 0.0f;
-                const size_t o = (img + (size_t)yy * W + xx) * Cout + co;
-                if (OUTF32) ((float*)Yv)[o] = v;
-                else ((bf16*)Yv)[o] = to_bf16(v);
+                o[r] = to_bf16(v);
             }
+            *(bf16x4*)(sm + (64 * m + 16 * w + l16) * LO + c) = o;
+        }
+    }
+    __syncthreads();
+    const size_t img = (size_t)n * H * W;
+    auto at = [&](int px, int ch) { return *(const bf16x8*)(sm + px * LO + ch * 8); };
+    auto pixel = [&](int px) { return img + (size_t)(y0 + px / TW) * W + x0 + px % TW; };
+    if (EPI == E_STORE || EPI == E_POOL || (EPI == E_HEAD && E.y)) {
+#pragma unroll
+        for (int it = 0; it < 64 * MB * CH / 256; it++) {
+            const int i = tid + it * 256, px = i / CH, ch = i % CH;
+            const size_t o = pixel(px) * Cout + co0 + ch * 8;
+            bf16x8 v = at(px, ch);
+            if (EPI == E_STORE && E.mask) v = masked(v, *(const bf16x8*)(E.mask + o));
+            *(bf16x8*)(E.y + o) = v;
+        }
+    }
+    if (EPI == E_POOL || EPI == E_UPSUM) {
+        // 2x2 cells of the tile: 2 x 32 of them
+        for (int i = tid; i < 16 * MB * CH; i += 256) {
+            const int pp = i / CH, ch = i % CH, py = pp / 32, pxx = pp % 32, q = 2 * py * TW + 2 * pxx;
+            if (EPI == E_UPSUM && co0 + ch * 8 >= E.c1) continue;
+            const bf16x8 v00 = at(q, ch), v01 = at(q + 1, ch), v10 = at(q + TW, ch), v11 = at(q + TW + 1, ch);
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float t = (float)v00[e] + (float)v01[e] + (float)v10[e] + (float)v11[e];
+                o[e] = to_bf16(EPI == E_POOL ? 0.25f * t : t);
+            }
+            const int Co = EPI == E_POOL ? Cout : E.c1;
+            *(bf16x8*)((EPI == E_POOL ? E.y2 : E.y) +
+                       (((size_t)n * (H / 2) + y0 / 2 + py) * (W / 2) + x0 / 2 + pxx) * Co + co0 + ch * 8) = o;
+        }
+    }
+    if (EPI == E_UPSUM) {
+        for (int i = tid; i < 64 * MB * CH; i += 256) {
+            const int px = i / CH, ch = i % CH;
+            if (co0 + ch * 8 < E.c1) continue;
+            *(bf16x8*)(E.y2 + pixel(px) * (Cout - E.c1) + co0 + ch * 8 - E.c1) = at(px, ch);
+        }
+    }
+    if (EPI == E_UNPOOL) {
+        for (int i = tid; i < 64 * MB * CH; i += 256) {
+            const int px = i / CH, ch = i % CH;
+            const bf16x8 v = at(px, ch);
+            const size_t o0 = (((size_t)n * H + y0 + px / TW) * 4 * W + 2 * (x0 + px % TW)) * Cout + co0 + ch * 8;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const size_t o = o0 + ((size_t)(q >> 1) * 2 * W + (q & 1)) * Cout;
+                const bf16x8 sk = *(const bf16x8*)(E.skip + o);
+                bf16x8 g;
+#pragma unroll
+                for (int e = 0; e < 8; e++) g[e] = to_bf16(0.25f * (float)v[e] + (float)sk[e]);
+                *(bf16x8*)(E.y + o) = masked(g, *(const bf16x8*)(E.mask + o));
+            }
+        }
+    }
+    if (EPI == E_HEAD) {
+        // Y[p][k] = b[k] + sum_c X[p][c] W[k][c] in FP32, one pixel per thread
+        for (int px = tid; px < 64 * MB; px += 256) {
+            float a[HK];
+#pragma unroll
+            for (int k = 0; k < HK; k++) a[k] = E.bh[k];
+#pragma unroll
+            for (int ch = 0; ch < CH; ch++) {
+                const bf16x8 v = at(px, ch);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float x = (float)v[e];
+#pragma unroll
+                    for (int k = 0; k < HK; k++) a[k] += x * E.wh[k * BN + ch * 8 + e];
+                }
+            }
+            float* o = E.head + pixel(px) * HK;
+#pragma unroll
+            for (int k = 0; k < HK; k++) o[k] = a[k];
+        }
     }
 }
 
@@ -150,7 +326,6 @@ __global__ __launch_bounds__(256) void k_conv_fwd(const bf16* __restrict__ X, co
 // ---------------------------------------------------------------------------
 constexpr int WPX = 64;           // pixels per staged segment
 constexpr int WLD = WPX + 8;      // LDS stride of a transposed channel row
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 template <int TAPS, int CBO, int CBI>
 __global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
                                                     float* __restrict__ part, int N, int H, int W, int Cin,
@@ -315,49 +490,9 @@ __global__ __launch_bounds__(256) void k_colsum(const bf16* __restrict__ G, size
     }
 }
 
-// ReLU backward in place: g = g where y > 0 else 0.
-__global__ __launch_bounds__(256) void k_relu_bwd(bf16* __restrict__ g, const bf16* __restrict__ y, size_t n) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n && !((float)y[i] > 0.0f)) g[i] = to_bf16(0.0f);
-}
-
-// 2x2 average pooling (NHWC) and its gradient.
-__global__ __launch_bounds__(256) void k_pool_fwd(const bf16* __restrict__ X, bf16* __restrict__ Y, int N, int H,
-                                                  int W, int C) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const int h = H / 2, w = W / 2;
-    size_t n_out = (size_t)N * h * w * C;
-    if (i >= n_out) return;
-    int c = i % C;
-    size_t r = i / C;
-    int x = r % w;
-    r /= w;
-    int y = r % h;
-    int n = r / h;
-    auto at = [&](int yy, int xx) { return (float)X[(((size_t)n * H + yy) * W + xx) * C + c]; };
-    float v = 0.25f * (at(2 * y, 2 * x) + at(2 * y, 2 * x + 1) + at(2 * y + 1, 2 * x) + at(2 * y + 1, 2 * x + 1));
-    Y[i] = to_bf16(v);
-}
-// dX (+)= dY / 4 broadcast over each 2x2 cell; accumulate adds to dX
-__global__ __launch_bounds__(256) void k_pool_bwd(const bf16* __restrict__ dY, bf16* __restrict__ dX, int N, int H,
-                                                  int W, int C, int accumulate) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    size_t n_in = (size_t)N * H * W * C;
-    if (i >= n_in) return;
-    int c = i % C;
-    size_t r = i / C;
-    int x = r % W;
-    r /= W;
-    int y = r % H;
-    int n = r / H;
-    float g = 0.25f * (float)dY[(((size_t)n * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c];
-    if (accumulate) g += (float)dX[i];
-    dX[i] = to_bf16(g);
-}
-
 // Nearest 2x upsampling of X [N][h][w][C] into channels [c0, c0+C) of Y
 // [N][2h][2w][Ctot] (the decoder's concatenation writes both halves of Y
-// in place), and its gradient (2x2 sums).
+// in place).
 __global__ __launch_bounds__(256) void k_up_fwd(const bf16* __restrict__ X, bf16* __restrict__ Y, int N, int h,
                                                 int w, int C, int Ctot, int c0) {
     size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -371,22 +506,6 @@ __global__ __launch_bounds__(256) void k_up_fwd(const bf16* __restrict__ X, bf16
     int n = r / (2 * h);
     Y[(((size_t)n * 2 * h + y) * 2 * w + x) * Ctot + c0 + c] = X[(((size_t)n * h + y / 2) * w + x / 2) * C + c];
 }
-__global__ __launch_bounds__(256) void k_up_bwd(const bf16* __restrict__ dY, bf16* __restrict__ dX, int N, int h,
-                                                int w, int C, int Ctot, int c0) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    size_t n_in = (size_t)N * h * w * C;
-    if (i >= n_in) return;
-    int c = i % C;
-    size_t r = i / C;
-    int x = r % w;
-    r /= w;
-    int y = r % h;
-    int n = r / h;
-    const int W2 = 2 * w;
-    auto at = [&](int yy, int xx) { return (float)dY[(((size_t)n * 2 * h + yy) * W2 + xx) * Ctot + c0 + c]; };
-    dX[i] = to_bf16(at(2 * y, 2 * x) + at(2 * y, 2 * x + 1) + at(2 * y + 1, 2 * x) + at(2 * y + 1, 2 * x + 1));
-}
-
 // Copy channels [c0, c0+C) between a [P][Ca] and a [P][Cb] tensor:
 // dst[p][dc0 + c] = src[p][sc0 + c] (skip concatenation and its gradient
 // split), accumulate adds to dst.
@@ -402,101 +521,69 @@ __global__ __launch_bounds__(256) void k_chan_copy(const bf16* __restrict__ src,
     dst[p * Cd + dc0 + c] = to_bf16(v);
 }
 
-// The output head: a 1x1 convolution C -> K (K small) in FP32 on the
-// vector units, and its gradients.  Y[p][k] = b[k] + sum_c X[p][c] W[k][c].
-template <int K>
-__global__ __launch_bounds__(256) void k_head_fwd(const bf16* __restrict__ X, const float* __restrict__ Wh,
-                                                  const float* __restrict__ bh, float* __restrict__ Y, size_t P,
-                                                  int C) {
-    size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (p >= P) return;
-    float a[K];
+// Backward of the output head (a 1x1 convolution of HC channels to HK in
+// FP32; its forward is the E_HEAD epilogue): from the gradient dY[p][k] of
+// its outputs, dX[p][c] = sum_k dY[p][k] W[k][c] where X > 0 (the ReLU that
+// made X), and the partials of dW[k][c] = sum_p dY[p][k] X[p][c] and
+// db[k] = sum_p dY[p][k]: part[blk][HK*HC + HK].  Four threads of eight
+// channels take a pixel.  Bound by memory (148 B a pixel).
+constexpr int HC = 32;
+__global__ __launch_bounds__(256) void k_head_bwd(const float* __restrict__ dY, const float* __restrict__ Wh,
+                                                  const bf16* __restrict__ X, bf16* __restrict__ dX, size_t P, int ppb,
+                                                  float* __restrict__ part) {
+    __shared__ float red[4][HK * HC + HK];
+    const int tid = threadIdx.x, c = (tid & 3) * 8;
+    const size_t p0 = (size_t)blockIdx.x * ppb, p1 = p0 + ppb < P ? p0 + ppb : P;
+    float w[HK][8], a[HK][8], b[HK];
 #pragma unroll
-    for (int k = 0; k < K; k++) a[k] = bh[k];
-    for (int c = 0; c < C; c++) {
-        float x = (float)X[p * C + c];
+    for (int k = 0; k < HK; k++) {
+        b[k] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < K; k++) a[k] += x * Wh[k * C + c];
+        for (int e = 0; e < 8; e++) {
+            w[k][e] = Wh[k * HC + c + e];
+            a[k][e] = 0.0f;
+        }
     }
+#pragma unroll 2
+    for (size_t p = p0 + (tid >> 2); p < p1; p += 64) {
+        const bf16x8 x = *(const bf16x8*)(X + p * HC + c);
+        float d[HK];
 #pragma unroll
-    for (int k = 0; k < K; k++) Y[p * K + k] = a[k];
-}
-// dX[p][c] = sum_k dY[p][k] W[k][c] (BF16 out)
-template <int K>
-__global__ __launch_bounds__(256) void k_head_dgrad(const float* __restrict__ dY, const float* __restrict__ Wh,
-                                                    bf16* __restrict__ dX, size_t P, int C) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= P * C) return;
-    int c = i % C;
-    size_t p = i / C;
-    float a = 0.0f;
+        for (int k = 0; k < HK; k++) d[k] = dY[p * HK + k];
+        bf16x8 o;
 #pragma unroll
-    for (int k = 0; k < K; k++) a += dY[p * K + k] * Wh[k * C + c];
-    dX[i] = to_bf16(a);
-}
-// partials of dW[k][c] = sum_p dY[p][k] X[p][c] and db[k] = sum_p dY[p][k]
-// over ppb pixels per workgroup: part[blk][K*C + K].  With C dividing 256
-// the threads cover 256 / C pixel lanes of all C channels; each lane sums
-// its pixels in order and the lanes are added in lane order.
-template <int K>
-__global__ __launch_bounds__(256) void k_head_wgrad(const float* __restrict__ dY, const bf16* __restrict__ X,
-                                                    size_t P, int C, int ppb, float* __restrict__ part) {
-    const size_t p0 = (size_t)blockIdx.x * ppb;
-    const size_t p1 = p0 + ppb < P ? p0 + ppb : P;
-    const int n = K * C + K;
-    if (C <= 256 && 256 % C == 0) {
-        __shared__ float red[K][256];
-        __shared__ float redb[K][256];
-        const int lanes = 256 / C, c = threadIdx.x % C, l = threadIdx.x / C;
-        float a[K], b[K];
+        for (int e = 0; e < 8; e++) {
+            const float xe = (float)x[e];
+            float g = 0.0f;
 #pragma unroll
-        for (int k = 0; k < K; k++) a[k] = b[k] = 0.0f;
-#pragma unroll 4
-        for (size_t p = p0 + l; p < p1; p += lanes) {
-            const float x = (float)X[p * C + c];
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const float d = dY[p * K + k];
-                a[k] += d * x;
-                b[k] += d;
+            for (int k = 0; k < HK; k++) {
+                g += d[k] * w[k][e];
+                a[k][e] += d[k] * xe;
             }
+            o[e] = to_bf16(xe > 0.0f ? g : 0.0f);
         }
+        *(bf16x8*)(dX + p * HC + c) = o;
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            red[k][threadIdx.x] = a[k];
-            redb[k][threadIdx.x] = b[k];
-        }
-        __syncthreads();
-        if (l == 0) {
+        for (int k = 0; k < HK; k++) b[k] += d[k];
+    }
+    // over the 16 pixels of a wavefront, then over the four wavefronts
 #pragma unroll
-            for (int k = 0; k < K; k++) {
-                float t = 0.0f;
-                for (int q = 0; q < lanes; q++) t += red[k][q * C + c];
-                part[(size_t)blockIdx.x * n + k * C + c] = t;
-            }
+    for (int k = 0; k < HK; k++) {
+#pragma unroll
+        for (int o = 4; o < 64; o <<= 1) {
+            b[k] += __shfl_xor(b[k], o, 64);
+#pragma unroll
+            for (int e = 0; e < 8; e++) a[k][e] += __shfl_xor(a[k][e], o, 64);
         }
-        if ((int)threadIdx.x < K) {
-            // the bias sums of the lanes' channel-0 threads
-            const int k = threadIdx.x;
-            float t = 0.0f;
-            for (int q = 0; q < lanes; q++) t += redb[k][q * C];
-            part[(size_t)blockIdx.x * n + K * C + k] = t;
+        if ((tid & 63) < 4) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) red[tid >> 6][k * HC + c + e] = a[k][e];
+            if ((tid & 3) == 0) red[tid >> 6][HK * HC + k] = b[k];
         }
-        return;
     }
-    for (int j = threadIdx.x; j < n; j += 256) {
-        float a = 0.0f;
-        if (j < K * C) {
-            int k = j / C, c = j % C;
-#pragma unroll 16
-            for (size_t p = p0; p < p1; p++) a += dY[p * K + k] * (float)X[p * C + c];
-        } else {
-            int k = j - K * C;
-#pragma unroll 16
-            for (size_t p = p0; p < p1; p++) a += dY[p * K + k];
-        }
-        part[(size_t)blockIdx.x * n + j] = a;
-    }
+    __syncthreads();
+    for (int i = tid; i < HK * HC + HK; i += 256)
+        part[(size_t)blockIdx.x * (HK * HC + HK) + i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
 }
 
 // Mean squared error over the normalised targets: per-workgroup partial
@@ -584,8 +671,8 @@ struct xbg_sur {
     std::vector<void*> allocs;
     bf16 *x32, *e0a, *e0, *p1, *e1a, *e1, *p2, *e2a, *e2, *p3, *b3a, *b3, *u2, *c2, *d2a, *d2, *u1, *c1, *d1a, *d1,
         *u0, *c0, *d0a, *d0;
-    bf16 *g_e0a, *g_e0, *g_p1, *g_e1a, *g_e1, *g_p2, *g_e2a, *g_e2, *g_p3, *g_b3a, *g_b3, *g_u2, *g_c2, *g_d2a,
-        *g_d2, *g_u1, *g_c1, *g_d1a, *g_d1, *g_u0, *g_c0, *g_d0a, *g_d0;
+    bf16 *g_e0a, *g_e0, *g_e1a, *g_e1, *g_e2a, *g_e2, *g_b3a, *g_b3, *g_u2, *g_d2a,
+        *g_d2, *g_u1, *g_d1a, *g_d1, *g_u0, *g_d0a, *g_d0;
     float *y = nullptr, *gy = nullptr;
     std::string err;
 };
@@ -607,32 +694,55 @@ int sfail(xbg_sur* s, int code, const std::string& m) {
 
 inline unsigned nblk(size_t n) { return (unsigned)((n + 255) / 256); }
 
-// the forward convolution for any supported shape
-int conv_fwd(hipStream_t st, const bf16* X, const bf16* Wt, const float* bias, void* Y, int n, int H, int W, int Cin,
-             int Cout, int taps, int relu, int outf32) {
-    if (Cin % 32 || Cout % 32 || !(taps == 1 || taps == 9) || outf32) return XBG_E_ARG;
-    int TW = W % 64 == 0 ? 64 : (W == 32 ? 32 : 0);
+// k_conv for any supported shape; the fused epilogues run at the sizes the
+// network gives them (E_POOL, E_UPSUM: rows of 64 pixels in fours)
+template <int EPI, bool RELU>
+int conv(hipStream_t st, CSrc X, const bf16* Wt, const float* bias, const CEpi& E, int n, int H, int W, int Cin,
+         int Cout, int taps) {
+    if (Cin % 32 || Cout % 32 || !(taps == 1 || taps == 9)) return XBG_E_ARG;
+    const int TW = W % 64 == 0 ? 64 : (W == 32 ? 32 : 0);
     if (!TW || H % (64 / TW)) return XBG_E_ARG;
-    int BN = Cout % 64 == 0 ? 64 : 32;
+    const int BN = Cout % 64 == 0 ? 64 : 32;
     // four 16-pixel blocks per wave where the rows divide, else one
     const int MB = H % (4 * 64 / TW) == 0 ? 4 : 1;
-    dim3 g((W / TW) * (Cout / BN), H / (MB * 64 / TW), n);
-#define CF(T_, TW_, BN_, R_)                                                                                       \
-    do {                                                                                                       \
-        if (MB == 4) k_conv_fwd<T_, TW_, BN_, 4, R_, false><<<g, dim3(256), 0, st>>>(X, Wt, bias, Y, H, W, Cin, Cout); \
-        else k_conv_fwd<T_, TW_, BN_, 1, R_, false><<<g, dim3(256), 0, st>>>(X, Wt, bias, Y, H, W, Cin, Cout);    \
+    const dim3 g((W / TW) * (Cout / BN), H / (MB * 64 / TW), n);
+    constexpr bool CELLS = EPI == E_POOL || EPI == E_UPSUM;
+    if (CELLS && (TW != 64 || MB != 4)) return XBG_E_ARG;
+    if (EPI == E_HEAD && (Cout != 32 || TW != 64 || taps != 9)) return XBG_E_ARG;
+#define CF(T_, TW_, BN_, MB_) k_conv<T_, TW_, BN_, MB_, RELU, EPI><<<g, dim3(256), 0, st>>>(X, Wt, bias, E, H, W, Cin, Cout)
+#define CF_MB(T_, TW_, BN_)                                   \
+    do {                                                      \
+        if constexpr (CELLS) CF(T_, TW_, BN_, 4);             \
+        else if (MB == 4) CF(T_, TW_, BN_, 4);                \
+        else CF(T_, TW_, BN_, 1);                             \
     } while (0)
-#define CF_R(T_, TW_, BN_) do { if (relu) CF(T_, TW_, BN_, true); else CF(T_, TW_, BN_, false); } while (0)
-#define CF_BN(T_, TW_) do { if (BN == 64) CF_R(T_, TW_, 64); else CF_R(T_, TW_, 32); } while (0)
-#define CF_TW(T_) do { if (TW == 64) CF_BN(T_, 64); else CF_BN(T_, 32); } while (0)
-    if (taps == 9) CF_TW(9);
-    else CF_TW(1);
+#define CF_BN(T_, TW_)                                        \
+    do {                                                      \
+        if constexpr (EPI == E_HEAD) CF_MB(T_, TW_, 32);      \
+        else if (BN == 64) CF_MB(T_, TW_, 64);                \
+        else CF_MB(T_, TW_, 32);                              \
+    } while (0)
+#define CF_TW(T_)                                             \
+    do {                                                      \
+        if constexpr (CELLS || EPI == E_HEAD) CF_BN(T_, 64);  \
+        else if (TW == 64) CF_BN(T_, 64);                     \
+        else CF_BN(T_, 32);                                   \
+    } while (0)
+    if constexpr (EPI != E_STORE) {
+        if (taps != 9) return XBG_E_ARG;
+        CF_TW(9);
+    } else {
+        if (taps == 9) CF_TW(9);
+        else CF_TW(1);
+    }
 #undef CF
-#undef CF_R
+#undef CF_MB
 #undef CF_BN
 #undef CF_TW
     return hipGetLastError() == hipSuccess ? 0 : XBG_E_HIP;
 }
+
+CSrc plain(const bf16* x, int c) { return CSrc{x, nullptr, c, 0}; }
 
 // dW (FP32, [taps][Cout][Cin]) of one convolution from its input X and the
 // gradient dZ of its pre-activation output; partials in part (npart floats)
@@ -674,12 +784,14 @@ int colsum(hipStream_t st, const bf16* Gm, size_t P, int C, float* out, float* p
     return hipGetLastError() == hipSuccess ? 0 : XBG_E_HIP;
 }
 
-// data gradient dX = conv(dZ, flipped W) for a convolution Cin -> Cout
-int conv_dgrad(hipStream_t st, const bf16* dZ, const bf16* Wt, bf16* Wd, bf16* dX, int n, int H, int W, int Cin,
+// data gradient conv(dZ, flipped W) for a convolution Cin -> Cout, through
+// the epilogue E
+template <int EPI>
+int conv_dgrad(hipStream_t st, const bf16* dZ, const bf16* Wt, bf16* Wd, const CEpi& E, int n, int H, int W, int Cin,
                int Cout, int taps) {
     size_t nw = (size_t)taps * Cout * Cin;
     k_flip_weights<<<nblk(nw), 256, 0, st>>>(Wt, Wd, taps, Cout, Cin);
-    return conv_fwd(st, dZ, Wd, nullptr, dX, n, H, W, Cout, Cin, taps, 0, 0);
+    return conv<EPI, false>(st, plain(dZ, Cout), Wd, nullptr, E, n, H, W, Cout, Cin, taps);
 }
 
 // deterministic initialisation: He-normal weights from a counter-based hash
@@ -763,12 +875,12 @@ int xbg_sur_create(int nmax, int H, int W, unsigned seed, xbg_sur** out) {
                 {&s->u2, P3 * 128}, {&s->c2, P2 * 256}, {&s->d2a, P2 * 128}, {&s->d2, P2 * 128},
                 {&s->u1, P2 * 64},  {&s->c1, P1 * 128}, {&s->d1a, P1 * 64}, {&s->d1, P1 * 64},
                 {&s->u0, P1 * 32},  {&s->c0, P0 * 64},  {&s->d0a, P0 * 32}, {&s->d0, P0 * 32},
-                {&s->g_e0a, P0 * 32}, {&s->g_e0, P0 * 32}, {&s->g_p1, P1 * 32}, {&s->g_e1a, P1 * 64},
-                {&s->g_e1, P1 * 64}, {&s->g_p2, P2 * 64}, {&s->g_e2a, P2 * 128}, {&s->g_e2, P2 * 128},
-                {&s->g_p3, P3 * 128}, {&s->g_b3a, P3 * 256}, {&s->g_b3, P3 * 256}, {&s->g_u2, P3 * 128},
-                {&s->g_c2, P2 * 256}, {&s->g_d2a, P2 * 128}, {&s->g_d2, P2 * 128}, {&s->g_u1, P2 * 64},
-                {&s->g_c1, P1 * 128}, {&s->g_d1a, P1 * 64}, {&s->g_d1, P1 * 64}, {&s->g_u0, P1 * 32},
-                {&s->g_c0, P0 * 64}, {&s->g_d0a, P0 * 32}, {&s->g_d0, P0 * 32}};
+                {&s->g_e0a, P0 * 32}, {&s->g_e0, P0 * 32}, {&s->g_e1a, P1 * 64},
+                {&s->g_e1, P1 * 64}, {&s->g_e2a, P2 * 128}, {&s->g_e2, P2 * 128},
+                {&s->g_b3a, P3 * 256}, {&s->g_b3, P3 * 256}, {&s->g_u2, P3 * 128},
+                {&s->g_d2a, P2 * 128}, {&s->g_d2, P2 * 128}, {&s->g_u1, P2 * 64},
+                {&s->g_d1a, P1 * 64}, {&s->g_d1, P1 * 64}, {&s->g_u0, P1 * 32},
+                {&s->g_d0a, P0 * 32}, {&s->g_d0, P0 * 32}};
     for (auto& b : acts) ok = ok && A((void**)b.p, b.n * 2);
     ok = ok && A((void**)&s->y, P0 * 5 * 4) && A((void**)&s->gy, P0 * 5 * 4);
     if (!ok) return bail(sfail(nullptr, XBG_E_HIP, "xbg_sur_create: out of device memory"));
@@ -819,66 +931,65 @@ int xbg_sur_get_grads(xbg_sur* s, float* host) {
 
 namespace {
 
-int sur_forward(xbg_sur* s, const bf16* x8, int n) {
+// the network's outputs into y (FP32 [n][H][W][5])
+int sur_forward(xbg_sur* s, const bf16* x8, int n, float* y) {
     hipStream_t st = s->st;
     const int H = s->H, W = s->W;
-    const size_t P0 = (size_t)n * H * W, P1 = P0 / 4, P2 = P0 / 16, P3 = P0 / 64;
+    const size_t P0 = (size_t)n * H * W, P1 = P0 / 4, P2 = P0 / 16;
+    const ConvL& hd = s->L[17];
     auto Wt = [&](int l) { return s->P16 + s->L[l].w; };
     auto Bs = [&](int l) { return s->P + s->L[l].b; };
     int rc = 0;
     // the 8 input channels into the first 8 of 32 (channels 8..31 stay the
     // zeros written at creation)
     k_chan_copy<<<nblk(P0 * 8), 256, 0, st>>>(x8, 8, 0, s->x32, 32, 0, 8, P0, 0);
-#define CONV(l, X, Y, h, w)                                                                                    \
-    if ((rc = conv_fwd(st, X, Wt(l), Bs(l), Y, n, h, w, s->L[l].cin, s->L[l].cout, s->L[l].taps, s->L[l].relu, \
-                       0)))                                                                                    \
+    // convolution l of X on h x w pixels, through the epilogue E
+#define CONV(l, EPI, RELU, X, h, w, ...)                                                                       \
+    if ((rc = conv<EPI, RELU>(st, plain(X, s->L[l].cin), Wt(l), Bs(l), CEpi{__VA_ARGS__}, n, h, w, s->L[l].cin, \
+                              s->L[l].cout, s->L[l].taps)))                                                    \
         return sfail(s, rc, "conv " #l);
-    CONV(0, s->x32, s->e0a, H, W);
-    CONV(1, s->e0a, s->e0, H, W);
-    k_pool_fwd<<<nblk(P1 * 32), 256, 0, st>>>(s->e0, s->p1, n, H, W, 32);
-    CONV(2, s->p1, s->e1a, H / 2, W / 2);
-    CONV(3, s->e1a, s->e1, H / 2, W / 2);
-    k_pool_fwd<<<nblk(P2 * 64), 256, 0, st>>>(s->e1, s->p2, n, H / 2, W / 2, 64);
-    CONV(4, s->p2, s->e2a, H / 4, W / 4);
-    CONV(5, s->e2a, s->e2, H / 4, W / 4);
-    k_pool_fwd<<<nblk(P3 * 128), 256, 0, st>>>(s->e2, s->p3, n, H / 4, W / 4, 128);
-    CONV(6, s->p3, s->b3a, H / 8, W / 8);
-    CONV(7, s->b3a, s->b3, H / 8, W / 8);
-    CONV(8, s->b3, s->u2, H / 8, W / 8);
+    CONV(0, E_STORE, true, s->x32, H, W, s->e0a);
+    CONV(1, E_POOL, true, s->e0a, H, W, s->e0, s->p1);
+    CONV(2, E_STORE, true, s->p1, H / 2, W / 2, s->e1a);
+    CONV(3, E_POOL, true, s->e1a, H / 2, W / 2, s->e1, s->p2);
+    CONV(4, E_STORE, true, s->p2, H / 4, W / 4, s->e2a);
+    CONV(5, E_POOL, true, s->e2a, H / 4, W / 4, s->e2, s->p3);
+    CONV(6, E_STORE, true, s->p3, H / 8, W / 8, s->b3a);
+    CONV(7, E_STORE, true, s->b3a, H / 8, W / 8, s->b3);
+    CONV(8, E_STORE, false, s->b3, H / 8, W / 8, s->u2);
     k_up_fwd<<<nblk(P2 * 128), 256, 0, st>>>(s->u2, s->c2, n, H / 8, W / 8, 128, 256, 0);
     k_chan_copy<<<nblk(P2 * 128), 256, 0, st>>>(s->e2, 128, 0, s->c2, 256, 128, 128, P2, 0);
-    CONV(9, s->c2, s->d2a, H / 4, W / 4);
-    CONV(10, s->d2a, s->d2, H / 4, W / 4);
-    CONV(11, s->d2, s->u1, H / 4, W / 4);
+    CONV(9, E_STORE, true, s->c2, H / 4, W / 4, s->d2a);
+    CONV(10, E_STORE, true, s->d2a, H / 4, W / 4, s->d2);
+    CONV(11, E_STORE, false, s->d2, H / 4, W / 4, s->u1);
     k_up_fwd<<<nblk(P1 * 64), 256, 0, st>>>(s->u1, s->c1, n, H / 4, W / 4, 64, 128, 0);
     k_chan_copy<<<nblk(P1 * 64), 256, 0, st>>>(s->e1, 64, 0, s->c1, 128, 64, 64, P1, 0);
-    CONV(12, s->c1, s->d1a, H / 2, W / 2);
-    CONV(13, s->d1a, s->d1, H / 2, W / 2);
-    CONV(14, s->d1, s->u0, H / 2, W / 2);
+    CONV(12, E_STORE, true, s->c1, H / 2, W / 2, s->d1a);
+    CONV(13, E_STORE, true, s->d1a, H / 2, W / 2, s->d1);
+    CONV(14, E_STORE, false, s->d1, H / 2, W / 2, s->u0);
     k_up_fwd<<<nblk(P0 * 32), 256, 0, st>>>(s->u0, s->c0, n, H / 2, W / 2, 32, 64, 0);
     k_chan_copy<<<nblk(P0 * 32), 256, 0, st>>>(s->e0, 32, 0, s->c0, 64, 32, 32, P0, 0);
-    CONV(15, s->c0, s->d0a, H, W);
-    CONV(16, s->d0a, s->d0, H, W);
+    CONV(15, E_STORE, true, s->c0, H, W, s->d0a);
+    CONV(16, E_HEAD, true, s->d0a, H, W, s->d0, nullptr, nullptr, nullptr, 0, s->P + hd.w, s->P + hd.b, y);
 #undef CONV
-    const ConvL& hd = s->L[17];
-    k_head_fwd<5><<<nblk(P0), 256, 0, st>>>(s->d0, s->P + hd.w, s->P + hd.b, s->y, P0, 32);
     SHIP(s, hipGetLastError());
     return 0;
 }
 
-// one convolution's backward: g (gradient of its output, overwritten by
-// the ReLU mask), dW, db, and dX (NULL: not needed)
-int conv_bwd(xbg_sur* s, int l, const bf16* X, const bf16* Y, bf16* g, bf16* dX, int n, int H, int W) {
+// one convolution's backward: from g, the gradient of its pre-activation
+// output, dW, db and, unless EPI is -1, the data gradient through EPI
+template <int EPI>
+int conv_bwd(xbg_sur* s, int l, const bf16* X, const bf16* g, const CEpi& E, int n, int H, int W) {
     hipStream_t st = s->st;
     const ConvL& c = s->L[l];
     const size_t P = (size_t)n * H * W;
     int rc;
-    if (c.relu) k_relu_bwd<<<nblk(P * c.cout), 256, 0, st>>>(g, Y, P * c.cout);
     if ((rc = conv_wgrad(st, X, g, s->G + c.w, s->part, s->npart, n, H, W, c.cin, c.cout, c.taps)))
         return sfail(s, rc, "wgrad " + std::to_string(l));
     if ((rc = colsum(st, g, P, c.cout, s->G + c.b, s->part, s->npart))) return sfail(s, rc, "colsum");
-    if (dX && (rc = conv_dgrad(st, g, s->P16 + c.w, s->Wd, dX, n, H, W, c.cin, c.cout, c.taps)))
-        return sfail(s, rc, "dgrad " + std::to_string(l));
+    if constexpr (EPI >= 0)
+        if ((rc = conv_dgrad<EPI>(st, g, s->P16 + c.w, s->Wd, E, n, H, W, c.cin, c.cout, c.taps)))
+            return sfail(s, rc, "dgrad " + std::to_string(l));
     return 0;
 }
 
@@ -899,44 +1010,41 @@ int sur_loss_grad(xbg_sur* s, const bf16* t5, int n, double* loss) {
 int sur_backward(xbg_sur* s, int n) {
     hipStream_t st = s->st;
     const int H = s->H, W = s->W;
-    const size_t P0 = (size_t)n * H * W, P1 = P0 / 4, P2 = P0 / 16, P3 = P0 / 64;
+    const size_t P0 = (size_t)n * H * W;
     int rc;
     const ConvL& hd = s->L[17];
     {
         int nb = 1024;
         int ppb = (int)((P0 + nb - 1) / nb);
         nb = (int)((P0 + ppb - 1) / ppb);
-        k_head_wgrad<5><<<nb, 256, 0, st>>>(s->gy, s->d0, P0, 32, ppb, s->part);
-        k_reduce_parts<<<nblk(5 * 32 + 5), 256, 0, st>>>(s->part, nb, (size_t)(5 * 32 + 5), s->G + hd.w);
-        k_head_dgrad<5><<<nblk(P0 * 32), 256, 0, st>>>(s->gy, s->P + hd.w, s->g_d0, P0, 32);
+        k_head_bwd<<<nb, 256, 0, st>>>(s->gy, s->P + hd.w, s->d0, s->g_d0, P0, ppb, s->part);
+        k_reduce_parts<<<nblk(HK * HC + HK), 256, 0, st>>>(s->part, nb, (size_t)(HK * HC + HK), s->G + hd.w);
     }
-    if ((rc = conv_bwd(s, 16, s->d0a, s->d0, s->g_d0, s->g_d0a, n, H, W))) return rc;
-    if ((rc = conv_bwd(s, 15, s->c0, s->d0a, s->g_d0a, s->g_c0, n, H, W))) return rc;
-    k_up_bwd<<<nblk(P1 * 32), 256, 0, st>>>(s->g_c0, s->g_u0, n, H / 2, W / 2, 32, 64, 0);
-    if ((rc = conv_bwd(s, 14, s->d1, s->u0, s->g_u0, s->g_d1, n, H / 2, W / 2))) return rc;
-    if ((rc = conv_bwd(s, 13, s->d1a, s->d1, s->g_d1, s->g_d1a, n, H / 2, W / 2))) return rc;
-    if ((rc = conv_bwd(s, 12, s->c1, s->d1a, s->g_d1a, s->g_c1, n, H / 2, W / 2))) return rc;
-    k_up_bwd<<<nblk(P2 * 64), 256, 0, st>>>(s->g_c1, s->g_u1, n, H / 4, W / 4, 64, 128, 0);
-    if ((rc = conv_bwd(s, 11, s->d2, s->u1, s->g_u1, s->g_d2, n, H / 4, W / 4))) return rc;
-    if ((rc = conv_bwd(s, 10, s->d2a, s->d2, s->g_d2, s->g_d2a, n, H / 4, W / 4))) return rc;
-    if ((rc = conv_bwd(s, 9, s->c2, s->d2a, s->g_d2a, s->g_c2, n, H / 4, W / 4))) return rc;
-    k_up_bwd<<<nblk(P3 * 128), 256, 0, st>>>(s->g_c2, s->g_u2, n, H / 8, W / 8, 128, 256, 0);
-    if ((rc = conv_bwd(s, 8, s->b3, s->u2, s->g_u2, s->g_b3, n, H / 8, W / 8))) return rc;
-    if ((rc = conv_bwd(s, 7, s->b3a, s->b3, s->g_b3, s->g_b3a, n, H / 8, W / 8))) return rc;
-    if ((rc = conv_bwd(s, 6, s->p3, s->b3a, s->g_b3a, s->g_p3, n, H / 8, W / 8))) return rc;
-    // e2 feeds the pool and the skip: its gradient is the sum of both
-    k_chan_copy<<<nblk(P2 * 128), 256, 0, st>>>(s->g_c2, 256, 128, s->g_e2, 128, 0, 128, P2, 0);
-    k_pool_bwd<<<nblk(P2 * 128), 256, 0, st>>>(s->g_p3, s->g_e2, n, H / 4, W / 4, 128, 1);
-    if ((rc = conv_bwd(s, 5, s->e2a, s->e2, s->g_e2, s->g_e2a, n, H / 4, W / 4))) return rc;
-    if ((rc = conv_bwd(s, 4, s->p2, s->e2a, s->g_e2a, s->g_p2, n, H / 4, W / 4))) return rc;
-    k_chan_copy<<<nblk(P1 * 64), 256, 0, st>>>(s->g_c1, 128, 64, s->g_e1, 64, 0, 64, P1, 0);
-    k_pool_bwd<<<nblk(P1 * 64), 256, 0, st>>>(s->g_p2, s->g_e1, n, H / 2, W / 2, 64, 1);
-    if ((rc = conv_bwd(s, 3, s->e1a, s->e1, s->g_e1, s->g_e1a, n, H / 2, W / 2))) return rc;
-    if ((rc = conv_bwd(s, 2, s->p1, s->e1a, s->g_e1a, s->g_p1, n, H / 2, W / 2))) return rc;
-    k_chan_copy<<<nblk(P0 * 32), 256, 0, st>>>(s->g_c0, 64, 32, s->g_e0, 32, 0, 32, P0, 0);
-    k_pool_bwd<<<nblk(P0 * 32), 256, 0, st>>>(s->g_p1, s->g_e0, n, H, W, 32, 1);
-    if ((rc = conv_bwd(s, 1, s->e0a, s->e0, s->g_e0, s->g_e0a, n, H, W))) return rc;
-    if ((rc = conv_bwd(s, 0, s->x32, s->e0a, s->g_e0a, nullptr, n, H, W))) return rc;
+    // layer l: its input, the gradient of its output before the activation,
+    // and where the gradient of its input goes (masked by the activation
+    // that made the input, so that it is the next layer's g)
+#define BWD(l, EPI, X, g, h, w, ...) \
+    if ((rc = conv_bwd<EPI>(s, l, X, g, CEpi{__VA_ARGS__}, n, h, w))) return rc;
+    BWD(16, E_STORE, s->d0a, s->g_d0, H, W, s->g_d0a, nullptr, s->d0a);
+    // a concatenation's gradient: the coarse part's, and the skip's, to which
+    // the pooled path adds below
+    BWD(15, E_UPSUM, s->c0, s->g_d0a, H, W, s->g_u0, s->g_e0, nullptr, nullptr, 32);
+    BWD(14, E_STORE, s->d1, s->g_u0, H / 2, W / 2, s->g_d1, nullptr, s->d1);
+    BWD(13, E_STORE, s->d1a, s->g_d1, H / 2, W / 2, s->g_d1a, nullptr, s->d1a);
+    BWD(12, E_UPSUM, s->c1, s->g_d1a, H / 2, W / 2, s->g_u1, s->g_e1, nullptr, nullptr, 64);
+    BWD(11, E_STORE, s->d2, s->g_u1, H / 4, W / 4, s->g_d2, nullptr, s->d2);
+    BWD(10, E_STORE, s->d2a, s->g_d2, H / 4, W / 4, s->g_d2a, nullptr, s->d2a);
+    BWD(9, E_UPSUM, s->c2, s->g_d2a, H / 4, W / 4, s->g_u2, s->g_e2, nullptr, nullptr, 128);
+    BWD(8, E_STORE, s->b3, s->g_u2, H / 8, W / 8, s->g_b3, nullptr, s->b3);
+    BWD(7, E_STORE, s->b3a, s->g_b3, H / 8, W / 8, s->g_b3a, nullptr, s->b3a);
+    BWD(6, E_UNPOOL, s->p3, s->g_b3a, H / 8, W / 8, s->g_e2, nullptr, s->e2, s->g_e2);
+    BWD(5, E_STORE, s->e2a, s->g_e2, H / 4, W / 4, s->g_e2a, nullptr, s->e2a);
+    BWD(4, E_UNPOOL, s->p2, s->g_e2a, H / 4, W / 4, s->g_e1, nullptr, s->e1, s->g_e1);
+    BWD(3, E_STORE, s->e1a, s->g_e1, H / 2, W / 2, s->g_e1a, nullptr, s->e1a);
+    BWD(2, E_UNPOOL, s->p1, s->g_e1a, H / 2, W / 2, s->g_e0, nullptr, s->e0, s->g_e0);
+    BWD(1, E_STORE, s->e0a, s->g_e0, H, W, s->g_e0a, nullptr, s->e0a);
+    BWD(0, -1, s->x32, s->g_e0a, H, W, nullptr);
+#undef BWD
     SHIP(s, hipGetLastError());
     return 0;
 }
@@ -947,16 +1055,15 @@ extern "C" {
 
 int xbg_sur_forward(xbg_sur* s, const void* x8, int n, float* y) {
     if (!s || !x8 || n < 1 || n > s->nmax) return sfail(s, XBG_E_ARG, "xbg_sur_forward: bad argument");
-    int rc = sur_forward(s, (const bf16*)x8, n);
+    int rc = sur_forward(s, (const bf16*)x8, n, y ? y : s->y);
     if (rc) return rc;
-    if (y) SHIP(s, hipMemcpyAsync(y, s->y, (size_t)n * s->H * s->W * 5 * 4, hipMemcpyDeviceToDevice, s->st));
     SHIP(s, hipStreamSynchronize(s->st));
     return XBG_OK;
 }
 
 int xbg_sur_loss(xbg_sur* s, const void* x8, const void* t5, int n, double* loss) {
     if (!s || !x8 || !t5 || n < 1 || n > s->nmax) return sfail(s, XBG_E_ARG, "xbg_sur_loss: bad argument");
-    int rc = sur_forward(s, (const bf16*)x8, n);
+    int rc = sur_forward(s, (const bf16*)x8, n, s->y);
     if (!rc) rc = sur_loss_grad(s, (const bf16*)t5, n, loss);
     return rc;
 }
@@ -990,7 +1097,10 @@ int xbg_sur_sync(xbg_sur* s) {
 // Layer-level entry points on caller device buffers (tests, benchmarks).
 int xbg_sur_conv_fwd(const void* X, const void* Wt, const float* bias, void* Y, int n, int H, int W, int Cin,
                      int Cout, int taps, int relu) {
-    int rc = conv_fwd(nullptr, (const bf16*)X, (const bf16*)Wt, bias, Y, n, H, W, Cin, Cout, taps, relu, 0);
+    const CSrc src = plain((const bf16*)X, Cin);
+    const CEpi out{(bf16*)Y};
+    int rc = relu ? conv<E_STORE, true>(nullptr, src, (const bf16*)Wt, bias, out, n, H, W, Cin, Cout, taps)
+                  : conv<E_STORE, false>(nullptr, src, (const bf16*)Wt, bias, out, n, H, W, Cin, Cout, taps);
     if (rc) return sfail(nullptr, rc, "xbg_sur_conv_fwd: unsupported shape");
     if (hipDeviceSynchronize() != hipSuccess) return sfail(nullptr, XBG_E_HIP, "xbg_sur_conv_fwd: run");
     return XBG_OK;
@@ -999,7 +1109,7 @@ int xbg_sur_conv_fwd(const void* X, const void* Wt, const float* bias, void* Y, 
 int xbg_sur_conv_dgrad(const void* dZ, const void* Wt, void* dX, int n, int H, int W, int Cin, int Cout, int taps) {
     bf16* Wd = nullptr;
     if (hipMalloc((void**)&Wd, (size_t)taps * Cin * Cout * 2) != hipSuccess) return XBG_E_HIP;
-    int rc = conv_dgrad(nullptr, (const bf16*)dZ, (const bf16*)Wt, Wd, (bf16*)dX, n, H, W, Cin, Cout, taps);
+    int rc = conv_dgrad<E_STORE>(nullptr, (const bf16*)dZ, (const bf16*)Wt, Wd, CEpi{(bf16*)dX}, n, H, W, Cin, Cout, taps);
     hipError_t e = hipDeviceSynchronize();
     hipFree(Wd);
     if (rc) return sfail(nullptr, rc, "xbg_sur_conv_dgrad: unsupported shape");
