@@ -178,3 +178,26 @@ def test_fused_network_equals_its_passes(need_gpu, n, H, W):
         for what, a, r in (("weights", gw, rw), ("bias", gb, rb)):
             err, scale = (a - r).norm().item(), r.norm().item()
             assert scale > 0 and err <= rel * scale, (l, what, err, scale)
+
+
+@pytest.mark.parametrize("n,H,W,cin,cout,taps", [(1, 5, 40, 32, 32, 9), (1, 7, 96, 64, 32, 9), (2, 3, 160, 32, 64, 1),
+                                                 (1, 9, 33, 64, 64, 9), (3, 1, 64, 32, 32, 9), (1, 33, 64, 64, 64, 9),
+                                                 (2, 19, 128, 32, 64, 9), (1, 2, 32, 32, 32, 1)])
+def test_weight_gradient_at_the_edges_of_its_stages(need_gpu, n, H, W, cin, cout, taps):
+    """Strips and row stages that do not divide, against torch on the CPU
+    (1e-5: FP32 sums in another order, as for the other weight gradients)."""
+    import torch.nn.functional as F
+
+    k = 3 if taps == 9 else 1
+    g = torch.Generator().manual_seed(H * W + cin)
+    X, dZ = rnd(n, H, W, cin, g=g).to(torch.bfloat16), rnd(n, H, W, cout, g=g).to(torch.bfloat16)
+    Xd, dZd = X.cuda(), dZ.cuda()
+    dW, db = torch.empty(taps, cout, cin, device="cuda"), torch.empty(cout, device="cuda")
+    torch.cuda.synchronize()
+    assert lib().xbg_sur_conv_wgrad(Xd.data_ptr(), dZd.data_ptr(), dW.data_ptr(), db.data_ptr(), n, H, W, cin, cout,
+                                    taps) == 0
+    w = torch.zeros(cout, cin, k, k, requires_grad=True)
+    b = torch.zeros(cout, requires_grad=True)
+    F.conv2d(X.float().permute(0, 3, 1, 2), w, b, padding=k // 2).backward(dZ.float().permute(0, 3, 1, 2))
+    for a, r in ((dW.cpu().reshape(k, k, cout, cin).permute(2, 3, 0, 1), w.grad), (db.cpu(), b.grad)):
+        assert (a - r).abs().max().item() <= 1e-5 * r.abs().max().item()

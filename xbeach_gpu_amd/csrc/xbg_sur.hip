@@ -312,137 +312,256 @@ __global__ __launch_bounds__(256, 2) void k_conv(CSrc X, const bf16* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient of a convolution: dW[tap][co][ci] = sum over pixels of
-// dZ[p][co] * X[p + tap offset][ci].  A workgroup takes a 64 x 64 (or
-// smaller) block of (co, ci), one row of taps (dy) and a range of image
-// rows; per 64-pixel segment dZ and the three x-shifted copies of X are
-// staged transposed (channel-major) in LDS so that a lane's 8 consecutive
-// pixels are one 16-B read; each thread stages four consecutive pixels of
-// eight channels and writes each channel's four values as one 8-B store.
-// Waves take the output-channel tiles in turn; with fewer than four tiles
-// (32 output channels) two waves share a tile and split its input-channel
-// tiles.  Partials go to part[split][tap][co][ci] (FP32).
-// Requires W % 64 == 0 or W == 32 (TW), Cout % CBO == 0, Cin % CBI == 0.
+// Weight and bias gradient of a convolution: dW[tap][co][ci] = sum over
+// pixels of dZ[p][co] * X[p + tap offset][ci], db[co] = sum of dZ[p][co].
+//
+// Pixels are the K index of the products, channels the contiguous index in
+// memory: rows of both tensors are staged as they lie, and the transposed
+// LDS read (four pixels of one channel per lane and read) makes the
+// fragments, so each value is staged once instead of once per shift, without
+// a transpose through registers.  A wave holds a 32 x 32 block of (co, ci)
+// for all taps (144 accumulators of 256 registers) and takes two rows of dZ
+// at a time, so that a fragment of an X row serves both (28 fragment reads
+// per 72 products).  A workgroup takes a CBO x CBI block; where that is
+// fewer than four such blocks, the waves share the pixels of a stage (the
+// two 32-pixel halves of a segment, then row pairs) and add their sums at
+// the end.  It walks down a range of rows of SEG-pixel strips, keeping the
+// rows that the next rows' taps need in a ring, the following rows in flight
+// in registers.  The bias sums are products with a block of ones.
+// Partials go to part[split][taps*Cout*Cin + Cout] (FP32).
+//
+// Bound by the LDS reads and the matrix rate at 64 channels, by memory at 32.
+// At 64 x 256 x 256 the 17 layers' weight and bias gradients and their
+// reductions take 1.8 ms, and took 8.2 ms before (one copy of X per shift,
+// transposed in registers, every X row read three times; bias sums in a pass
+// of their own).
+// Requires Cout % CBO == 0, Cin % CBI == 0; any W (pixels past it are zero).
 // ---------------------------------------------------------------------------
-constexpr int WPX = 64;           // pixels per staged segment
-constexpr int WLD = WPX + 8;      // LDS stride of a transposed channel row
-template <int TAPS, int CBO, int CBI>
-__global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
-                                                    float* __restrict__ part, int N, int H, int W, int Cin,
-                                                    int Cout, int rows_per_split) {
-    constexpr int NDX = TAPS == 9 ? 3 : 1;
-    __shared__ __attribute__((aligned(16))) bf16 sD[CBO * WLD];
-    __shared__ __attribute__((aligned(16))) bf16 sXt[NDX * CBI * WLD];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, s = lane >> 4;
-    const int nco = Cout / CBO, nci = Cin / CBI;
-    int b = blockIdx.x;
-    const int cob = b % nco;
-    b /= nco;
-    const int cib = b % nci;
-    const int dy = blockIdx.y;  // 0..2 (TAPS 9) or 0
-    const int split = blockIdx.z;
-    const int co0 = cob * CBO, ci0 = cib * CBI;
-    constexpr int MT = CBO / 16;  // output-channel tiles
-    constexpr int NT = CBI / 16;  // input-channel tiles
-    constexpr int WPM = MT >= 4 ? 1 : 4 / MT;        // waves per output-channel tile
-    constexpr int MT_PER_W = MT >= 4 ? MT / 4 : 1;
-    constexpr int NT_W = NT / WPM;                   // input-channel tiles per wave
-    static_assert(MT >= 4 ? MT % 4 == 0 : 4 % MT == 0, "output-channel tiles over four waves");
-    static_assert(NT % WPM == 0, "input-channel tiles over the waves of an output tile");
-    const int t0 = MT >= 4 ? 0 : (w / MT) * NT_W;
-    f32x4 acc[MT_PER_W][NDX][NT_W];
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// Lane l of a wave gets channel l % 16 at the eight pixels 8 (l / 16) + 0..7
+// of the block whose first pixel's channels are at q, pixels PS apart.
+template <int PS>
+__device__ __forceinline__ bf16x8 tr_frag(const bf16* q, int lane) {
+    const bf16* a = q + (8 * (lane >> 4) + ((lane & 15) >> 2)) * PS + (lane & 3) * 4;
+    typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+    const bf16x4 u = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)a));
+    const bf16x4 v = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(a + 4 * PS)));
+    return __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+template <int CBO, int CBI, int SEG>
+struct WShape {
+    static constexpr int NS = (CBO / 32) * (CBI / 32), WK = 4 / NS;  // 32 x 32 blocks; waves that share one
+    static constexpr int KC = SEG / 32, KG = WK < KC ? WK : KC;      // 32-pixel chunks of a row; chunk groups
+    static constexpr int RW = 2, RS = (WK / KG) * RW;                // rows per wave and per stage
+};
+
+template <int TAPS, int CBO, int CBI, int SEG>
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad(CSrc X, const bf16* __restrict__ dZ, float* __restrict__ part,
+                                                       int N, int H, int W, int Cin, int Cout, int rows_per_split) {
+    using S = WShape<CBO, CBI, SEG>;
+    constexpr int HALO = TAPS == 9 ? 1 : 0, NDX = 2 * HALO + 1;
+    constexpr int RS = S::RS, RW = S::RW, NRX = RS + 2 * HALO, XP = SEG + 2 * HALO;
+    // pixel strides that spread the four pixel rows of a transposed read over the banks
+    constexpr int PX = CBI == 64 ? 72 : 48, PD = CBO == 64 ? 72 : 48;
+    constexpr int XROW = XP * PX, DROW = SEG * PD;
+    constexpr int CX = CBI / 8, CD = CBO / 8;  // 16-byte chunks of a pixel
+    constexpr int NX = (RS * XP * CX + 255) / 256, ND = (RS * SEG * CD + 255) / 256;
+    constexpr int TG = TAPS == 9 ? 3 : 1;                         // taps added per round of the waves' final sum
+    constexpr int RED = (S::WK - 1) * S::NS * (TG * 4 + 2) * 256 * 2;  // in bf16 units
+    constexpr int LDS = NRX * XROW + RS * DROW;
+    __shared__ __attribute__((aligned(16))) bf16 sm[LDS > RED ? LDS : RED];
+    bf16 *sX = sm, *sD = sm + NRX * XROW;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, s = lane >> 4, l16 = lane & 15;
+    const int cob = blockIdx.x % (Cout / CBO), cib = blockIdx.x / (Cout / CBO);
+    const int co0 = cob * CBO, ci0 = cib * CBI, split = blockIdx.y;
+    const int sub = w % S::NS, kg = w / S::NS;
+    const int cs = (sub % (CBO / 32)) * 32, is = (sub / (CBO / 32)) * 32;  // the wave's block
+    const int kc0 = kg % S::KG, row0 = (kg / S::KG) * RW;                  // its chunk and its first row of a stage
+    const bool bias = cib == 0 && is == 0;
+    f32x4 acc[TAPS][2][2], accb[2];
 #pragma unroll
-    for (int a = 0; a < MT_PER_W; a++)
+    for (int t = 0; t < TAPS; t++)
 #pragma unroll
-        for (int d = 0; d < NDX; d++)
+        for (int q = 0; q < 4; q++) acc[t][q >> 1][q & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    accb[0] = accb[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 ones;
 #pragma unroll
-            for (int t = 0; t < NT_W; t++) acc[a][d][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int total_rows = N * H;
-    const int r0 = split * rows_per_split, r1 = min(total_rows, r0 + rows_per_split);
-    const int segs = (W + WPX - 1) / WPX;
-    for (int row = r0; row < r1; row++) {
-        const int n = row / H, y = row % H;
-        const int ys = y + (TAPS == 9 ? dy - 1 : 0);
-        for (int sg = 0; sg < segs; sg++) {
-            const int x0 = sg * WPX;
-            const int np = min(WPX, W - x0);
-            __syncthreads();
-            // dZ segment, transposed: sD[co][p], four pixels per thread
-            for (int k = tid; k < (WPX / 4) * (CBO / 8); k += 256) {
-                const int p = (k / (CBO / 8)) * 4, ch = (k % (CBO / 8)) * 8;
-                bf16x8 v[4];
+    for (int e = 0; e < 8; e++) ones[e] = to_bf16(1.0f);
+    const int nseg = (W + SEG - 1) / SEG;
+    const int r1 = min(N * nseg * H, (split + 1) * rows_per_split);
+    int n = 0, x0 = 0, yend = 0;
+    // 16-byte chunks of X (rows yb.., nothing past the run's last tap row)
+    // and of dZ (rows yb.. of the run)
+    auto ldx = [&](int k, int yb) {
+        const int c = ci0 + (k % CX) * 8, px = (k / CX) % XP, y = yb + k / (CX * XP), x = x0 + px - HALO;
+        const bool second = c >= X.ca && X.b;
+        const int up = second ? 0 : X.up, C = second ? Cin - X.ca : X.ca, cc = second ? c - X.ca : c;
+        bf16x8 v = {};
+        if (y >= 0 && y < min(H, yend + HALO) && x >= 0 && x < W && cc < C)
+            v = *(const bf16x8*)((second ? X.b : X.a) + (((size_t)n * (H >> up) + (y >> up)) * (W >> up) + (x >> up)) * C + cc);
+        return v;
+    };
+    auto ldd = [&](int k, int yb) {
+        const int c = co0 + (k % CD) * 8, px = (k / CD) % SEG, y = yb + k / (CD * SEG), x = x0 + px;
+        bf16x8 v = {};
+        if (y < yend && x < W) v = *(const bf16x8*)(dZ + (((size_t)n * H + y) * W + x) * Cout + c);
+        return v;
+    };
+    for (int r = split * rows_per_split; r < r1;) {
+        const int strip = r / H, y0 = r % H;
+        n = strip / nseg;
+        x0 = (strip % nseg) * SEG;
+        yend = min(H, y0 + r1 - r);
+        r += yend - y0;
+        int base = 0;  // ring slot of row yy - HALO
+        __syncthreads();
+        for (int k = tid; k < NRX * XP * CX; k += 256)
+            *(bf16x8*)(sX + (k / CX) * PX + (k % CX) * 8) = ldx(k, y0 - HALO);
+        for (int k = tid; k < RS * SEG * CD; k += 256)
+            *(bf16x8*)(sD + (k / CD) * PD + (k % CD) * 8) = ldd(k, y0);
+        __syncthreads();
+        for (int yy = y0; yy < yend; yy += RS) {
+            const bool more = yy + RS < yend;
+            bf16x8 rx[NX], rd[ND];
+            if (more) {
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    v[u] = bf16x8{};
-                    if (p + u < np) v[u] = *(const bf16x8*)(dZ + (((size_t)n * H + y) * W + x0 + p + u) * Cout + co0 + ch);
+                for (int it = 0; it < NX; it++) rx[it] = ldx(tid + it * 256, yy + RS + HALO);
+#pragma unroll
+                for (int it = 0; it < ND; it++) rd[it] = ldd(tid + it * 256, yy + RS);
+            }
+#pragma unroll
+            for (int kc = 0; kc < S::KC / S::KG; kc++) {
+                const int p0 = (kc0 + kc * S::KG) * 32;
+                bf16x8 a[RW][2];
+#pragma unroll
+                for (int z = 0; z < RW; z++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++) a[z][t] = tr_frag<PD>(sD + (row0 + z) * DROW + p0 * PD + cs + 16 * t, lane);
+                if (bias) {
+#pragma unroll
+                    for (int z = 0; z < RW; z++)
+#pragma unroll
+                        for (int t = 0; t < 2; t++) accb[t] = mfma16(a[z][t], ones, accb[t]);
                 }
 #pragma unroll
-                for (int e = 0; e < 8; e++)
-                    *(bf16x4*)(sD + (ch + e) * WLD + p) = bf16x4{v[0][e], v[1][e], v[2][e], v[3][e]};
-            }
-            // X of the shifted row, one copy per dx, transposed: sXt[dx][ci][p]
-            for (int k = tid; k < NDX * (WPX / 4) * (CBI / 8); k += 256) {
-                const int d = k / ((WPX / 4) * (CBI / 8));
-                const int r = k % ((WPX / 4) * (CBI / 8));
-                const int p = (r / (CBI / 8)) * 4, ch = (r % (CBI / 8)) * 8;
-                bf16x8 v[4];
+                for (int xr = 0; xr < RW + 2 * HALO; xr++) {
+                    int slot = base + row0 + xr;
+                    if (slot >= NRX) slot -= NRX;
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const int xs = x0 + p + u + (TAPS == 9 ? d - 1 : 0);
-                    v[u] = bf16x8{};
-                    if (p + u < np && ys >= 0 && ys < H && xs >= 0 && xs < W)
-                        v[u] = *(const bf16x8*)(X + (((size_t)n * H + ys) * W + xs) * Cin + ci0 + ch);
-                }
+                    for (int dx = 0; dx < NDX; dx++) {
+                        bf16x8 b[2];
 #pragma unroll
-                for (int e = 0; e < 8; e++)
-                    *(bf16x4*)(sXt + (d * CBI + ch + e) * WLD + p) = bf16x4{v[0][e], v[1][e], v[2][e], v[3][e]};
-            }
-            __syncthreads();
+                        for (int u = 0; u < 2; u++) b[u] = tr_frag<PX>(sX + slot * XROW + (p0 + dx) * PX + is + 16 * u, lane);
 #pragma unroll
-            for (int kk = 0; kk < WPX / 32; kk++) {
+                        for (int z = 0; z < RW; z++) {
+                            const int dy = xr - z;
+                            if (dy < 0 || dy >= NDX || yy + row0 + z >= yend) continue;
 #pragma unroll
-                for (int a = 0; a < MT_PER_W; a++) {
-                    const int mt = MT >= 4 ? w + 4 * a : w % MT;
-                    bf16x8 av = *(const bf16x8*)(sD + (mt * 16 + (lane & 15)) * WLD + kk * 32 + s * 8);
+                            for (int t = 0; t < 2; t++)
 #pragma unroll
-                    for (int d = 0; d < NDX; d++)
-#pragma unroll
-                        for (int t = 0; t < NT_W; t++) {
-                            bf16x8 bv = *(const bf16x8*)(sXt + (d * CBI + (t0 + t) * 16 + (lane & 15)) * WLD +
-                                                         kk * 32 + s * 8);
-                            acc[a][d][t] = mfma16(av, bv, acc[a][d][t]);
+                                for (int u = 0; u < 2; u++)
+                                    acc[dy * NDX + dx][t][u] = mfma16(a[z][t], b[u], acc[dy * NDX + dx][t][u]);
                         }
+                    }
                 }
+            }
+            if (more) {
+                __syncthreads();
+                // the oldest RS rows of the ring give way
+#pragma unroll
+                for (int it = 0; it < NX; it++) {
+                    const int k = tid + it * 256;
+                    if (k < RS * XP * CX) {
+                        int slot = base + k / (CX * XP);
+                        if (slot >= NRX) slot -= NRX;
+                        *(bf16x8*)(sX + slot * XROW + ((k / CX) % XP) * PX + (k % CX) * 8) = rx[it];
+                    }
+                }
+#pragma unroll
+                for (int it = 0; it < ND; it++) {
+                    const int k = tid + it * 256;
+                    if (k < RS * SEG * CD) *(bf16x8*)(sD + (k / CD) * PD + (k % CD) * 8) = rd[it];
+                }
+                base += RS;
+                if (base >= NRX) base -= NRX;
+                __syncthreads();
             }
         }
     }
-    // lane holds rows (co) 4s + r of tile mt, column (ci) lane & 15 of tile t0 + t
+    // the waves that share a block add their sums, in wave order
+    if constexpr (S::WK > 1) {
+        f32x4* red = (f32x4*)sm;
+        constexpr int SL = TG * 4 + 2;
 #pragma unroll
-    for (int a = 0; a < MT_PER_W; a++)
+        for (int g = 0; g < TAPS / TG; g++) {
+            __syncthreads();
+            if (kg > 0) {
+                f32x4* o = red + ((kg - 1) * S::NS + sub) * SL * 64 + lane;
 #pragma unroll
-        for (int d = 0; d < NDX; d++)
+                for (int t = 0; t < TG; t++)
 #pragma unroll
-            for (int t = 0; t < NT_W; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int mt = MT >= 4 ? w + 4 * a : w % MT;
-                    const int co = co0 + mt * 16 + 4 * s + r;
-                    const int ci = ci0 + (t0 + t) * 16 + (lane & 15);
-                    const int tap = TAPS == 9 ? dy * 3 + d : 0;
-                    part[(((size_t)split * TAPS + tap) * Cout + co) * Cin + ci] = acc[a][d][t][r];
+                    for (int q = 0; q < 4; q++) o[(t * 4 + q) * 64] = acc[g * TG + t][q >> 1][q & 1];
+                if (g == 0) {
+                    o[TG * 4 * 64] = accb[0];
+                    o[(TG * 4 + 1) * 64] = accb[1];
                 }
+            }
+            __syncthreads();
+            if (kg == 0) {
+#pragma unroll
+                for (int j = 0; j < S::WK - 1; j++) {
+                    const f32x4* o = red + (j * S::NS + sub) * SL * 64 + lane;
+#pragma unroll
+                    for (int t = 0; t < TG; t++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) acc[g * TG + t][q >> 1][q & 1] += o[(t * 4 + q) * 64];
+                    if (g == 0) {
+                        accb[0] += o[TG * 4 * 64];
+                        accb[1] += o[(TG * 4 + 1) * 64];
+                    }
+                }
+            }
+        }
+        if (kg > 0) return;
+    }
+    // lane holds rows (co) 4 s + r of tile t, column (ci) l16 of tile u
+    float* o = part + (size_t)split * ((size_t)TAPS * Cout * Cin + Cout);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int co = co0 + cs + 16 * t + 4 * s + r;
+#pragma unroll
+            for (int tap = 0; tap < TAPS; tap++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    o[((size_t)tap * Cout + co) * Cin + ci0 + is + 16 * u + l16] = acc[tap][t][u][r];
+            if (bias && l16 == 0) o[(size_t)TAPS * Cout * Cin + co] = accb[t][r];
+        }
 }
 
-// out[i] = sum over splits of part[s*n + i], in split order
-__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, int nsplit, size_t n,
-                                                      float* __restrict__ out) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
+// out[i] (i < nw) and outb[i - nw] (unless NULL) = sum over splits of
+// part[s*n + i]: four threads take every fourth split in order, their sums
+// are added in order.  64 values per workgroup: the loads of a wavefront are
+// contiguous, and a short vector still spreads over many workgroups.
+__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, int nsplit, size_t n, size_t nw,
+                                                      float* __restrict__ out, float* __restrict__ outb) {
+    __shared__ float red[4][64];
+    const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const size_t i = (size_t)blockIdx.x * 64 + l;
     float a = 0.0f;
-    // unrolled: many loads in flight, the sum still in split order
-#pragma unroll 16
-    for (int sp = 0; sp < nsplit; sp++) a += part[(size_t)sp * n + i];
-    out[i] = a;
+    if (i < n) {
+#pragma unroll 8
+        for (int sp = g; sp < nsplit; sp += 4) a += part[(size_t)sp * n + i];
+    }
+    red[g][l] = a;
+    __syncthreads();
+    if (g == 0 && i < n) {
+        a = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
+        if (i < nw) out[i] = a;
+        else if (outb) outb[i - nw] = a;
+    }
 }
 
 // Flipped, transposed weights for the data gradient: Wd[tap][ci][co] =
@@ -457,37 +576,6 @@ __global__ __launch_bounds__(256) void k_flip_weights(const bf16* __restrict__ W
     int co = r % Cout;
     int tap = r / Cout;
     Wd[((size_t)(taps - 1 - tap) * Cin + ci) * Cout + co] = Wt[i];
-}
-
-// Per-channel sums of a [P][C] BF16 tensor (bias gradient), partials per
-// workgroup over a range of pixels: part[blockIdx.x][c].  With C dividing
-// 256 the workgroup's threads cover 256 / C pixel lanes of all C channels;
-// each lane sums its pixels in order and the lanes are added in lane order.
-__global__ __launch_bounds__(256) void k_colsum(const bf16* __restrict__ G, size_t P, int C, int ppb,
-                                                float* __restrict__ part) {
-    __shared__ float red[256];
-    const size_t p0 = (size_t)blockIdx.x * ppb;
-    const size_t p1 = p0 + ppb < P ? p0 + ppb : P;
-    if (C <= 256 && 256 % C == 0) {
-        const int lanes = 256 / C, c = threadIdx.x % C, l = threadIdx.x / C;
-        float a = 0.0f;
-#pragma unroll 8
-        for (size_t p = p0 + l; p < p1; p += lanes) a += (float)G[p * C + c];
-        red[threadIdx.x] = a;
-        __syncthreads();
-        if (l == 0) {
-            float t = 0.0f;
-            for (int k = 0; k < lanes; k++) t += red[k * C + c];
-            part[(size_t)blockIdx.x * C + c] = t;
-        }
-        return;
-    }
-    for (int c = threadIdx.x; c < C; c += 256) {
-        float a = 0.0f;
-#pragma unroll 16
-        for (size_t p = p0; p < p1; p++) a += (float)G[p * C + c];
-        part[(size_t)blockIdx.x * C + c] = a;
-    }
 }
 
 // Nearest 2x upsampling of X [N][h][w][C] into channels [c0, c0+C) of Y
@@ -744,24 +832,38 @@ int conv(hipStream_t st, CSrc X, const bf16* Wt, const float* bias, const CEpi& 
 
 CSrc plain(const bf16* x, int c) { return CSrc{x, nullptr, c, 0}; }
 
-// dW (FP32, [taps][Cout][Cin]) of one convolution from its input X and the
-// gradient dZ of its pre-activation output; partials in part (npart floats)
-int conv_wgrad(hipStream_t st, const bf16* X, const bf16* dZ, float* dW, float* part, size_t npart, int n, int H,
+// part[nsplit][n] summed over the splits: nw values into out, the rest into outb
+void reduce_parts(hipStream_t st, const float* part, int nsplit, size_t n, size_t nw, float* out, float* outb) {
+    k_reduce_parts<<<(unsigned)((n + 63) / 64), dim3(256), 0, st>>>(part, nsplit, n, nw, out, outb);
+}
+
+// dW (FP32, [taps][Cout][Cin]) and db (Cout, may be NULL) of one convolution
+// from its input X and the gradient dZ of its pre-activation output; partials
+// in part (npart floats)
+int conv_wgrad(hipStream_t st, CSrc X, const bf16* dZ, float* dW, float* db, float* part, size_t npart, int n, int H,
                int W, int Cin, int Cout, int taps) {
     if (Cin % 32 || Cout % 32 || !(taps == 1 || taps == 9)) return XBG_E_ARG;
     const int CBO = Cout % 64 == 0 ? 64 : 32, CBI = Cin % 64 == 0 ? 64 : 32;
-    const int gx = (Cout / CBO) * (Cin / CBI), gy = taps == 9 ? 3 : 1;
-    const size_t per = (size_t)taps * Cout * Cin;
-    int rows = n * H;
-    int want = 2048 / (gx * gy);
+    const int gx = (Cout / CBO) * (Cin / CBI);
+    const size_t per = (size_t)taps * Cout * Cin, np = per + Cout;
+    // strips of 64 pixels, of 32 where rows are not a multiple of 64
+    const int SEG = W % 64 == 0 ? 64 : 32;
+    const int rows = n * ((W + SEG - 1) / SEG) * H;
+    // two workgroups per CU, each of at least 16 rows (the partials of a
+    // workgroup cost as much as the products of some rows), within the buffer
+    int want = 512 / gx;
     if (want < 1) want = 1;
-    if ((size_t)want * per > npart) want = (int)(npart / per);
+    if (npart / np < (size_t)want) want = (int)(npart / np);
     if (want < 1) return XBG_E_ARG;
-    if (want > rows) want = rows;
     int rps = (rows + want - 1) / want;
-    int nsplit = (rows + rps - 1) / rps;
-    dim3 g(gx, gy, nsplit);
-#define CW(T_, O_, I_) k_conv_wgrad<T_, O_, I_><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps)
+    if (rps < 16) rps = 16;
+    rps = (rps + 7) / 8 * 8;  // whole stages of every shape
+    const dim3 g(gx, (rows + rps - 1) / rps);
+#define CW(T_, O_, I_)                                                                                                  \
+    do {                                                                                                                \
+        if (SEG == 64) k_conv_wgrad<T_, O_, I_, 64><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps);      \
+        else k_conv_wgrad<T_, O_, I_, 32><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps);                \
+    } while (0)
 #define CW_I(T_, O_) do { if (CBI == 64) CW(T_, O_, 64); else CW(T_, O_, 32); } while (0)
 #define CW_O(T_) do { if (CBO == 64) CW_I(T_, 64); else CW_I(T_, 32); } while (0)
     if (taps == 9) CW_O(9);
@@ -769,18 +871,7 @@ int conv_wgrad(hipStream_t st, const bf16* X, const bf16* dZ, float* dW, float* 
 #undef CW
 #undef CW_I
 #undef CW_O
-    k_reduce_parts<<<nblk(per), dim3(256), 0, st>>>(part, nsplit, per, dW);
-    return hipGetLastError() == hipSuccess ? 0 : XBG_E_HIP;
-}
-
-// per-channel sums of a [P][C] gradient into out (bias gradient)
-int colsum(hipStream_t st, const bf16* Gm, size_t P, int C, float* out, float* part, size_t npart) {
-    int nb = 1024;
-    if ((size_t)nb * C > npart) nb = (int)(npart / C);
-    int ppb = (int)((P + nb - 1) / nb);
-    nb = (int)((P + ppb - 1) / ppb);
-    k_colsum<<<nb, 256, 0, st>>>(Gm, P, C, ppb, part);
-    k_reduce_parts<<<nblk(C), 256, 0, st>>>(part, nb, (size_t)C, out);
+    reduce_parts(st, part, (int)g.y, np, per, dW, db);
     return hipGetLastError() == hipSuccess ? 0 : XBG_E_HIP;
 }
 
@@ -982,11 +1073,9 @@ template <int EPI>
 int conv_bwd(xbg_sur* s, int l, const bf16* X, const bf16* g, const CEpi& E, int n, int H, int W) {
     hipStream_t st = s->st;
     const ConvL& c = s->L[l];
-    const size_t P = (size_t)n * H * W;
     int rc;
-    if ((rc = conv_wgrad(st, X, g, s->G + c.w, s->part, s->npart, n, H, W, c.cin, c.cout, c.taps)))
+    if ((rc = conv_wgrad(st, plain(X, c.cin), g, s->G + c.w, s->G + c.b, s->part, s->npart, n, H, W, c.cin, c.cout, c.taps)))
         return sfail(s, rc, "wgrad " + std::to_string(l));
-    if ((rc = colsum(st, g, P, c.cout, s->G + c.b, s->part, s->npart))) return sfail(s, rc, "colsum");
     if constexpr (EPI >= 0)
         if ((rc = conv_dgrad<EPI>(st, g, s->P16 + c.w, s->Wd, E, n, H, W, c.cin, c.cout, c.taps)))
             return sfail(s, rc, "dgrad " + std::to_string(l));
@@ -1018,7 +1107,7 @@ int sur_backward(xbg_sur* s, int n) {
         int ppb = (int)((P0 + nb - 1) / nb);
         nb = (int)((P0 + ppb - 1) / ppb);
         k_head_bwd<<<nb, 256, 0, st>>>(s->gy, s->P + hd.w, s->d0, s->g_d0, P0, ppb, s->part);
-        k_reduce_parts<<<nblk(HK * HC + HK), 256, 0, st>>>(s->part, nb, (size_t)(HK * HC + HK), s->G + hd.w);
+        reduce_parts(st, s->part, nb, HK * HC + HK, HK * HC, s->G + hd.w, s->G + hd.b);
     }
     // layer l: its input, the gradient of its output before the activation,
     // and where the gradient of its input goes (masked by the activation
@@ -1121,8 +1210,7 @@ int xbg_sur_conv_wgrad(const void* X, const void* dZ, float* dW, float* db, int 
     size_t np = (size_t)16 << 20;
     float* part = nullptr;
     if (hipMalloc((void**)&part, np * 4) != hipSuccess) return XBG_E_HIP;
-    int rc = conv_wgrad(nullptr, (const bf16*)X, (const bf16*)dZ, dW, part, np, n, H, W, Cin, Cout, taps);
-    if (!rc && db) rc = colsum(nullptr, (const bf16*)dZ, (size_t)n * H * W, Cout, db, part, np);
+    int rc = conv_wgrad(nullptr, plain((const bf16*)X, Cin), (const bf16*)dZ, dW, db, part, np, n, H, W, Cin, Cout, taps);
     hipError_t e = hipDeviceSynchronize();
     hipFree(part);
     if (rc) return sfail(nullptr, rc, "xbg_sur_conv_wgrad: unsupported shape");
