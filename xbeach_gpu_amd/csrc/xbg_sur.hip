@@ -578,37 +578,6 @@ __global__ __launch_bounds__(256) void k_flip_weights(const bf16* __restrict__ W
     Wd[((size_t)(taps - 1 - tap) * Cin + ci) * Cout + co] = Wt[i];
 }
 
-// Nearest 2x upsampling of X [N][h][w][C] into channels [c0, c0+C) of Y
-// [N][2h][2w][Ctot] (the decoder's concatenation writes both halves of Y
-// in place).
-__global__ __launch_bounds__(256) void k_up_fwd(const bf16* __restrict__ X, bf16* __restrict__ Y, int N, int h,
-                                                int w, int C, int Ctot, int c0) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    size_t n_out = (size_t)N * 2 * h * 2 * w * C;
-    if (i >= n_out) return;
-    int c = i % C;
-    size_t r = i / C;
-    int x = r % (2 * w);
-    r /= 2 * w;
-    int y = r % (2 * h);
-    int n = r / (2 * h);
-    Y[(((size_t)n * 2 * h + y) * 2 * w + x) * Ctot + c0 + c] = X[(((size_t)n * h + y / 2) * w + x / 2) * C + c];
-}
-// Copy channels [c0, c0+C) between a [P][Ca] and a [P][Cb] tensor:
-// dst[p][dc0 + c] = src[p][sc0 + c] (skip concatenation and its gradient
-// split), accumulate adds to dst.
-__global__ __launch_bounds__(256) void k_chan_copy(const bf16* __restrict__ src, int Cs, int sc0,
-                                                   bf16* __restrict__ dst, int Cd, int dc0, int C, size_t P,
-                                                   int accumulate) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= P * C) return;
-    int c = i % C;
-    size_t p = i / C;
-    float v = (float)src[p * Cs + sc0 + c];
-    if (accumulate) v += (float)dst[p * Cd + dc0 + c];
-    dst[p * Cd + dc0 + c] = to_bf16(v);
-}
-
 // Backward of the output head (a 1x1 convolution of HC channels to HK in
 // FP32; its forward is the E_HEAD epilogue): from the gradient dY[p][k] of
 // its outputs, dX[p][c] = sum_k dY[p][k] W[k][c] where X > 0 (the ReLU that
@@ -730,8 +699,8 @@ __global__ __launch_bounds__(256) void k_f32_to_bf16(const float* __restrict__ a
 //   decoder: conv1 (halve channels) at the coarse level, nearest 2x
 //   upsampling, concatenation with the skip, conv3 x2; head conv1 32 -> 5
 // ReLU after every 3x3 convolution; the 1x1 convolutions are linear.
-// Inputs: 8 channels (zb, zs, uu, vv, Hm0, Tp, dir, 0), zero-padded to 32
-// on the device; outputs: 5 channels (H, Dw, Dr, Fx, Fy), normalised.
+// Inputs: 8 channels (zb, zs, uu, vv, Hm0, Tp, dir, 0) of the first
+// convolution's 32; outputs: 5 channels (H, Dw, Dr, Fx, Fy), normalised.
 // 1.8 M parameters.  H must be even and W/8 either 32 or a multiple of 64.
 // ===========================================================================
 namespace {
@@ -757,8 +726,8 @@ struct xbg_sur {
     int adam_t = 0;
     // activations (A) and their gradients (D), by name
     std::vector<void*> allocs;
-    bf16 *x32, *e0a, *e0, *p1, *e1a, *e1, *p2, *e2a, *e2, *p3, *b3a, *b3, *u2, *c2, *d2a, *d2, *u1, *c1, *d1a, *d1,
-        *u0, *c0, *d0a, *d0;
+    bf16 *e0a, *e0, *p1, *e1a, *e1, *p2, *e2a, *e2, *p3, *b3a, *b3, *u2, *d2a, *d2, *u1, *d1a, *d1,
+        *u0, *d0a, *d0;
     bf16 *g_e0a, *g_e0, *g_e1a, *g_e1, *g_e2a, *g_e2, *g_b3a, *g_b3, *g_u2, *g_d2a,
         *g_d2, *g_u1, *g_d1a, *g_d1, *g_u0, *g_d0a, *g_d0;
     float *y = nullptr, *gy = nullptr;
@@ -830,7 +799,12 @@ int conv(hipStream_t st, CSrc X, const bf16* Wt, const float* bias, const CEpi& 
     return hipGetLastError() == hipSuccess ? 0 : XBG_E_HIP;
 }
 
+// a tensor of c channels; the network's input has 8 and its convolution 32,
+// the others being zero
 CSrc plain(const bf16* x, int c) { return CSrc{x, nullptr, c, 0}; }
+// the concatenation of a tensor of c channels at half resolution, each pixel
+// standing for 2 x 2, and a skip of the other channels
+CSrc concat(const bf16* u, const bf16* e, int c) { return CSrc{u, e, c, 1}; }
 
 // part[nsplit][n] summed over the splits: nw values into out, the rest into outb
 void reduce_parts(hipStream_t st, const float* part, int nsplit, size_t n, size_t nw, float* out, float* outb) {
@@ -960,12 +934,12 @@ int xbg_sur_create(int nmax, int H, int W, unsigned seed, xbg_sur** out) {
     struct B {
         bf16** p;
         size_t n;
-    } acts[] = {{&s->x32, P0 * 32}, {&s->e0a, P0 * 32}, {&s->e0, P0 * 32},  {&s->p1, P1 * 32},
+    } acts[] = {{&s->e0a, P0 * 32}, {&s->e0, P0 * 32},  {&s->p1, P1 * 32},
                 {&s->e1a, P1 * 64}, {&s->e1, P1 * 64},  {&s->p2, P2 * 64},  {&s->e2a, P2 * 128},
                 {&s->e2, P2 * 128}, {&s->p3, P3 * 128}, {&s->b3a, P3 * 256}, {&s->b3, P3 * 256},
-                {&s->u2, P3 * 128}, {&s->c2, P2 * 256}, {&s->d2a, P2 * 128}, {&s->d2, P2 * 128},
-                {&s->u1, P2 * 64},  {&s->c1, P1 * 128}, {&s->d1a, P1 * 64}, {&s->d1, P1 * 64},
-                {&s->u0, P1 * 32},  {&s->c0, P0 * 64},  {&s->d0a, P0 * 32}, {&s->d0, P0 * 32},
+                {&s->u2, P3 * 128}, {&s->d2a, P2 * 128}, {&s->d2, P2 * 128},
+                {&s->u1, P2 * 64},  {&s->d1a, P1 * 64}, {&s->d1, P1 * 64},
+                {&s->u0, P1 * 32},  {&s->d0a, P0 * 32}, {&s->d0, P0 * 32},
                 {&s->g_e0a, P0 * 32}, {&s->g_e0, P0 * 32}, {&s->g_e1a, P1 * 64},
                 {&s->g_e1, P1 * 64}, {&s->g_e2a, P2 * 128}, {&s->g_e2, P2 * 128},
                 {&s->g_b3a, P3 * 256}, {&s->g_b3, P3 * 256}, {&s->g_u2, P3 * 128},
@@ -1026,42 +1000,32 @@ namespace {
 int sur_forward(xbg_sur* s, const bf16* x8, int n, float* y) {
     hipStream_t st = s->st;
     const int H = s->H, W = s->W;
-    const size_t P0 = (size_t)n * H * W, P1 = P0 / 4, P2 = P0 / 16;
     const ConvL& hd = s->L[17];
     auto Wt = [&](int l) { return s->P16 + s->L[l].w; };
     auto Bs = [&](int l) { return s->P + s->L[l].b; };
     int rc = 0;
-    // the 8 input channels into the first 8 of 32 (channels 8..31 stay the
-    // zeros written at creation)
-    k_chan_copy<<<nblk(P0 * 8), 256, 0, st>>>(x8, 8, 0, s->x32, 32, 0, 8, P0, 0);
     // convolution l of X on h x w pixels, through the epilogue E
 #define CONV(l, EPI, RELU, X, h, w, ...)                                                                       \
-    if ((rc = conv<EPI, RELU>(st, plain(X, s->L[l].cin), Wt(l), Bs(l), CEpi{__VA_ARGS__}, n, h, w, s->L[l].cin, \
+    if ((rc = conv<EPI, RELU>(st, X, Wt(l), Bs(l), CEpi{__VA_ARGS__}, n, h, w, s->L[l].cin, \
                               s->L[l].cout, s->L[l].taps)))                                                    \
         return sfail(s, rc, "conv " #l);
-    CONV(0, E_STORE, true, s->x32, H, W, s->e0a);
-    CONV(1, E_POOL, true, s->e0a, H, W, s->e0, s->p1);
-    CONV(2, E_STORE, true, s->p1, H / 2, W / 2, s->e1a);
-    CONV(3, E_POOL, true, s->e1a, H / 2, W / 2, s->e1, s->p2);
-    CONV(4, E_STORE, true, s->p2, H / 4, W / 4, s->e2a);
-    CONV(5, E_POOL, true, s->e2a, H / 4, W / 4, s->e2, s->p3);
-    CONV(6, E_STORE, true, s->p3, H / 8, W / 8, s->b3a);
-    CONV(7, E_STORE, true, s->b3a, H / 8, W / 8, s->b3);
-    CONV(8, E_STORE, false, s->b3, H / 8, W / 8, s->u2);
-    k_up_fwd<<<nblk(P2 * 128), 256, 0, st>>>(s->u2, s->c2, n, H / 8, W / 8, 128, 256, 0);
-    k_chan_copy<<<nblk(P2 * 128), 256, 0, st>>>(s->e2, 128, 0, s->c2, 256, 128, 128, P2, 0);
-    CONV(9, E_STORE, true, s->c2, H / 4, W / 4, s->d2a);
-    CONV(10, E_STORE, true, s->d2a, H / 4, W / 4, s->d2);
-    CONV(11, E_STORE, false, s->d2, H / 4, W / 4, s->u1);
-    k_up_fwd<<<nblk(P1 * 64), 256, 0, st>>>(s->u1, s->c1, n, H / 4, W / 4, 64, 128, 0);
-    k_chan_copy<<<nblk(P1 * 64), 256, 0, st>>>(s->e1, 64, 0, s->c1, 128, 64, 64, P1, 0);
-    CONV(12, E_STORE, true, s->c1, H / 2, W / 2, s->d1a);
-    CONV(13, E_STORE, true, s->d1a, H / 2, W / 2, s->d1);
-    CONV(14, E_STORE, false, s->d1, H / 2, W / 2, s->u0);
-    k_up_fwd<<<nblk(P0 * 32), 256, 0, st>>>(s->u0, s->c0, n, H / 2, W / 2, 32, 64, 0);
-    k_chan_copy<<<nblk(P0 * 32), 256, 0, st>>>(s->e0, 32, 0, s->c0, 64, 32, 32, P0, 0);
-    CONV(15, E_STORE, true, s->c0, H, W, s->d0a);
-    CONV(16, E_HEAD, true, s->d0a, H, W, s->d0, nullptr, nullptr, nullptr, 0, s->P + hd.w, s->P + hd.b, y);
+    CONV(0, E_STORE, true, plain(x8, 8), H, W, s->e0a);
+    CONV(1, E_POOL, true, plain(s->e0a, 32), H, W, s->e0, s->p1);
+    CONV(2, E_STORE, true, plain(s->p1, 32), H / 2, W / 2, s->e1a);
+    CONV(3, E_POOL, true, plain(s->e1a, 64), H / 2, W / 2, s->e1, s->p2);
+    CONV(4, E_STORE, true, plain(s->p2, 64), H / 4, W / 4, s->e2a);
+    CONV(5, E_POOL, true, plain(s->e2a, 128), H / 4, W / 4, s->e2, s->p3);
+    CONV(6, E_STORE, true, plain(s->p3, 128), H / 8, W / 8, s->b3a);
+    CONV(7, E_STORE, true, plain(s->b3a, 256), H / 8, W / 8, s->b3);
+    CONV(8, E_STORE, false, plain(s->b3, 256), H / 8, W / 8, s->u2);
+    CONV(9, E_STORE, true, concat(s->u2, s->e2, 128), H / 4, W / 4, s->d2a);
+    CONV(10, E_STORE, true, plain(s->d2a, 128), H / 4, W / 4, s->d2);
+    CONV(11, E_STORE, false, plain(s->d2, 128), H / 4, W / 4, s->u1);
+    CONV(12, E_STORE, true, concat(s->u1, s->e1, 64), H / 2, W / 2, s->d1a);
+    CONV(13, E_STORE, true, plain(s->d1a, 64), H / 2, W / 2, s->d1);
+    CONV(14, E_STORE, false, plain(s->d1, 64), H / 2, W / 2, s->u0);
+    CONV(15, E_STORE, true, concat(s->u0, s->e0, 32), H, W, s->d0a);
+    CONV(16, E_HEAD, true, plain(s->d0a, 32), H, W, s->d0, nullptr, nullptr, nullptr, 0, s->P + hd.w, s->P + hd.b, y);
 #undef CONV
     SHIP(s, hipGetLastError());
     return 0;
@@ -1070,11 +1034,11 @@ int sur_forward(xbg_sur* s, const bf16* x8, int n, float* y) {
 // one convolution's backward: from g, the gradient of its pre-activation
 // output, dW, db and, unless EPI is -1, the data gradient through EPI
 template <int EPI>
-int conv_bwd(xbg_sur* s, int l, const bf16* X, const bf16* g, const CEpi& E, int n, int H, int W) {
+int conv_bwd(xbg_sur* s, int l, CSrc X, const bf16* g, const CEpi& E, int n, int H, int W) {
     hipStream_t st = s->st;
     const ConvL& c = s->L[l];
     int rc;
-    if ((rc = conv_wgrad(st, plain(X, c.cin), g, s->G + c.w, s->G + c.b, s->part, s->npart, n, H, W, c.cin, c.cout, c.taps)))
+    if ((rc = conv_wgrad(st, X, g, s->G + c.w, s->G + c.b, s->part, s->npart, n, H, W, c.cin, c.cout, c.taps)))
         return sfail(s, rc, "wgrad " + std::to_string(l));
     if constexpr (EPI >= 0)
         if ((rc = conv_dgrad<EPI>(st, g, s->P16 + c.w, s->Wd, E, n, H, W, c.cin, c.cout, c.taps)))
@@ -1096,7 +1060,7 @@ int sur_loss_grad(xbg_sur* s, const bf16* t5, int n, double* loss) {
     return 0;
 }
 
-int sur_backward(xbg_sur* s, int n) {
+int sur_backward(xbg_sur* s, const bf16* x8, int n) {
     hipStream_t st = s->st;
     const int H = s->H, W = s->W;
     const size_t P0 = (size_t)n * H * W;
@@ -1114,25 +1078,25 @@ int sur_backward(xbg_sur* s, int n) {
     // that made the input, so that it is the next layer's g)
 #define BWD(l, EPI, X, g, h, w, ...) \
     if ((rc = conv_bwd<EPI>(s, l, X, g, CEpi{__VA_ARGS__}, n, h, w))) return rc;
-    BWD(16, E_STORE, s->d0a, s->g_d0, H, W, s->g_d0a, nullptr, s->d0a);
+    BWD(16, E_STORE, plain(s->d0a, 32), s->g_d0, H, W, s->g_d0a, nullptr, s->d0a);
     // a concatenation's gradient: the coarse part's, and the skip's, to which
     // the pooled path adds below
-    BWD(15, E_UPSUM, s->c0, s->g_d0a, H, W, s->g_u0, s->g_e0, nullptr, nullptr, 32);
-    BWD(14, E_STORE, s->d1, s->g_u0, H / 2, W / 2, s->g_d1, nullptr, s->d1);
-    BWD(13, E_STORE, s->d1a, s->g_d1, H / 2, W / 2, s->g_d1a, nullptr, s->d1a);
-    BWD(12, E_UPSUM, s->c1, s->g_d1a, H / 2, W / 2, s->g_u1, s->g_e1, nullptr, nullptr, 64);
-    BWD(11, E_STORE, s->d2, s->g_u1, H / 4, W / 4, s->g_d2, nullptr, s->d2);
-    BWD(10, E_STORE, s->d2a, s->g_d2, H / 4, W / 4, s->g_d2a, nullptr, s->d2a);
-    BWD(9, E_UPSUM, s->c2, s->g_d2a, H / 4, W / 4, s->g_u2, s->g_e2, nullptr, nullptr, 128);
-    BWD(8, E_STORE, s->b3, s->g_u2, H / 8, W / 8, s->g_b3, nullptr, s->b3);
-    BWD(7, E_STORE, s->b3a, s->g_b3, H / 8, W / 8, s->g_b3a, nullptr, s->b3a);
-    BWD(6, E_UNPOOL, s->p3, s->g_b3a, H / 8, W / 8, s->g_e2, nullptr, s->e2, s->g_e2);
-    BWD(5, E_STORE, s->e2a, s->g_e2, H / 4, W / 4, s->g_e2a, nullptr, s->e2a);
-    BWD(4, E_UNPOOL, s->p2, s->g_e2a, H / 4, W / 4, s->g_e1, nullptr, s->e1, s->g_e1);
-    BWD(3, E_STORE, s->e1a, s->g_e1, H / 2, W / 2, s->g_e1a, nullptr, s->e1a);
-    BWD(2, E_UNPOOL, s->p1, s->g_e1a, H / 2, W / 2, s->g_e0, nullptr, s->e0, s->g_e0);
-    BWD(1, E_STORE, s->e0a, s->g_e0, H, W, s->g_e0a, nullptr, s->e0a);
-    BWD(0, -1, s->x32, s->g_e0a, H, W, nullptr);
+    BWD(15, E_UPSUM, concat(s->u0, s->e0, 32), s->g_d0a, H, W, s->g_u0, s->g_e0, nullptr, nullptr, 32);
+    BWD(14, E_STORE, plain(s->d1, 64), s->g_u0, H / 2, W / 2, s->g_d1, nullptr, s->d1);
+    BWD(13, E_STORE, plain(s->d1a, 64), s->g_d1, H / 2, W / 2, s->g_d1a, nullptr, s->d1a);
+    BWD(12, E_UPSUM, concat(s->u1, s->e1, 64), s->g_d1a, H / 2, W / 2, s->g_u1, s->g_e1, nullptr, nullptr, 64);
+    BWD(11, E_STORE, plain(s->d2, 128), s->g_u1, H / 4, W / 4, s->g_d2, nullptr, s->d2);
+    BWD(10, E_STORE, plain(s->d2a, 128), s->g_d2, H / 4, W / 4, s->g_d2a, nullptr, s->d2a);
+    BWD(9, E_UPSUM, concat(s->u2, s->e2, 128), s->g_d2a, H / 4, W / 4, s->g_u2, s->g_e2, nullptr, nullptr, 128);
+    BWD(8, E_STORE, plain(s->b3, 256), s->g_u2, H / 8, W / 8, s->g_b3, nullptr, s->b3);
+    BWD(7, E_STORE, plain(s->b3a, 256), s->g_b3, H / 8, W / 8, s->g_b3a, nullptr, s->b3a);
+    BWD(6, E_UNPOOL, plain(s->p3, 128), s->g_b3a, H / 8, W / 8, s->g_e2, nullptr, s->e2, s->g_e2);
+    BWD(5, E_STORE, plain(s->e2a, 128), s->g_e2, H / 4, W / 4, s->g_e2a, nullptr, s->e2a);
+    BWD(4, E_UNPOOL, plain(s->p2, 64), s->g_e2a, H / 4, W / 4, s->g_e1, nullptr, s->e1, s->g_e1);
+    BWD(3, E_STORE, plain(s->e1a, 64), s->g_e1, H / 2, W / 2, s->g_e1a, nullptr, s->e1a);
+    BWD(2, E_UNPOOL, plain(s->p1, 32), s->g_e1a, H / 2, W / 2, s->g_e0, nullptr, s->e0, s->g_e0);
+    BWD(1, E_STORE, plain(s->e0a, 32), s->g_e0, H, W, s->g_e0a, nullptr, s->e0a);
+    BWD(0, -1, plain(x8, 8), s->g_e0a, H, W, nullptr);
 #undef BWD
     SHIP(s, hipGetLastError());
     return 0;
@@ -1159,14 +1123,14 @@ int xbg_sur_loss(xbg_sur* s, const void* x8, const void* t5, int n, double* loss
 
 int xbg_sur_backward(xbg_sur* s, const void* x8, const void* t5, int n, double* loss) {
     int rc = xbg_sur_loss(s, x8, t5, n, loss);
-    if (!rc) rc = sur_backward(s, n);
+    if (!rc) rc = sur_backward(s, (const bf16*)x8, n);
     if (!rc) SHIP(s, hipStreamSynchronize(s->st));
     return rc;
 }
 
 int xbg_sur_train_step(xbg_sur* s, const void* x8, const void* t5, int n, double lr, double* loss) {
     int rc = xbg_sur_loss(s, x8, t5, n, loss);
-    if (!rc) rc = sur_backward(s, n);
+    if (!rc) rc = sur_backward(s, (const bf16*)x8, n);
     if (rc) return rc;
     s->adam_t++;
     const float b1 = 0.9f, b2 = 0.999f;
