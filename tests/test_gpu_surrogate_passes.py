@@ -201,3 +201,22 @@ def test_weight_gradient_at_the_edges_of_its_stages(need_gpu, n, H, W, cin, cout
     F.conv2d(X.float().permute(0, 3, 1, 2), w, b, padding=k // 2).backward(dZ.float().permute(0, 3, 1, 2))
     for a, r in ((dW.cpu().reshape(k, k, cout, cin).permute(2, 3, 0, 1), w.grad), (db.cpu(), b.grad)):
         assert (a - r).abs().max().item() <= 1e-5 * r.abs().max().item()
+
+
+def test_inputs_at_any_element_address(need_gpu):
+    """Inputs and targets that start 2 bytes into an allocation give the same
+    loss, outputs and gradients (the kernels read 8 and 16 bytes at a time)."""
+    n, H, W = 1, 16, 256
+    s = Surrogate(n, H, W, seed=2)
+    g = torch.Generator().manual_seed(5)
+    x, t = rnd(n * H * W * 8, g=g).to(torch.bfloat16), rnd(n * H * W * 5, g=g).to(torch.bfloat16)
+    got = []
+    for shift in (0, 1):
+        xd = torch.empty(x.numel() + 1, dtype=torch.bfloat16, device="cuda")[shift:shift + x.numel()].copy_(x)
+        td = torch.empty(t.numel() + 1, dtype=torch.bfloat16, device="cuda")[shift:shift + t.numel()].copy_(t)
+        y = torch.empty(n, H, W, 5, device="cuda")
+        torch.cuda.synchronize()
+        s.forward(xd.data_ptr(), n, y.data_ptr())
+        got.append((s.backward(xd.data_ptr(), td.data_ptr(), n), y.cpu(), s.grads()))
+    s.close()
+    assert got[0][0] == got[1][0] and torch.equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])

@@ -541,41 +541,63 @@ __global__ __launch_bounds__(256, 2) void k_conv_wgrad(CSrc X, const bf16* __res
         }
 }
 
-// out[i] (i < nw) and outb[i - nw] (unless NULL) = sum over splits of
-// part[s*n + i]: four threads take every fourth split in order, their sums
-// are added in order.  64 values per workgroup: the loads of a wavefront are
-// contiguous, and a short vector still spreads over many workgroups.
-__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, int nsplit, size_t n, size_t nw,
-                                                      float* __restrict__ out, float* __restrict__ outb) {
+// Sums over splits: job j sums part[s*n + i] over its splits into out[i]
+// (i < nw) or outb[i - nw] (unless NULL).  Four threads take every fourth
+// split in order, their sums are added in order.  64 values per workgroup:
+// the loads of a wavefront are contiguous, and a short vector still spreads
+// over many workgroups.  One launch serves as many layers as the partials
+// buffer holds (18 launches of 5 us each on small batches before).
+constexpr int NLAYER = 18;
+struct SumJob {
+    const float* part;
+    float *out, *outb;
+    int nsplit, blk0;  // first workgroup of the job
+    unsigned n, nw;
+};
+struct SumJobs {
+    int count, blocks;
+    SumJob j[NLAYER];
+};
+__global__ __launch_bounds__(256) void k_reduce_parts(SumJobs J) {
     __shared__ float red[4][64];
+    int k = 0;
+    while (k + 1 < J.count && (int)blockIdx.x >= J.j[k + 1].blk0) k++;
+    const SumJob q = J.j[k];
     const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const size_t i = (size_t)blockIdx.x * 64 + l;
+    const size_t i = (size_t)(blockIdx.x - q.blk0) * 64 + l;
     float a = 0.0f;
-    if (i < n) {
+    if (i < q.n) {
 #pragma unroll 8
-        for (int sp = g; sp < nsplit; sp += 4) a += part[(size_t)sp * n + i];
+        for (int sp = g; sp < q.nsplit; sp += 4) a += q.part[(size_t)sp * q.n + i];
     }
     red[g][l] = a;
     __syncthreads();
-    if (g == 0 && i < n) {
+    if (g == 0 && i < q.n) {
         a = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
-        if (i < nw) out[i] = a;
-        else if (outb) outb[i - nw] = a;
+        if (i < q.nw) q.out[i] = a;
+        else if (q.outb) q.outb[i - q.nw] = a;
     }
 }
 
-// Flipped, transposed weights for the data gradient: Wd[tap][ci][co] =
-// W[TAPS-1-tap][co][ci] (the 180-degree rotation of a 3x3 kernel).
-__global__ __launch_bounds__(256) void k_flip_weights(const bf16* __restrict__ Wt, bf16* __restrict__ Wd, int taps,
-                                                      int Cout, int Cin) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    size_t n = (size_t)taps * Cout * Cin;
-    if (i >= n) return;
-    int ci = i % Cin;
-    size_t r = i / Cin;
-    int co = r % Cout;
-    int tap = r / Cout;
-    Wd[((size_t)(taps - 1 - tap) * Cin + ci) * Cout + co] = Wt[i];
+// Flipped, transposed weights for the data gradients: per layer
+// Wd[tap][ci][co] = W[taps-1-tap][co][ci] (the 180-degree rotation of a 3x3
+// kernel), at the layer's offset w.  All layers in one launch.
+struct FlipJob {
+    size_t w;
+    int taps, cout, cin, blk0;
+};
+struct FlipJobs {
+    int count, blocks;
+    FlipJob j[NLAYER];
+};
+__global__ __launch_bounds__(256) void k_flip_weights(const bf16* __restrict__ Wt, bf16* __restrict__ Wd, FlipJobs J) {
+    int k = 0;
+    while (k + 1 < J.count && (int)blockIdx.x >= J.j[k + 1].blk0) k++;
+    const FlipJob q = J.j[k];
+    const int i = (blockIdx.x - q.blk0) * 256 + threadIdx.x;
+    if (i >= q.taps * q.cout * q.cin) return;
+    const int ci = i % q.cin, co = i / q.cin % q.cout, tap = i / q.cin / q.cout;
+    Wd[q.w + ((size_t)(q.taps - 1 - tap) * q.cin + ci) * q.cout + co] = Wt[q.w + i];
 }
 
 // Backward of the output head (a 1x1 convolution of HC channels to HK in
@@ -644,16 +666,24 @@ __global__ __launch_bounds__(256) void k_head_bwd(const float* __restrict__ dY, 
 }
 
 // Mean squared error over the normalised targets: per-workgroup partial
-// sums of (y - t)^2 and the gradient g = 2 (y - t) / n.
+// sums of (y - t)^2 (double) and, with G, the gradient g = 2 (y - t) / n.
+// n is a multiple of 4.
 __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ Y, const bf16* __restrict__ T, size_t n,
-                                             float* __restrict__ G, float* __restrict__ part) {
-    __shared__ float red[256];
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    float e = 0.0f;
-    if (i < n) {
-        float d = Y[i] - (float)T[i];
-        G[i] = 2.0f * d / (float)n;
-        e = d * d;
+                                             float* __restrict__ G, double* __restrict__ part) {
+    __shared__ double red[256];
+    double e = 0.0;
+#pragma unroll 2
+    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
+        const f32x4 y = *(const f32x4*)(Y + i);
+        const bf16x4 t = *(const bf16x4*)(T + i);
+        f32x4 g;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float d = y[k] - (float)t[k];
+            g[k] = 2.0f * d / (float)n;
+            e += (double)(d * d);
+        }
+        if (G) *(f32x4*)(G + i) = g;
     }
     red[threadIdx.x] = e;
     __syncthreads();
@@ -662,6 +692,20 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ Y, const 
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+// out = sum of part[0..n-1] / cnt, by one workgroup
+__global__ __launch_bounds__(256) void k_mean(const double* __restrict__ part, int n, double cnt,
+                                              double* __restrict__ out) {
+    __shared__ double red[256];
+    double e = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) e += part[i];
+    red[threadIdx.x] = e;
+    __syncthreads();
+    for (int st = 128; st > 0; st >>= 1) {
+        if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = red[0] / cnt;
 }
 
 // Adam (Kingma and Ba 2015) on FP32 masters; the BF16 copy (may be NULL)
@@ -719,10 +763,13 @@ struct xbg_sur {
     size_t nparam = 0;
     float *P = nullptr, *G = nullptr, *M = nullptr, *V = nullptr;  // FP32 params, grads, Adam moments
     bf16* P16 = nullptr;                                           // BF16 copy of the parameter vector
-    bf16* Wd = nullptr;                                            // flipped weights for a data gradient
+    bf16* Wd = nullptr;                                            // flipped weights for the data gradients
     float* part = nullptr;                                         // split-K / reduction partials
-    size_t npart = 0;
-    float* lossp = nullptr;
+    size_t npart = 0, upart = 0;                                   // size, and how much the queued sums use
+    SumJobs sums{};                                                // sums queued for the next launch
+    double* lossp = nullptr;                                       // loss partials, then the loss
+    double* hloss = nullptr;                                       // the loss on the host (pinned)
+    hipEvent_t loss_done = nullptr;
     int adam_t = 0;
     // activations (A) and their gradients (D), by name
     std::vector<void*> allocs;
@@ -806,16 +853,30 @@ CSrc plain(const bf16* x, int c) { return CSrc{x, nullptr, c, 0}; }
 // standing for 2 x 2, and a skip of the other channels
 CSrc concat(const bf16* u, const bf16* e, int c) { return CSrc{u, e, c, 1}; }
 
-// part[nsplit][n] summed over the splits: nw values into out, the rest into outb
-void reduce_parts(hipStream_t st, const float* part, int nsplit, size_t n, size_t nw, float* out, float* outb) {
-    k_reduce_parts<<<(unsigned)((n + 63) / 64), dim3(256), 0, st>>>(part, nsplit, n, nw, out, outb);
+constexpr int MSE_PARTS = 1024;
+
+// sums queued over part[nsplit][n]: nw values into out, the rest into outb
+void queue_sum(SumJobs& J, const float* part, int nsplit, size_t n, size_t nw, float* out, float* outb) {
+    J.j[J.count++] = SumJob{part, out, outb, nsplit, J.blocks, (unsigned)n, (unsigned)nw};
+    J.blocks += (int)((n + 63) / 64);
+}
+void run_sums(hipStream_t st, SumJobs& J) {
+    if (J.count) k_reduce_parts<<<J.blocks, dim3(256), 0, st>>>(J);
+    J.count = J.blocks = 0;
+}
+
+// rows of one stage of k_conv_wgrad (WShape::RS)
+int wgrad_stage_rows(int CBO, int CBI, int SEG) {
+    const int wk = 4 / ((CBO / 32) * (CBI / 32)), kg = wk < SEG / 32 ? wk : SEG / 32;
+    return 2 * (wk / kg);
 }
 
 // dW (FP32, [taps][Cout][Cin]) and db (Cout, may be NULL) of one convolution
-// from its input X and the gradient dZ of its pre-activation output; partials
-// in part (npart floats)
-int conv_wgrad(hipStream_t st, CSrc X, const bf16* dZ, float* dW, float* db, float* part, size_t npart, int n, int H,
-               int W, int Cin, int Cout, int taps) {
+// from its input X and the gradient dZ of its pre-activation output: partials
+// behind the *used floats of part (npart) that queued sums hold, their sum
+// queued; queued sums run first where the buffer or the table is full
+int conv_wgrad(hipStream_t st, CSrc X, const bf16* dZ, float* dW, float* db, float* part, size_t npart, size_t* used,
+               SumJobs& J, int n, int H, int W, int Cin, int Cout, int taps) {
     if (Cin % 32 || Cout % 32 || !(taps == 1 || taps == 9)) return XBG_E_ARG;
     const int CBO = Cout % 64 == 0 ? 64 : 32, CBI = Cin % 64 == 0 ? 64 : 32;
     const int gx = (Cout / CBO) * (Cin / CBI);
@@ -823,16 +884,23 @@ int conv_wgrad(hipStream_t st, CSrc X, const bf16* dZ, float* dW, float* db, flo
     // strips of 64 pixels, of 32 where rows are not a multiple of 64
     const int SEG = W % 64 == 0 ? 64 : 32;
     const int rows = n * ((W + SEG - 1) / SEG) * H;
-    // two workgroups per CU, each of at least 16 rows (the partials of a
-    // workgroup cost as much as the products of some rows), within the buffer
+    // two workgroups per CU, each of at least two stages (a small batch is
+    // bound by the walk down the rows, about 3 us a stage: 16 rows each made
+    // the 3 x 48 x 256 gradients 0.28 ms at 64 channels), within the buffer
+    const int rs = wgrad_stage_rows(CBO, CBI, SEG);
     int want = 512 / gx;
     if (want < 1) want = 1;
     if (npart / np < (size_t)want) want = (int)(npart / np);
     if (want < 1) return XBG_E_ARG;
     int rps = (rows + want - 1) / want;
-    if (rps < 16) rps = 16;
-    rps = (rps + 7) / 8 * 8;  // whole stages of every shape
+    if (rps < 2 * rs) rps = 2 * rs;
+    rps = (rps + rs - 1) / rs * rs;
     const dim3 g(gx, (rows + rps - 1) / rps);
+    if (J.count == NLAYER || *used + g.y * np > npart) {
+        run_sums(st, J);
+        *used = 0;
+    }
+    part += *used;
 #define CW(T_, O_, I_)                                                                                                  \
     do {                                                                                                                \
         if (SEG == 64) k_conv_wgrad<T_, O_, I_, 64><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps);      \
@@ -845,18 +913,14 @@ int conv_wgrad(hipStream_t st, CSrc X, const bf16* dZ, float* dW, float* db, flo
 #undef CW
 #undef CW_I
 #undef CW_O
-    reduce_parts(st, part, (int)g.y, np, per, dW, db);
+    queue_sum(J, part, (int)g.y, np, per, dW, db);
+    *used += g.y * np;
     return hipGetLastError() == hipSuccess ? 0 : XBG_E_HIP;
 }
 
-// data gradient conv(dZ, flipped W) for a convolution Cin -> Cout, through
-// the epilogue E
-template <int EPI>
-int conv_dgrad(hipStream_t st, const bf16* dZ, const bf16* Wt, bf16* Wd, const CEpi& E, int n, int H, int W, int Cin,
-               int Cout, int taps) {
-    size_t nw = (size_t)taps * Cout * Cin;
-    k_flip_weights<<<nblk(nw), 256, 0, st>>>(Wt, Wd, taps, Cout, Cin);
-    return conv<EPI, false>(st, plain(dZ, Cout), Wd, nullptr, E, n, H, W, Cout, Cin, taps);
+void queue_flip(FlipJobs& J, size_t w, int taps, int cout, int cin) {
+    J.j[J.count++] = FlipJob{w, taps, cout, cin, J.blocks};
+    J.blocks += (int)nblk((size_t)taps * cout * cin);
 }
 
 // deterministic initialisation: He-normal weights from a counter-based hash
@@ -883,6 +947,8 @@ int xbg_sur_destroy(xbg_sur* s) {
     if (!s) return XBG_OK;
     if (s->st) hipStreamSynchronize(s->st);
     for (void* p : s->allocs) hipFree(p);
+    if (s->hloss) hipHostFree(s->hloss);
+    if (s->loss_done) hipEventDestroy(s->loss_done);
     if (s->st) hipStreamDestroy(s->st);
     delete s;
     return XBG_OK;
@@ -928,9 +994,11 @@ int xbg_sur_create(int nmax, int H, int W, unsigned seed, xbg_sur** out) {
     };
     const size_t P0 = (size_t)nmax * H * W, P1 = P0 / 4, P2 = P0 / 16, P3 = P0 / 64;
     bool ok = A((void**)&s->P, off * 4) && A((void**)&s->G, off * 4) && A((void**)&s->M, off * 4) &&
-              A((void**)&s->V, off * 4) && A((void**)&s->P16, off * 2) && A((void**)&s->Wd, 9 * 256 * 256 * 2);
+              A((void**)&s->V, off * 4) && A((void**)&s->P16, off * 2) && A((void**)&s->Wd, off * 2);
     s->npart = (size_t)32 << 20;
-    ok = ok && A((void**)&s->part, s->npart * 4) && A((void**)&s->lossp, nblk(P0 * 5) * 4);
+    ok = ok && A((void**)&s->part, s->npart * 4) && A((void**)&s->lossp, (MSE_PARTS + 1) * 8) &&
+         hipHostMalloc((void**)&s->hloss, sizeof(double), hipHostMallocDefault) == hipSuccess &&
+         hipEventCreateWithFlags(&s->loss_done, hipEventDisableTiming) == hipSuccess;
     struct B {
         bf16** p;
         size_t n;
@@ -1038,25 +1106,32 @@ int conv_bwd(xbg_sur* s, int l, CSrc X, const bf16* g, const CEpi& E, int n, int
     hipStream_t st = s->st;
     const ConvL& c = s->L[l];
     int rc;
-    if ((rc = conv_wgrad(st, X, g, s->G + c.w, s->G + c.b, s->part, s->npart, n, H, W, c.cin, c.cout, c.taps)))
+    if ((rc = conv_wgrad(st, X, g, s->G + c.w, s->G + c.b, s->part, s->npart, &s->upart, s->sums, n, H, W, c.cin, c.cout,
+                         c.taps)))
         return sfail(s, rc, "wgrad " + std::to_string(l));
     if constexpr (EPI >= 0)
-        if ((rc = conv_dgrad<EPI>(st, g, s->P16 + c.w, s->Wd, E, n, H, W, c.cin, c.cout, c.taps)))
+        if ((rc = conv<EPI, false>(st, plain(g, c.cout), s->Wd + c.w, nullptr, E, n, H, W, c.cout, c.cin, c.taps)))
             return sfail(s, rc, "dgrad " + std::to_string(l));
     return 0;
 }
 
-int sur_loss_grad(xbg_sur* s, const bf16* t5, int n, double* loss) {
+// the loss of s->y on its way to s->hloss and, with grad, its gradient into s->gy
+int sur_loss_grad(xbg_sur* s, const bf16* t5, int n, int grad) {
     hipStream_t st = s->st;
-    const size_t P0 = (size_t)n * s->H * s->W, ne = P0 * 5;
-    const unsigned nb = nblk(ne);
-    k_mse<<<nb, 256, 0, st>>>(s->y, t5, ne, s->gy, s->lossp);
-    std::vector<float> h(nb);
-    SHIP(s, hipMemcpyAsync(h.data(), s->lossp, nb * 4, hipMemcpyDeviceToHost, st));
-    SHIP(s, hipStreamSynchronize(st));
-    double a = 0.0;
-    for (float v : h) a += v;
-    if (loss) *loss = a / (double)ne;
+    const size_t ne = (size_t)n * s->H * s->W * 5;
+    const size_t want = (ne + 1023) / 1024;
+    const int nb = want < MSE_PARTS ? (int)want : MSE_PARTS;
+    k_mse<<<nb, 256, 0, st>>>(s->y, t5, ne, grad ? s->gy : nullptr, s->lossp);
+    k_mean<<<1, 256, 0, st>>>(s->lossp, nb, (double)ne, s->lossp + MSE_PARTS);
+    SHIP(s, hipMemcpyAsync(s->hloss, s->lossp + MSE_PARTS, sizeof(double), hipMemcpyDeviceToHost, st));
+    SHIP(s, hipEventRecord(s->loss_done, st));
+    return 0;
+}
+
+// waits for the loss (not for what was queued behind it)
+int sur_loss_wait(xbg_sur* s, double* loss) {
+    SHIP(s, hipEventSynchronize(s->loss_done));
+    if (loss) *loss = *s->hloss;
     return 0;
 }
 
@@ -1071,7 +1146,12 @@ int sur_backward(xbg_sur* s, const bf16* x8, int n) {
         int ppb = (int)((P0 + nb - 1) / nb);
         nb = (int)((P0 + ppb - 1) / ppb);
         k_head_bwd<<<nb, 256, 0, st>>>(s->gy, s->P + hd.w, s->d0, s->g_d0, P0, ppb, s->part);
-        reduce_parts(st, s->part, nb, HK * HC + HK, HK * HC, s->G + hd.w, s->G + hd.b);
+        s->sums.count = s->sums.blocks = 0;
+        queue_sum(s->sums, s->part, nb, HK * HC + HK, HK * HC, s->G + hd.w, s->G + hd.b);
+        s->upart = (size_t)nb * (HK * HC + HK);
+        FlipJobs F{};
+        for (int l = 1; l < 17; l++) queue_flip(F, s->L[l].w, s->L[l].taps, s->L[l].cout, s->L[l].cin);
+        k_flip_weights<<<F.blocks, 256, 0, st>>>(s->P16, s->Wd, F);
     }
     // layer l: its input, the gradient of its output before the activation,
     // and where the gradient of its input goes (masked by the activation
@@ -1098,6 +1178,7 @@ int sur_backward(xbg_sur* s, const bf16* x8, int n) {
     BWD(1, E_STORE, plain(s->e0a, 32), s->g_e0, H, W, s->g_e0a, nullptr, s->e0a);
     BWD(0, -1, plain(x8, 8), s->g_e0a, H, W, nullptr);
 #undef BWD
+    run_sums(st, s->sums);
     SHIP(s, hipGetLastError());
     return 0;
 }
@@ -1117,20 +1198,37 @@ int xbg_sur_forward(xbg_sur* s, const void* x8, int n, float* y) {
 int xbg_sur_loss(xbg_sur* s, const void* x8, const void* t5, int n, double* loss) {
     if (!s || !x8 || !t5 || n < 1 || n > s->nmax) return sfail(s, XBG_E_ARG, "xbg_sur_loss: bad argument");
     int rc = sur_forward(s, (const bf16*)x8, n, s->y);
-    if (!rc) rc = sur_loss_grad(s, (const bf16*)t5, n, loss);
+    if (!rc) rc = sur_loss_grad(s, (const bf16*)t5, n, 0);
+    if (!rc) rc = sur_loss_wait(s, loss);
     return rc;
 }
+
+}  // extern "C"
+
+namespace {
+// forward, loss and every parameter gradient, queued
+int sur_gradients(xbg_sur* s, const void* x8, const void* t5, int n) {
+    if (!s || !x8 || !t5 || n < 1 || n > s->nmax) return sfail(s, XBG_E_ARG, "xbg_sur_backward: bad argument");
+    int rc = sur_forward(s, (const bf16*)x8, n, s->y);
+    if (!rc) rc = sur_loss_grad(s, (const bf16*)t5, n, 1);
+    if (!rc) rc = sur_backward(s, (const bf16*)x8, n);
+    return rc;
+}
+}  // namespace
+
+extern "C" {
 
 int xbg_sur_backward(xbg_sur* s, const void* x8, const void* t5, int n, double* loss) {
-    int rc = xbg_sur_loss(s, x8, t5, n, loss);
-    if (!rc) rc = sur_backward(s, (const bf16*)x8, n);
+    int rc = sur_gradients(s, x8, t5, n);
     if (!rc) SHIP(s, hipStreamSynchronize(s->st));
+    if (!rc) rc = sur_loss_wait(s, loss);
     return rc;
 }
 
+// The update is queued before the loss is waited for: the device runs on
+// while the host takes the loss.
 int xbg_sur_train_step(xbg_sur* s, const void* x8, const void* t5, int n, double lr, double* loss) {
-    int rc = xbg_sur_loss(s, x8, t5, n, loss);
-    if (!rc) rc = sur_backward(s, (const bf16*)x8, n);
+    int rc = sur_gradients(s, x8, t5, n);
     if (rc) return rc;
     s->adam_t++;
     const float b1 = 0.9f, b2 = 0.999f;
@@ -1138,7 +1236,7 @@ int xbg_sur_train_step(xbg_sur* s, const void* x8, const void* t5, int n, double
     k_adam<<<nblk(s->nparam), 256, 0, s->st>>>(s->P, s->P16, s->G, s->M, s->V, s->nparam, (float)lr, b1, b2, 1e-8f,
                                                bc1, bc2);
     SHIP(s, hipGetLastError());
-    return XBG_OK;
+    return sur_loss_wait(s, loss);
 }
 
 int xbg_sur_sync(xbg_sur* s) {
@@ -1162,7 +1260,10 @@ int xbg_sur_conv_fwd(const void* X, const void* Wt, const float* bias, void* Y, 
 int xbg_sur_conv_dgrad(const void* dZ, const void* Wt, void* dX, int n, int H, int W, int Cin, int Cout, int taps) {
     bf16* Wd = nullptr;
     if (hipMalloc((void**)&Wd, (size_t)taps * Cin * Cout * 2) != hipSuccess) return XBG_E_HIP;
-    int rc = conv_dgrad<E_STORE>(nullptr, (const bf16*)dZ, (const bf16*)Wt, Wd, CEpi{(bf16*)dX}, n, H, W, Cin, Cout, taps);
+    FlipJobs F{};
+    queue_flip(F, 0, taps, Cout, Cin);
+    k_flip_weights<<<F.blocks, 256>>>((const bf16*)Wt, Wd, F);
+    int rc = conv<E_STORE, false>(nullptr, plain((const bf16*)dZ, Cout), Wd, nullptr, CEpi{(bf16*)dX}, n, H, W, Cout, Cin, taps);
     hipError_t e = hipDeviceSynchronize();
     hipFree(Wd);
     if (rc) return sfail(nullptr, rc, "xbg_sur_conv_dgrad: unsupported shape");
@@ -1174,7 +1275,10 @@ int xbg_sur_conv_wgrad(const void* X, const void* dZ, float* dW, float* db, int 
     size_t np = (size_t)16 << 20;
     float* part = nullptr;
     if (hipMalloc((void**)&part, np * 4) != hipSuccess) return XBG_E_HIP;
-    int rc = conv_wgrad(nullptr, plain((const bf16*)X, Cin), (const bf16*)dZ, dW, db, part, np, n, H, W, Cin, Cout, taps);
+    SumJobs J{};
+    size_t used = 0;
+    int rc = conv_wgrad(nullptr, plain((const bf16*)X, Cin), (const bf16*)dZ, dW, db, part, np, &used, J, n, H, W, Cin, Cout, taps);
+    run_sums(nullptr, J);
     hipError_t e = hipDeviceSynchronize();
     hipFree(part);
     if (rc) return sfail(nullptr, rc, "xbg_sur_conv_wgrad: unsupported shape");
