@@ -119,6 +119,15 @@ XDEV T ld32(const T* base, size_t idx) {
     return *(const __attribute__((address_space(1))) T*)((const __attribute__((address_space(1))) char*)base + off);
 }
 
+// Values needed in registers at this point.  Stencils that read their
+// operands under data-dependent branches, or after stores the compiler
+// cannot prove independent, would issue each load after the branch or store
+// above it: one round trip to memory per level.  Their operands are loaded
+// into locals and named here, ahead of the first branch and store, so all
+// loads are in flight together.  The asm emits no instruction.
+XDEV void need(float a, float b, float c, float d) { asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d)); }
+XDEV void need(int a, int b, int c, int d) { asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d)); }
+
 // Block (tile) coordinates of a kernel body: blockIdx in a single-domain
 // launch, the tile-map entry in a batched ensemble launch.
 struct BI {
@@ -140,15 +149,14 @@ XDEV float tab(const float* t, int th) {
     return ((cfloat_ptr)t)[k];
 }
 
-// The wave kernel's copy of the direction table in LDS (filled at its
-// start): its lookups are then LDS reads, which complete in order with the
-// plane and face reads, where a scalar load (whose results may return out
-// of order) makes each wait on it a wait for every outstanding LDS read.
-__shared__ float s_dirs[8 * MAXT];
+// L: t is the wave kernel's copy of the table in LDS (filled at its start):
+// its lookups complete in order with the plane and face reads, where a scalar
+// load (whose results may return out of order) makes each wait on it a wait
+// for every outstanding LDS read.
 template <bool L>
-XDEV float dtab(const float* g, int k, int th) {
-    if (L) return s_dirs[k * MAXT + th];
-    return tab(g + k * MAXT, th);
+XDEV float dtab(const float* t, int k, int th) {
+    if (L) return t[k * MAXT + th];
+    return tab(t + k * MAXT, th);
 }
 
 // ---------------------------------------------------------------------------
@@ -157,10 +165,11 @@ XDEV float dtab(const float* g, int k, int th) {
 // summed in row order by one lane, as a sequential sweep would.
 // ---------------------------------------------------------------------------
 // ubnd1D / ubnd1Dnowaves (Flow_kernel.cu:167-242, 332) for the offshore
-// column, by one workgroup of nthr threads (tid = flat thread index).
-XDEV void offshore_wg(const KP& p, const SP& s, const Fld& f, int waves, int tid, int nthr) {
-    __shared__ float col[1024];
-    __shared__ float avg;
+// column, by one workgroup of nthr threads (tid = flat thread index); col:
+// OFF_LDS floats of the workgroup's LDS.
+constexpr int OFF_LDS = 1025;
+XDEV void offshore_wg(const KP& p, const SP& s, const Fld& f, int waves, int tid, int nthr, float* col) {
+    float& avg = col[1024];
     const int nx = p.nx, ny = p.ny;
     float acc = 0.0f;
     for (int base = 0; base < ny; base += 1024) {
@@ -200,7 +209,8 @@ XDEV void offshore_wg(const KP& p, const SP& s, const Fld& f, int waves, int tid
 }
 
 __global__ __launch_bounds__(1024) void k_bnd_offshore(KP p, SP s, Fld f, int waves) {
-    offshore_wg(p, s, f, waves, threadIdx.x, blockDim.x);
+    __shared__ float col[OFF_LDS];
+    offshore_wg(p, s, f, waves, threadIdx.x, blockDim.x, col);
 }
 
 // ---------------------------------------------------------------------------
@@ -218,7 +228,10 @@ XDEV void dispersion_body(const KP& p, const SP& s, const Fld& f, int offshore, 
     int by = bi.y;
     if (offshore) {
         if (by == 0) {
-            if (bi.x == 0) offshore_wg(p, s, f, 1, threadIdx.x + threadIdx.y * BX, BX * BY);
+            if (bi.x == 0) {
+                __shared__ float col[OFF_LDS];
+                offshore_wg(p, s, f, 1, threadIdx.x + threadIdx.y * BX, BX * BY, col);
+            }
             return;
         }
         by -= 1;
@@ -241,12 +254,6 @@ __global__ __launch_bounds__(256) void k_dispersion(KP p, SP s, Fld f, int offsh
     dispersion_body(p, s, f, offshore, BI{(int)blockIdx.x, (int)blockIdx.y});
 }
 
-// Wave action after offshorebndWav + sanity + action (wave_CPU.cpp:24-309).
-XDEV float act_ee(const KP& p, const SP& s, const Fld& f, int x, int y, int th) {
-    float v = (x == 0) ? G(f.St)[y + th * p.ny] * s.taper
-                       : G(f.ee_in)[(size_t)x + (size_t)y * p.nx + (size_t)th * p.N];
-    return div_uniform(fmx(v, 0.000f), s.sigm, s.rsigm, s.sigm_recip);
-}
 XDEV float act_rr(const KP& p, const Fld& f, int x, int y, int th) {
     return G(f.rr_in)[(size_t)x + (size_t)y * p.nx + (size_t)th * p.N];
 }
@@ -287,9 +294,8 @@ XDEV Refr refr_cell(const KP& p, const SP& s, const Fld& f, int x, int y) {
 // CUR = false: wci == 0, where every current term is a product with w = 0
 // (a signed zero added to the rest; it can change only the sign of a zero
 // result, which no later step distinguishes), so it is left out.
-template <bool CUR, bool L = false>
-XDEV float ctheta_of(const KP& p, const float* dirs, const Refr& r, int th) {
-    float cs = dtab<L>(dirs, 1, th), sn = dtab<L>(dirs, 2, th);
+template <bool CUR>
+XDEV float ctheta_of(const Refr& r, float cs, float sn) {
     float ctht;
     if (CUR)
         ctht = r.sig * (r.dhdx * sn - r.dhdy * cs) + r.w * (cs * (sn * r.dudx - cs * r.dudy) + sn * (sn * r.dvdx - cs * r.dvdy));
@@ -298,61 +304,51 @@ XDEV float ctheta_of(const KP& p, const float* dirs, const Refr& r, int th) {
     return fmn(fmx(ctht, r.lo), r.hi);
 }
 
-// Face speeds of the x/y upwind advection at one cell
-// (xadvecupwind2CPU / yadvecupwind2CPU, wave_CPU.cpp:367-564): group (ee)
-// or phase (rr) speed at the cell and its +-1 neighbours, current times the
-// cell's wci.
+// Speeds of the x/y upwind advection at one cell (xadvecupwind2CPU /
+// yadvecupwind2CPU, wave_CPU.cpp:367-564), halved: group (ee) or phase (rr)
+// speed at the cell and its +-1 neighbours.  The face speed is 0.5 times a
+// sum of products with them; halving the factors first gives the same value
+// (wave speeds are nowhere near the subnormal range).
 struct AdvC {
-    float sc, sxm, sxp, sym, syp, ui, uxm, uxp, vi, vym, vyp;
-    float lsc, lsxm;  // speed at (x0, y0+cx) and its -x neighbour (left-face lanes)
+    float sc, sxm, sxp, sym, syp;
 };
-template <bool CUR>
-XDEV AdvC advc_cell(const KP& p, const Fld& f, const float* S, int x, int y) {
+XDEV AdvC advc_cell(const KP& p, const float* S, int x, int y) {
     const int nx = p.nx, ny = p.ny;
-    int xm = m1(x), xp = p1(x, nx), ym = m1(y), yp = p1(y, ny);
-    size_t row = (size_t)y * nx;
+    const int xm = m1(x), xp = p1(x, nx), ym = m1(y), yp = p1(y, ny);
+    const size_t row = (size_t)y * nx;
     AdvC a;
-    a.sc = S[x + row];
-    a.sxm = S[xm + row];
-    a.sxp = S[xp + row];
-    a.sym = S[x + (size_t)ym * nx];
-    a.syp = S[x + (size_t)yp * nx];
-    a.lsc = a.lsxm = 0.0f;
-    if (!CUR) {
-        a.ui = a.uxm = a.uxp = a.vi = a.vym = a.vyp = 0.0f;
-        return a;
-    }
-    float w = p.wci * fmn(G(f.hh)[x + row] / p.hwci, 1.0f);
-    a.ui = G(f.uu)[x + row] * w;
-    a.uxm = G(f.uu)[xm + row] * w;
-    a.uxp = G(f.uu)[xp + row] * w;
-    a.vi = w * G(f.vv)[x + row];
-    a.vym = w * G(f.vv)[x + (size_t)ym * nx];
-    a.vyp = w * G(f.vv)[x + (size_t)yp * nx];
+    a.sc = 0.5f * G(S)[x + row];
+    a.sxm = 0.5f * G(S)[xm + row];
+    a.sxp = 0.5f * G(S)[xp + row];
+    a.sym = 0.5f * G(S)[x + (size_t)ym * nx];
+    a.syp = 0.5f * G(S)[x + (size_t)yp * nx];
     return a;
 }
+// The current at the cell and its neighbours, times the cell's wci.
+struct CurC {
+    float ui, uxm, uxp, vi, vym, vyp;
+};
+XDEV CurC cur_cell(const KP& p, const Fld& f, int x, int y) {
+    const int nx = p.nx, ny = p.ny;
+    const int xm = m1(x), xp = p1(x, nx), ym = m1(y), yp = p1(y, ny);
+    const size_t row = (size_t)y * nx;
+    const float w = p.wci * fmn(G(f.hh)[x + row] / p.hwci, 1.0f);
+    CurC c;
+    c.ui = G(f.uu)[x + row] * w;
+    c.uxm = G(f.uu)[xm + row] * w;
+    c.uxp = G(f.uu)[xp + row] * w;
+    c.vi = w * G(f.vv)[x + row];
+    c.vym = w * G(f.vv)[x + (size_t)ym * nx];
+    c.vyp = w * G(f.vv)[x + (size_t)yp * nx];
+    return c;
+}
 
-// x + y flux divergence of one bin from its 9-point cross stencil
-// (values at the clamped neighbour indices).
-template <bool CUR, bool L = false>
-XDEV float adv_xy(const KP& p, const float* dirs, const AdvC& a, float dxi, int th, float ec, float exm, float exm2, float exp_,
-                  float exp2, float eym, float eym2, float eyp, float eyp2) {
-    float cs = dtab<L>(dirs, 1, th), sn = dtab<L>(dirs, 2, th);
-    // upwind operands are selected first so each face evaluates one
-    // 2nd-order value (branch-free code would otherwise evaluate both)
-    float cgx = CUR ? 0.5f * (a.sc * cs + a.ui + a.sxp * cs + a.uxp) : 0.5f * (a.sc * cs + a.sxp * cs);
-    float cgxmin = CUR ? 0.5f * (a.sc * cs + a.ui + a.sxm * cs + a.uxm) : 0.5f * (a.sc * cs + a.sxm * cs);
-    bool px = cgx > 0.0f, pxm = cgxmin > 0.0f;
-    float ain = upw2d(px ? ec : exp_, px ? exm : exp2) * cgx;
-    float amin = upw2d(pxm ? exm : ec, pxm ? exm2 : exp_) * cgxmin;
-    float xa = (ain - amin) * dxi;
-    float cgy = CUR ? 0.5f * (a.sc * sn + a.vi + a.syp * sn + a.vyp) : 0.5f * (a.sc * sn + a.syp * sn);
-    float cgymin = CUR ? 0.5f * (a.sc * sn + a.vi + a.sym * sn + a.vym) : 0.5f * (a.sc * sn + a.sym * sn);
-    bool py = cgy > 0.0f, pym = cgymin > 0.0f;
-    ain = upw2d(py ? ec : eyp, py ? eym : eyp2) * cgy;
-    amin = upw2d(pym ? eym : ec, pym ? eym2 : eyp) * cgymin;
-    float ya = (ain - amin) * dxi;
-    return xa + ya;
+// Flux through a face of speed cg between the cell holding lo (lo2 beyond
+// it) and the cell holding hi (hi2 beyond it).  The upwind operands are
+// selected first so that one 2nd-order value is evaluated.
+XDEV float face_flux(float cg, float lo, float lo2, float hi, float hi2) {
+    const bool pos = cg > 0.0f;
+    return upw2d(pos ? lo : hi, pos ? lo2 : hi2) * cg;
 }
 
 // roelvinkCPU (wave_CPU.cpp:932-985): Qb and D in double as written.
@@ -382,14 +378,15 @@ XDEV float baldock_cell(const KP& p, float Trep, float Ht, float h, float k, flo
 // energyCPU + energintCPU + roelvink/baldock + dissipationCPU
 // (wave_CPU.cpp:873-1089) at cell i: e (action after Euler) -> ee after
 // dissipation, r (roller after Euler) -> rr after dissipation.
-template <int NT, bool CUR, bool L = false>
-XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, size_t i, float* e, float* r, float& Rout,
-                      float& DRout) {
-    const int nt = NT > 0 ? NT : p.nt;
+// A bins at most: p.nt of them, A itself when EX.
+template <int A, bool EX, bool CUR, bool L>
+XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, float* e, float* r,
+                      float& Rout, float& DRout) {
+    const int nt = EX ? A : p.nt;
     float h = G(f.hh)[i];
     float Et = 0.0f;
 #pragma unroll
-    for (int th = 0; th < (NT > 0 ? NT : MAXT); th++) {
+    for (int th = 0; th < A; th++) {
         if (th >= nt) break;
         e[th] = fmx(e[th] * s.sigm, 0.0f);
         Et = Et + e[th];
@@ -416,17 +413,17 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, size_t i, float* e
     // x / 1 == x exactly: the division is needed only where energint capped H
     if (idiv != 1.0f) {
 #pragma unroll
-        for (int th = 0; th < (NT > 0 ? NT : MAXT); th++) {
+        for (int th = 0; th < A; th++) {
             if (th >= nt) break;
             e[th] = e[th] / idiv;
         }
     }
 #pragma unroll
-    for (int th = 0; th < (NT > 0 ? NT : MAXT); th++) {
+    for (int th = 0; th < A; th++) {
         if (th >= nt) break;
         float eet = e[th];
-        float cx = CUR ? cc * dtab<L>(f.dirs, 1, th) + uui : cc * dtab<L>(f.dirs, 1, th);
-        float cy = CUR ? cc * dtab<L>(f.dirs, 2, th) + vvi : cc * dtab<L>(f.dirs, 2, th);
+        float cx = CUR ? cc * dtab<L>(dirs, 1, th) + uui : cc * dtab<L>(dirs, 1, th);
+        float cy = CUR ? cc * dtab<L>(dirs, 2, th) + vvi : cc * dtab<L>(dirs, 2, th);
         float dd = eet * Dv / Emx;
         float rrt;
         if (wetc) {
@@ -451,26 +448,26 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, size_t i, float* e
 // meandirCPU (wave_CPU.cpp:1092-1116), radstressCPU (1118-1157) and
 // breakerdelayCPU (1334-1374, called with R) at cell i on the final ee/rr;
 // stores the directional state of the cell.
-template <int NT, bool L = false>
-XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, size_t i, const float* efin, const float* r, float Rv,
-                      float DRv) {
-    const int nt = NT > 0 ? NT : p.nt;
+template <int A, bool EX, bool L>
+XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const float* efin,
+                      const float* r, float Rv, float DRv) {
+    const int nt = EX ? A : p.nt;
     const size_t N = p.N;
     float cgi = G(f.cg)[i], ci = G(f.c)[i];
     float nn = cgi / ci;
     float sume = 0.0f, sumethet = 0.0f, txx = 0.0f, tyy = 0.0f, txy = 0.0f, rxx = 0.0f, ryy = 0.0f, rxy = 0.0f;
 #pragma unroll
-    for (int th = 0; th < (NT > 0 ? NT : MAXT); th++) {
+    for (int th = 0; th < A; th++) {
         if (th >= nt) break;
         float ev = efin[th], rv = r[th];
         sume = sume + ev;
-        sumethet = sumethet + ev * dtab<L>(f.dirs, 0, th);
-        txx = txx + (dtab<L>(f.dirs, 3, th) * ev);   // (1 + cs*cs) * ev
-        tyy = tyy + (dtab<L>(f.dirs, 4, th) * ev);   // (1 + sn*sn) * ev
-        txy = txy + (dtab<L>(f.dirs, 5, th) * ev);   // sn*cs*ev
-        rxx = rxx + (dtab<L>(f.dirs, 6, th) * rv);   // (cs*cs) * rv
-        ryy = ryy + (dtab<L>(f.dirs, 7, th) * rv);   // (sn*sn) * rv
-        rxy = rxy + (dtab<L>(f.dirs, 5, th) * rv);   // sn*cs*rv
+        sumethet = sumethet + ev * dtab<L>(dirs, 0, th);
+        txx = txx + (dtab<L>(dirs, 3, th) * ev);   // (1 + cs*cs) * ev
+        tyy = tyy + (dtab<L>(dirs, 4, th) * ev);   // (1 + sn*sn) * ev
+        txy = txy + (dtab<L>(dirs, 5, th) * ev);   // sn*cs*ev
+        rxx = rxx + (dtab<L>(dirs, 6, th) * rv);   // (cs*cs) * rv
+        ryy = ryy + (dtab<L>(dirs, 7, th) * rv);   // (sn*sn) * rv
+        rxy = rxy + (dtab<L>(dirs, 5, th) * rv);   // sn*cs*rv
         gstore(f.ee_out + i + (size_t)th * N, ev);
         gstore(f.rr_out + i + (size_t)th * N, rv);
     }
@@ -529,231 +526,307 @@ __host__ __device__ inline int xcd_tile(int b, int ntiles) {
 // written by this kernel, so only LDS needs ordering.
 XDEV void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
 
-// Staging of one directional plane of the tile (+halo) into LDS.  Halo
+// Staging of the directional planes of the tile (+halo) into LDS.  Halo
 // cells hold the values at the clamped neighbour indices
 // (mminus/pplus/mminus2/pplus2 equal clamping), so the stencil reads are
-// plain offsets.  The element a thread stages is the same in every plane:
-// its in-plane offset is computed once (Slots) and each plane adds only its
-// uniform base.  Offshore-column elements (gxx == 0) of ee come from the
-// boundary spectrum instead (offshorebndWav); they are coded as -(gyy+1).
+// plain offsets.  The element a thread stages is the same in every plane: a
+// byte offset from the plane's base, which a buffer load takes from scalar
+// registers, so that staging costs no address arithmetic.  The second slot
+// of the threads counts down from the last one: the first two wavefronts,
+// which also form the tile's bottom and left faces, have none.
 constexpr int NSLOT = (PN + WTHREADS - 1) / WTHREADS;
-struct Slots {
-    int code[NSLOT];
-};
-XDEV Slots make_slots(const KP& p, int x0, int y0, int tid) {
-    Slots sl;
-#pragma unroll
-    for (int it = 0; it < NSLOT; it++) {
-        int l = tid + it * WTHREADS;
-        int r = l / PW, c = l - r * PW;
-        int gxx = min(max(x0 + c - 2, 0), p.nx - 1);
-        int gyy = min(max(y0 + r - 2, 0), p.ny - 1);
-        sl.code[it] = l >= PN ? 0 : (gxx == 0 ? -(gyy + 1) : gxx + gyy * p.nx);
-    }
-    return sl;
+static_assert(NSLOT == 2, "two slots: one per thread, the rest on the last wavefronts");
+XDEV int slot_of(int it, int tid) { return it == 0 ? tid : 2 * WTHREADS - 1 - tid; }
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+XDEV rsrc_t plane_rsrc(const float* base, uint32_t N) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(N * 4u), 0x00027000);
 }
-
-
-// The raw values of one plane (+halo) for the thread's staging slots: the
-// global loads are issued here and consumed by store_plane one bin later,
-// so their latency overlaps the arithmetic of the current bin.
-template <bool IS_EE>
-XDEV void load_plane(float* raw, const KP& p, const Fld& f, const Slots& sl, int th) {
-    // opaque bin index: keeps the compiler from precomputing (and holding
-    // in registers) the plane addresses of every bin of the unrolled loop
+XDEV float buf_load(rsrc_t r, int off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+XDEV void buf_store(rsrc_t r, int off, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, off, 0, 0);
+}
+// a pointer that is the same in every lane, in scalar registers
+template <class T>
+XDEV T* uniform_ptr(T* q) {
+    const uint64_t b = (uint64_t)q;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    return (T*)(((uint64_t)hi << 32) | lo);
+}
+// plane th of a directional field; the bin index is opaque, so that the
+// addresses of every plane are not formed (and held) ahead of the bin loop
+XDEV rsrc_t plane_of(const float* field, int th, uint32_t N) {
     int thv = th;
     asm volatile("" : "+s"(thv));
-    const uint32_t pbase = (uint32_t)thv * p.N;
-    const float* plane = (IS_EE ? f.ee_in : f.rr_in) + pbase;
-    // one load per slot from a per-lane address (unused slots read the
-    // plane's first element): no divergent branches around the loads
-#pragma unroll
-    for (int it = 0; it < NSLOT; it++) {
-        int code = sl.code[it];
-        const float* src;
-        if (IS_EE)  // offshore column from the boundary spectrum
-            src = code >= 0 ? plane + (uint32_t)code : f.St + ((uint32_t)(-code - 1) + (uint32_t)thv * p.ny);
-        else        // rr: the offshore column carries its own value
-            src = plane + (code >= 0 ? (uint32_t)code : (uint32_t)(-code - 1) * p.nx);
-        raw[it] = gload(src);
-    }
-}
-// RQ: the divisions by sigm and dtheta go through their double reciprocals
-// unconditionally (the host launches it only when both divisors are below 2,
-// where that gives the IEEE quotient: div_uniform).
-template <bool IS_EE, bool RQ>
-XDEV void store_plane(float* pl, const SP& s, const Slots& sl, const float* raw, int tid) {
-#pragma unroll
-    for (int it = 0; it < NSLOT; it++) {
-        int l = tid + it * WTHREADS;
-        if (l < PN) {
-            float v = raw[it];
-            if (IS_EE) {
-                if (sl.code[it] < 0) v = v * s.taper;  // offshorebndWav (wave_CPU.cpp:24-56)
-                v = fmx(v, 0.000f);  // sanity + action (wave_CPU.cpp:58-82, 289-309)
-                v = RQ ? (float)((double)v * s.rsigm) : div_uniform(v, s.sigm, s.rsigm, s.sigm_recip);
-            }
-            pl[l] = v;
-        }
-    }
+    return plane_rsrc(field + (size_t)(uint32_t)thv * N, N);
 }
 
-// Speeds for the lanes that form the left faces of the tile's first column
-// (lane cx < WTY of the tile's second row of threads: row y0 + cx).
-XDEV bool left_lane(int cx, int cy) { return cy == 1 && cx < WTY; }
-XDEV void left_speeds(AdvC& a, const KP& p, const float* S, int x0, int y0, int cx, int cy) {
-    if (left_lane(cx, cy)) {
-        size_t row = (size_t)min(y0 + cx, p.ny - 1) * p.nx;
-        a.lsc = S[x0 + row];
-        a.lsxm = S[m1(x0) + row];
-    }
+// The value of the lane to the left; lane 0 gets first.
+XDEV float from_left(float v, float first) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, first), __builtin_bit_cast(int, v),
+                                                                 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
 }
 
-// x/y advection, theta advection and Euler update of all bins of one field
-// for the thread's cell.  Planes are staged through two LDS buffers (the
-// load of bin th+1 overlaps bin th).  Bin th-2 is finished as soon as the
-// action of bin th is known (its theta stencil reaches th-2..th+2), so only
-// a 5-bin window of pre-update values is live.  ea[] holds the updated
-// field on exit (eulerupwindCPU, wave_CPU.cpp:810-828).  With WAVEDT the
-// largest |ctheta| over the bins, in bin order, is returned in *cmax: the
-// theta fluxes evaluate ctheta of every bin once.
+// LDS of a wave tile of at most A bins: the direction table first (its reads
+// then fit the 16-bit offset of an LDS instruction).
+template <int A, bool CUR>
+struct WaveLds {
+    static constexpr int NF = CUR ? 0 : 2;  // face buffers, one per bin parity
+    float dirs[8 * MAXT];
+    float work[4 * PN + NF * 2 * (WTY + 1) * BX + NF * 2 * WTY + (CUR ? A * BX : 0)];
+    float red[WTHREADS / 64];
+    float stash[A][WTHREADS];  // the ee bins after the Euler step
+    XDEV float* pl(int th, int fld) { return work + ((th & 1) * 2 + fld) * PN; }
+    // flux through the top face of row (r - 1), r = 0: the tile's bottom
+    XDEV float& gy(int th, int fld, int r, int c) {
+        return work[4 * PN + (((th & 1) * 2 + fld) * (WTY + 1) + r) * BX + c];
+    }
+    XDEV float& lx(int th, int fld, int r) { return work[4 * PN + 4 * (WTY + 1) * BX + ((th & 1) * 2 + fld) * WTY + r]; }
+};
+
+// x/y advection, theta advection and Euler update (xadvecupwind2CPU ..
+// eulerupwindCPU, wave_CPU.cpp:367-828) of every bin of ee and rr for the
+// thread's cell, both fields bin by bin in one sweep: they share the
+// direction cosines, the refraction speed and the barrier of each bin.
+// The planes go through two LDS buffers per field: plane th is read while
+// plane th+1 is written from registers (loaded one bin earlier) and plane
+// th+2 is in flight.  All LDS operands of a bin are read before its first
+// use, so a bin waits for one LDS latency (selecting between two LDS values
+// by a condition made the compiler read each behind its branch).  Bin th-2 is
+// finished as soon as the action of bin th is known (its theta stencil
+// reaches th-2..th+2), so only a window of pre-update values is live.  The
+// updated ee bins go to L.stash, the rr bins to ra; the largest |ctheta| over
+// the bins (WAVEDT) is returned.
 //
 // Without the current (CUR = false) the flux through the face between two
 // cells is the same IEEE expression in both cells' stencils (the face speed
-// 0.5*(S[a]*cs + S[b]*cs) is symmetric and the upwind operands are the same
-// clamped neighbours), so each face is formed once: every cell forms its
-// right and top faces, the tile's first row also its bottom faces and eight
-// lanes the left faces of its first column; the faces go through LDS
-// (fx / gy, one buffer per bin parity) and each cell takes its left and
-// bottom face one bin later, behind the bin's barrier.
-template <int NT, bool IS_EE, bool CUR, bool RQ>
-XDEV void advect_planes(float (*pl)[PN], float (*fx)[WTY][BX + 1], float (*gy)[WTY + 1][BX], const KP& p,
-                        const SP& s, const Fld& f, const AdvC& a, const Refr& rf, const Slots& sl, int tid, int cx,
-                        int cy, float* ea, float* cmax) {
-    constexpr int A = NT > 0 ? NT : MAXT;
-    const int nt = NT > 0 ? NT : p.nt;
-    const float dxi = 1.0f / p.dx;
-    float e0[A];
-    float ctl = ctheta_of<CUR, true>(p, f.dirs, rf, 0), fl = 0.0f;
-    float cm = 0.0f;
-    if (IS_EE) {
-        float v = fabsf(ctl);
-        cm = v > cm ? v : cm;
+// is symmetric and the upwind operands are the same clamped neighbours), so
+// each face is formed once: every cell forms its right and top faces, the
+// tile's first wavefront also its bottom faces and eight lanes of the second
+// the left faces of its first column.  A cell takes its left face from the
+// lane to the left and its bottom face through LDS, one bin later, behind the
+// bin's barrier.
+//
+// Bound by VALU issue: at 2048 x 1024 x 24 the whole kernel takes 392 us, and
+// took 460 with a sweep per field, each behind its own barriers, the face
+// operands read from LDS behind the upwind test and the staged elements
+// addressed with 64-bit arithmetic in every lane.
+//
+// A, EX: at most A bins, p.nt of them (A exactly when EX).  FLEX: the roller
+// switch and the divisions by sigm and dtheta decided at run time; otherwise
+// the roller is on and both divisors are below 2 (div_uniform).
+template <int A, bool EX, bool CUR, bool FLEX>
+XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f, int x0, int y0, int x, int y, int cx,
+                      int cy, float* ra) {
+    const int nt = EX ? A : p.nt;
+    const int tid = cx + cy * BX, nx = p.nx, ny = p.ny;
+    const uint32_t N = p.N;
+    const bool rol = FLEX ? p.roller == 1 : true;
+    const float dxi = 1.0f / p.dx, dt = s.dt;
+    const Refr rf = refr_cell<CUR>(p, s, f, x, y);
+    AdvC ae = advc_cell(p, f.cg, x, y), ar = advc_cell(p, f.c, x, y);
+    CurC cu{};
+    if (CUR) cu = cur_cell(p, f, x, y);
+    const int row = __builtin_amdgcn_readfirstlane(cy);  // one wavefront per row
+    // the lanes that form the left faces of row y0 + cx
+    const bool left = !CUR && row == 1 && cx < WTY;
+    if (left) {
+        const size_t r = (size_t)min(y0 + cx, ny - 1) * nx;
+        ae.sym = 0.5f * G(f.cg)[x0 + r];  // (the second wavefront forms no bottom faces)
+        ae.sxm = 0.5f * G(f.cg)[m1(x0) + r];
+        ar.sym = 0.5f * G(f.c)[x0 + r];
+        ar.sxm = 0.5f * G(f.c)[m1(x0) + r];
     }
-    // finish bin b (0 <= b < nt) once e0[b-1..b+2] are known; theta flux
-    // through the face between b and b+1 formed once (thetaadvecuw2hoCPU,
-    // wave_CPU.cpp:706-808, forms it twice from identical operands)
-    auto finish = [&](int b) {
-        float ta;
-        if (nt <= 1) {
-            ta = 0.0f;
-        } else if (b < nt - 1) {
-            int tm = m1(b), tp = b + 1, tp2 = p2(b, nt);
-            float ctr = ctheta_of<CUR, true>(p, f.dirs, rf, tp);
-            if (IS_EE) {
-                float v = fabsf(ctr);
-                cm = v > cm ? v : cm;
-            }
-            float cb = 0.5f * (ctl + ctr);
-            bool pc = cb > 0.0f;
-            float eu = upw2f(pc ? e0[b] : e0[tp], pc ? e0[tm] : e0[tp2]);
-            float fr = cb * eu;
-            const float num = b == 0 ? fr - 0.0f : fr - fl;
-            ta = RQ ? (float)((double)num * p.rdtheta) : div_uniform(num, p.dtheta, p.rdtheta, p.dth_recip);
-            fl = fr;
-            ctl = ctr;
-        } else {
-            ta = RQ ? (float)((double)(0.0f - fl) * p.rdtheta) : div_uniform(0.0f - fl, p.dtheta, p.rdtheta, p.dth_recip);
-        }
-        ea[b] = e0[b] - s.dt * (ea[b] + ta);
-    };
-    // plane th is read from LDS while plane th+1 is written to the other
-    // buffer (from registers loaded one bin earlier) and plane th+2 is in
-    // flight from HBM
-    float raw[NSLOT];
-    load_plane<IS_EE>(raw, p, f, sl, 0);
-    store_plane<IS_EE, RQ>(pl[0], s, sl, raw, tid);
-    if (nt > 1) load_plane<IS_EE>(raw, p, f, sl, 1);
-    lds_barrier();
-    const int c0 = (cy + 2) * PW + (cx + 2);
-    if (!CUR) {
-        const int cl = (cx + 2) * PW + 2;  // left-face lanes: first cell of row cx
-        float fxo = 0.0f, gyo = 0.0f;      // this cell's right / top face of the previous bin
+    // staging slots; the offshore column of ee comes from the boundary
+    // spectrum (offshorebndWav, wave_CPU.cpp:24-56): only tiles at x0 = 0
+    const float *pe = uniform_ptr(f.ee_in), *pr = uniform_ptr(f.rr_in);
+    const bool first = x0 == 0;
+    int off[NSLOT], sto[NSLOT];
+    bool offs[NSLOT];
 #pragma unroll
-        for (int th = 0; th <= A; th++) {
-            if (th > nt) break;
-            if (th >= 1) {
-                const int b = (th - 1) & 1;
-                ea[th - 1] = (fxo - fx[b][cy][cx]) * dxi + (gyo - gy[b][cy][cx]) * dxi;
-                asm volatile("" : "+v"(ea[th - 1]) : : "memory");
+    for (int it = 0; it < NSLOT; it++) {
+        const int l = min(slot_of(it, tid), PN - 1), r = l / PW, c = l - r * PW;
+        const int gx_ = min(max(x0 + c - 2, 0), nx - 1), gy_ = min(max(y0 + r - 2, 0), ny - 1);
+        off[it] = (gx_ + gy_ * nx) * 4;
+        sto[it] = gy_;
+        offs[it] = gx_ == 0;
+    }
+    float re[NSLOT], rs[NSLOT] = {}, rr[NSLOT] = {};
+    auto load = [&](int th) {
+        const rsrc_t qe = plane_of(pe, th, N);
+#pragma unroll
+        for (int it = 0; it < NSLOT; it++) re[it] = buf_load(qe, off[it]);
+        if (first) {
+#pragma unroll
+            for (int it = 0; it < NSLOT; it++) rs[it] = gload(f.St + (uint32_t)(sto[it] + th * ny));
+        }
+        if (rol) {
+            const rsrc_t qr = plane_of(pr, th, N);
+#pragma unroll
+            for (int it = 0; it < NSLOT; it++) rr[it] = buf_load(qr, off[it]);
+        }
+    };
+    auto div = [&](float a, double rb, float b, int use) { return FLEX ? div_uniform(a, b, rb, use) : (float)((double)a * rb); };
+    auto store = [&](int th) {
+        float *de = L.pl(th, 0), *dr = L.pl(th, 1);
+#pragma unroll
+        for (int it = 0; it < NSLOT; it++) {
+            const int l = slot_of(it, tid);
+            if (it == 0 || l < PN) {
+                float v = re[it];
+                if (first) v = offs[it] ? rs[it] * s.taper : v;
+                v = fmx(v, 0.000f);  // sanity + action (wave_CPU.cpp:58-82, 289-309)
+                de[l] = div(v, s.rsigm, s.sigm, s.sigm_recip);
+                if (rol) dr[l] = rr[it];
             }
-            if (th == nt) break;
-            const float* q = pl[th & 1];
-            const float cs = dtab<true>(f.dirs, 1, th), sn = dtab<true>(f.dirs, 2, th);
-            float ec = q[c0];
-            e0[th] = ec;
-            float cgx = 0.5f * (a.sc * cs + a.sxp * cs);
-            bool px = cgx > 0.0f;
-            fxo = upw2d(px ? ec : q[c0 + 1], px ? q[c0 - 1] : q[c0 + 2]) * cgx;
-            float cgy = 0.5f * (a.sc * sn + a.syp * sn);
-            bool py = cgy > 0.0f;
-            gyo = upw2d(py ? ec : q[c0 + PW], py ? q[c0 - PW] : q[c0 + 2 * PW]) * cgy;
-            fx[th & 1][cy][cx + 1] = fxo;
-            gy[th & 1][cy + 1][cx] = gyo;
-            if (cy == 0) {  // bottom faces of the tile
-                float cgymin = 0.5f * (a.sc * sn + a.sym * sn);
-                bool pym = cgymin > 0.0f;
-                gy[th & 1][0][cx] = upw2d(pym ? q[c0 - PW] : ec, pym ? q[c0 - 2 * PW] : q[c0 + PW]) * cgymin;
+        }
+    };
+    load(0);
+    store(0);
+    if (nt > 1) load(1);
+    lds_barrier();
+    const int c0 = (cy + 2) * PW + (cx + 2), cl = (cx + 2) * PW + 2;
+    // window of pre-update values: bins th-3, th-2, th-1; x/y divergence of
+    // bins th-2, th-1; theta flux below bin th-2; right and top faces of th-1
+    float e3 = 0, e2 = 0, e1 = 0, xe2 = 0, xe1 = 0, fle = 0, fxe = 0, gye = 0;
+    float r3 = 0, r2 = 0, r1 = 0, xr2 = 0, xr1 = 0, flr = 0, fxr = 0, gyr = 0;
+    float cs1 = 0, sn1 = 0, ctl = 0, cm = 0;
+#pragma unroll
+    for (int th = 0; th <= A; th++) {
+        if (!EX && th > nt) break;
+        const bool bin = EX ? th < A : th < nt;
+        float ec = e1, rc = r1, cs = 0, sn = 0;  // past the last bin: the clamped neighbour
+        float gbe = 0, gbr = 0, lxe = 0, lxr = 0;
+        float xen = 0, xrn = 0;
+        if (!CUR && th >= 1) {
+            gbe = L.gy(th - 1, 0, cy, cx);
+            lxe = L.lx(th - 1, 0, cy);
+            gbr = L.gy(th - 1, 1, cy, cx);
+            lxr = L.lx(th - 1, 1, cy);
+        }
+        float fxen = 0, gyen = 0, fxrn = 0, gyrn = 0;
+        if (bin) {
+            const float *q = L.pl(th, 0) + c0, *t = L.pl(th, 1) + c0;
+            cs = dtab<true>(L.dirs, 1, th);
+            sn = dtab<true>(L.dirs, 2, th);
+            ec = q[0];
+            const float el = q[-1], er = q[1], er2 = q[2], eb = q[-PW], et = q[PW], et2 = q[2 * PW];
+            rc = t[0];
+            const float rl = t[-1], rx = t[1], rx2 = t[2], rb = t[-PW], rt = t[PW], rt2 = t[2 * PW];
+            if (!CUR) {
+                need(gbe, gbr, lxe, lxr);
+                need(ec, el, er, er2);
+                need(eb, et, et2, cs);
+                need(rc, rl, rx, rx2);
+                need(rb, rt, rt2, sn);
+                fxen = face_flux(ae.sc * cs + ae.sxp * cs, ec, el, er, er2);
+                gyen = face_flux(ae.sc * sn + ae.syp * sn, ec, eb, et, et2);
+                fxrn = face_flux(ar.sc * cs + ar.sxp * cs, rc, rl, rx, rx2);
+                gyrn = face_flux(ar.sc * sn + ar.syp * sn, rc, rb, rt, rt2);
+                L.gy(th, 0, cy + 1, cx) = gyen;
+                L.gy(th, 1, cy + 1, cx) = gyrn;
+                if (row == 0) {  // bottom faces of the tile
+                    L.gy(th, 0, 0, cx) = face_flux(ae.sc * sn + ae.sym * sn, eb, q[-2 * PW], ec, et);
+                    L.gy(th, 1, 0, cx) = face_flux(ar.sc * sn + ar.sym * sn, rb, t[-2 * PW], rc, rt);
+                }
+                if (row == 1) {  // left faces of the tile
+                    if (left) {
+                        const float *a = L.pl(th, 0) + cl, *b = L.pl(th, 1) + cl;
+                        const float a0 = a[0], am = a[-1], am2 = a[-2], ap = a[1];
+                        const float b0 = b[0], bm = b[-1], bm2 = b[-2], bp = b[1];
+                        need(a0, am, am2, ap);
+                        need(b0, bm, bm2, bp);
+                        L.lx(th, 0, cx) = face_flux(ae.sym * cs + ae.sxm * cs, am, am2, a0, ap);
+                        L.lx(th, 1, cx) = face_flux(ar.sym * cs + ar.sxm * cs, bm, bm2, b0, bp);
+                    }
+                }
+            } else {
+                const float el2 = q[-2], eb2 = q[-2 * PW], rl2 = t[-2], rb2 = t[-2 * PW];
+                need(ec, el, er, er2);
+                need(eb, et, et2, cs);
+                need(rc, rl, rx, rx2);
+                need(rb, rt, rt2, sn);
+                need(el2, eb2, rl2, rb2);
+                // 0.5 (S cs + u + S' cs + u') in the reference's order
+                auto spd = [](float a, float u, float b, float v, float d) { return 0.5f * ((2.0f * a) * d + u + (2.0f * b) * d + v); };
+                xen = (face_flux(spd(ae.sc, cu.ui, ae.sxp, cu.uxp, cs), ec, el, er, er2) -
+                       face_flux(spd(ae.sc, cu.ui, ae.sxm, cu.uxm, cs), el, el2, ec, er)) * dxi +
+                      (face_flux(spd(ae.sc, cu.vi, ae.syp, cu.vyp, sn), ec, eb, et, et2) -
+                       face_flux(spd(ae.sc, cu.vi, ae.sym, cu.vym, sn), eb, eb2, ec, et)) * dxi;
+                xrn = (face_flux(spd(ar.sc, cu.ui, ar.sxp, cu.uxp, cs), rc, rl, rx, rx2) -
+                       face_flux(spd(ar.sc, cu.ui, ar.sxm, cu.uxm, cs), rl, rl2, rc, rx)) * dxi +
+                      (face_flux(spd(ar.sc, cu.vi, ar.syp, cu.vyp, sn), rc, rb, rt, rt2) -
+                       face_flux(spd(ar.sc, cu.vi, ar.sym, cu.vym, sn), rb, rb2, rc, rt)) * dxi;
             }
-            if (left_lane(cx, cy)) {  // left faces of the tile
-                float cgxmin = 0.5f * (a.lsc * cs + a.lsxm * cs);
-                bool pxm = cgxmin > 0.0f;
-                fx[th & 1][cx][0] = upw2d(pxm ? q[cl - 1] : q[cl], pxm ? q[cl - 2] : q[cl + 1]) * cgxmin;
+        }
+        if (!CUR && th >= 1) {
+            xe1 = (fxe - from_left(fxe, lxe)) * dxi + (gye - gbe) * dxi;
+            xr1 = (fxr - from_left(fxr, lxr)) * dxi + (gyr - gbr) * dxi;
+        }
+        if (th == 0) {
+            ctl = ctheta_of<CUR>(rf, cs, sn);
+            const float v = fabsf(ctl);
+            cm = v > cm ? v : cm;
+        }
+        if (th >= 2) {
+            // bin b = th - 2: the theta flux through its upper face is formed
+            // once (thetaadvecuw2hoCPU, wave_CPU.cpp:706-808, forms it twice
+            // from identical operands)
+            const float ctr = ctheta_of<CUR>(rf, cs1, sn1);
+            const float v = fabsf(ctr);
+            cm = v > cm ? v : cm;
+            const float cb = 0.5f * (ctl + ctr);
+            const bool pc = cb > 0.0f;
+            const float fe = cb * upw2f(pc ? e2 : e1, pc ? (th == 2 ? e2 : e3) : ec);
+            const float fr = cb * upw2f(pc ? r2 : r1, pc ? (th == 2 ? r2 : r3) : rc);
+            const float te = div(fe - fle, p.rdtheta, p.dtheta, p.dth_recip);
+            const float tr = div(fr - flr, p.rdtheta, p.dtheta, p.dth_recip);
+            fle = fe;
+            flr = fr;
+            ctl = ctr;
+            L.stash[th - 2][tid] = e2 - dt * (xe2 + te);
+            ra[th - 2] = r2 - dt * (xr2 + tr);
+            asm volatile("" : "+v"(ra[th - 2]) : : "memory");
+        }
+        if (th >= 1 && !bin) {  // the last bin: nothing leaves through its upper face
+            const float te = div(0.0f - fle, p.rdtheta, p.dtheta, p.dth_recip);
+            const float tr = div(0.0f - flr, p.rdtheta, p.dtheta, p.dth_recip);
+            L.stash[th - 1][tid] = e1 - dt * (xe1 + te);
+            ra[th - 1] = r1 - dt * (xr1 + tr);
+        }
+        if (bin) {
+            xe2 = xe1;
+            xr2 = xr1;
+            if (CUR) {
+                xe1 = xen;
+                xr1 = xrn;
             }
-            if (th >= 2) finish(th - 2);
-            asm volatile("" : "+v"(fxo), "+v"(gyo) : : "memory");
-            if (th >= 2) asm volatile("" : "+v"(ea[th - 2]) : : "memory");
-            if (th + 1 < nt) {
-                store_plane<IS_EE, RQ>(pl[(th + 1) & 1], s, sl, raw, tid);
-                if (th + 2 < nt) load_plane<IS_EE>(raw, p, f, sl, th + 2);
+            e3 = e2;
+            e2 = e1;
+            e1 = ec;
+            r3 = r2;
+            r2 = r1;
+            r1 = rc;
+            cs1 = cs;
+            sn1 = sn;
+            fxe = fxen;
+            gye = gyen;
+            fxr = fxrn;
+            gyr = gyrn;
+            // keep this bin's arithmetic ahead of the staging of the next
+            // plane, whose wait for memory must not move in front of it
+            asm volatile("" : "+v"(fxe), "+v"(gye), "+v"(fxr), "+v"(gyr) : : "memory");
+            asm volatile("" : "+v"(xe2), "+v"(xr2), "+v"(xe1), "+v"(xr1) : : "memory");
+            if (EX ? th + 1 < A : th + 1 < nt) {
+                store(th + 1);
+                if (EX ? th + 2 < A : th + 2 < nt) load(th + 2);
             }
             lds_barrier();
         }
-#pragma unroll
-        for (int b = 0; b < A; b++) {
-            if (b >= nt) break;
-            if (b >= nt - 2) finish(b);
-        }
-        if (IS_EE) *cmax = cm;
-        return;
     }
-#pragma unroll
-    for (int th = 0; th < A; th++) {
-        if (th >= nt) break;
-        const float* q = pl[th & 1];
-        float ec = q[c0];
-        e0[th] = ec;
-        ea[th] = adv_xy<CUR, true>(p, f.dirs, a, dxi, th, ec, q[c0 - 1], q[c0 - 2], q[c0 + 1], q[c0 + 2], q[c0 - PW], q[c0 - 2 * PW],
-                        q[c0 + PW], q[c0 + 2 * PW]);
-        if (th >= 2) finish(th - 2);
-        // materialise this bin's results (otherwise the arithmetic is sunk
-        // past the barriers and the stencil values of every bin stay live),
-        // and keep the staging of the next plane behind them (its wait for
-        // HBM must not move ahead of this bin's arithmetic)
-        asm volatile("" : "+v"(ea[th]) : : "memory");
-        if (th >= 2) asm volatile("" : "+v"(ea[th - 2]) : : "memory");
-        if (th + 1 < nt) {
-            store_plane<IS_EE, RQ>(pl[(th + 1) & 1], s, sl, raw, tid);
-            if (th + 2 < nt) load_plane<IS_EE>(raw, p, f, sl, th + 2);
-        }
-        lds_barrier();
-    }
-#pragma unroll
-    for (int b = 0; b < A; b++) {
-        if (b >= nt) break;
-        if (b >= nt - 2) finish(b);
-    }
-    if (IS_EE) *cmax = cm;
+    return cm;
 }
 
 // The fused wave step, one thread per cell of a 64 x WTY tile:
@@ -763,16 +836,13 @@ XDEV void advect_planes(float (*pl)[PN], float (*fx)[WTY][BX + 1], float (*gy)[W
 // (rollerlatbnd copies from rows 1 and ny-2) are finished in the tile when
 // it also holds the source row (fold_rows), else by k_wave_rows from the
 // post-Euler bins this kernel saves.  Also the block minimum of WAVEDT.
-// Four waves per SIMD (<= 128 VGPRs): two workgroups per CU.
-template <int NT, bool CUR, bool RQ>
-XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi) {
-    constexpr int A = NT > 0 ? NT : MAXT;
-    const int nt = NT > 0 ? NT : p.nt;
-    __shared__ float pl[2][PN];
-    __shared__ float wred[WTHREADS / 64];
-    __shared__ float stash[NT > 0 ? NT : 1][WTHREADS];
-    __shared__ float fx[CUR ? 1 : 2][WTY][BX + 1];
-    __shared__ float gy[CUR ? 1 : 2][WTY + 1][BX];
+// Up to 24 bins: four waves per SIMD (<= 128 VGPRs) and at most 80 KB of LDS,
+// two workgroups per CU; more bins: one workgroup.
+constexpr int wave_occ(int A) { return A <= 24 ? 4 : 2; }
+template <int A, bool EX, bool CUR, bool FLEX>
+XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CUR>& L) {
+    static_assert(A > 24 || 2 * sizeof(WaveLds<A, CUR>) <= 160 * 1024, "two workgroups per CU");
+    const int nt = EX ? A : p.nt;
     const int cx = threadIdx.x, cy = threadIdx.y, tid = cx + cy * BX;
     const int tile = bi.x;  // tile of the domain, after the XCD remap
     const int x0 = (tile % p.wtiles_x) * BX, y0 = (tile / p.wtiles_x) * WTY;
@@ -780,48 +850,16 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi) {
     const int x = min(x0 + cx, nx - 1), y = min(y0 + cy, ny - 1);
     const bool valid = (x0 + cx < nx) && (y0 + cy < ny);
     const uint32_t i = (uint32_t)x + (uint32_t)y * nx;
-    float ea[A];
-    for (int l = tid; l < 8 * MAXT; l += WTHREADS) s_dirs[l] = G(f.dirs)[l];
-    const Refr rf = refr_cell<CUR>(p, s, f, x, y);
-    const Slots sl = make_slots(p, x0, y0, tid);
+    const bool rol = FLEX ? p.roller == 1 : true;
+    for (int l = tid; l < 8 * MAXT; l += WTHREADS) L.dirs[l] = G(f.dirs)[l];
     __syncthreads();
+    float ra[A], ea[A];
     // WAVEDT (Wave_kernel.cu:232-249): min over bins of CFL*dtheta/|ctheta|.
     // Rounded division is monotonic in the divisor, so this equals one
     // division by the largest |ctheta| (NaN speeds ignored as fminf does).
-    float cmax;
-    {
-        AdvC a = advc_cell<CUR>(p, f, f.cg, x, y);
-        if (!CUR) left_speeds(a, p, f.cg, x0, y0, cx, cy);
-        advect_planes<NT, true, CUR, RQ>(pl, fx, gy, p, s, f, a, rf, sl, tid, cx, cy, ea, &cmax);
-    }
+    const float cmax = wave_sweep<A, EX, CUR, FLEX>(L, p, s, f, x0, y0, x, y, cx, cy, ra);
     float wmin = fmn(9999999.9f, p.CFL * p.dtheta / cmax);
-    const int side = p.fold_rows && NT > 0 ? -1 : ((y == 1) ? 0 : (y == ny - 2 ? 1 : -1));
-    if (valid && side >= 0) {
-#pragma unroll
-        for (int th = 0; th < A; th++) {
-            if (th >= nt) break;
-            G(f.bnd_e1)[((uint32_t)side * nt + th) * nx + x] = ea[th];
-        }
-    }
-    // the post-Euler ee bins wait in LDS while rr is advected (they would
-    // otherwise hold nTheta registers through the roller pass)
-    if (NT > 0) {
-#pragma unroll
-        for (int th = 0; th < A; th++) stash[th][tid] = ea[th];
-    }
-    float ra[A];
-    if (p.roller == 1) {
-        AdvC a = advc_cell<CUR>(p, f, f.c, x, y);
-        if (!CUR) left_speeds(a, p, f.c, x0, y0, cx, cy);
-        advect_planes<NT, false, CUR, RQ>(pl, fx, gy, p, s, f, a, rf, sl, tid, cx, cy, ra, nullptr);
-        if (valid && side >= 0) {
-#pragma unroll
-            for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
-                G(f.bnd_r1)[((uint32_t)side * nt + th) * nx + x] = ra[th];
-            }
-        }
-    } else {
+    if (!rol) {
 #pragma unroll
         for (int th = 0; th < A; th++) {
             if (th >= nt) break;
@@ -835,60 +873,80 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi) {
     // condition: the barriers below are reached by every thread or none)
     // the source row's values come through LDS; otherwise k_wave_rows
     // finishes the rows after this kernel.
-    const bool ftile = NT > 0 && p.fold_rows && (y0 == 0 || (ny - 1 >= y0 && ny - 1 < y0 + WTY));
+    const bool ftile = p.fold_rows && (y0 == 0 || (ny - 1 >= y0 && ny - 1 < y0 + WTY));
     const int bsrc = !ftile || !valid ? 0 : (y == 0 ? BX : (y == ny - 1 ? -BX : 0));
     const bool bsink = valid && ((y0 == 0 && cy == 1) || y == ny - 2);
-    float (*rx)[BX] = reinterpret_cast<float (*)[BX]>(&pl[0][0]);  // A x BX, planes no longer needed
+    float* rx = L.work;  // A x BX, the planes are no longer needed
+    static_assert(sizeof(L.work) / sizeof(float) >= (size_t)A * BX || A > 64, "roller exchange");
     float wetb = 1.0f;
     if (ftile) {
-        if (p.roller == 1) {
-            lds_barrier();  // the last plane reads of the rr pass are done
-            if (bsink) {
+        lds_barrier();  // the last plane and face reads are done, every row of the stash is written
+        if (rol && bsink) {
 #pragma unroll
-                for (int th = 0; th < A; th++) rx[th][cx] = ra[th];
+            for (int th = 0; th < A; th++) {
+                if (th >= nt) break;
+                rx[th * BX + cx] = ra[th];
             }
-            lds_barrier();
         }
+        lds_barrier();
         if (bsrc != 0) wetb = G(f.hh)[i] > p.eps ? 1.0f : 0.0f;
     }
-    if (NT > 0) {
 #pragma unroll
-        for (int th = 0; th < A; th++) ea[th] = stash[th][tid + bsrc];
-        if (bsrc != 0) {
+    for (int th = 0; th < A; th++) {
+        if (th >= nt) break;
+        ea[th] = L.stash[th][tid + bsrc];
+    }
+    if (!p.fold_rows) {
+        const int side = (y == 1) ? 0 : (y == ny - 2 ? 1 : -1);
+        if (valid && side >= 0) {
 #pragma unroll
-            for (int th = 0; th < A; th++) ea[th] = ea[th] * wetb;
-            if (p.roller == 1) {
-#pragma unroll
-                for (int th = 0; th < A; th++) ra[th] = rx[th][cx] * wetb;
+            for (int th = 0; th < A; th++) {
+                if (th >= nt) break;
+                G(f.bnd_e1)[((uint32_t)side * nt + th) * nx + x] = ea[th];
+                if (rol) G(f.bnd_r1)[((uint32_t)side * nt + th) * nx + x] = ra[th];
             }
+        }
+    }
+    if (bsrc != 0) {
+#pragma unroll
+        for (int th = 0; th < A; th++) {
+            if (th >= nt) break;
+            ea[th] = ea[th] * wetb;
+            if (rol) ra[th] = rx[th * BX + cx] * wetb;
         }
     }
     float Rv = 0.0f, DRv = 0.0f;
-    if (valid) dissip_cell<NT, CUR, true>(p, s, f, i, ea, ra, Rv, DRv);
+    if (valid) dissip_cell<A, EX, CUR, true>(p, s, f, L.dirs, i, ea, ra, Rv, DRv);
     if (ftile) {
         lds_barrier();  // every thread has read its row of the stash
         if (bsink) {
 #pragma unroll
-            for (int th = 0; th < A; th++) stash[th][tid] = ea[th];
+            for (int th = 0; th < A; th++) {
+                if (th >= nt) break;
+                L.stash[th][tid] = ea[th];
+            }
         }
         lds_barrier();
         if (bsrc != 0) {
 #pragma unroll
-            for (int th = 0; th < A; th++) ea[th] = stash[th][tid + bsrc] * wetb;
+            for (int th = 0; th < A; th++) {
+                if (th >= nt) break;
+                ea[th] = L.stash[th][tid + bsrc] * wetb;
+            }
         }
     }
     if (valid) {
-        finish_cell<NT, true>(p, s, f, i, ea, ra, Rv, DRv);
+        finish_cell<A, EX, true>(p, s, f, L.dirs, i, ea, ra, Rv, DRv);
     } else {
         wmin = 9999999.9f;
     }
     // block minimum: wavefront reduction, then across the WTY/... waves
     for (int o = 32; o > 0; o >>= 1) wmin = fmn(wmin, __shfl_xor(wmin, o, 64));
-    if ((tid & 63) == 0) wred[tid >> 6] = wmin;
+    if ((tid & 63) == 0) L.red[tid >> 6] = wmin;
     __syncthreads();
     if (tid == 0) {
-        float m = wred[0];
-        for (int w = 1; w < WTHREADS / 64; w++) m = fmn(m, wred[w]);
+        float m = L.red[0];
+        for (int w = 1; w < WTHREADS / 64; w++) m = fmn(m, L.red[w]);
         G(f.red_wave)[tile] = m;
     }
 }
@@ -896,25 +954,72 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi) {
 // fields ubnd1D writes, and ubnd1D none that it writes) the first workgroup
 // runs the offshore boundary beside the wave tiles, which take the
 // following ones (their XCD bands rotate by one XCD and stay contiguous).
-template <int NT, bool CUR, bool RQ>
-__global__ __launch_bounds__(WTHREADS, 4) void k_wave(KP p, SP s, Fld f, int offshore) {
+template <int A, bool EX, bool CUR, bool FLEX>
+__global__ __launch_bounds__(WTHREADS, wave_occ(A)) void k_wave(KP p, SP s, Fld f, int offshore) {
+    __shared__ WaveLds<A, CUR> lds;
     const int ntiles = p.wtiles_x * p.wtiles_y;
     const int off = !CUR && offshore ? 1 : 0;
     if (off && blockIdx.x == 0) {
-        offshore_wg(p, s, f, 1, threadIdx.x + threadIdx.y * BX, WTHREADS);
+        offshore_wg(p, s, f, 1, threadIdx.x + threadIdx.y * BX, WTHREADS, lds.work);
         return;
     }
-    wave_body<NT, CUR, RQ>(p, s, f, BI{xcd_tile((int)blockIdx.x - off, ntiles), 0});
+    wave_body<A, EX, CUR, FLEX>(p, s, f, BI{xcd_tile((int)blockIdx.x - off, ntiles), 0}, lds);
 }
+
+// The wave kernel of a number of bins: 12 and 24 have one with every count
+// known to the compiler; other counts run in the smallest of 12, 24, 36 and
+// 64 bins that holds them (registers and LDS are sized by it; one kernel of
+// 64 bins for all, its arrays in scratch, and its boundary rows in a launch
+// of their own took 57 + 34 us at 413 x 287 x 18).  flex: the
+// roller is off, or sigm or dtheta is not below 2.
+struct WaveK {
+    int A;
+    bool ex, cur, flex;
+    bool operator<(const WaveK& o) const {
+        return std::make_tuple(A, ex, cur, flex) < std::make_tuple(o.A, o.ex, o.cur, o.flex);
+    }
+};
+inline bool wave_flex(const KP& p, const SP& s) { return p.roller != 1 || !(s.sigm_recip && p.dth_recip); }
+inline WaveK wave_kernel(int nt, bool cur, bool flex) {
+    const int A = nt <= 12 ? 12 : (nt <= 24 ? 24 : (nt <= 36 ? 36 : MAXT));
+    return WaveK{A, !flex && (nt == 12 || nt == 24), cur, flex};
+}
+// the kernel of rows 0 / ny-1 does not depend on flex
+inline WaveK rows_kernel(WaveK k) { return WaveK{k.A, k.ex, k.cur, false}; }
+#define WAVE_SWITCH_A(C_, F_, k, RUN)                    \
+    switch ((k).A) {                                     \
+        case 12: RUN(12, false, C_, F_); break;          \
+        case 24: RUN(24, false, C_, F_); break;          \
+        case 36: RUN(36, false, C_, F_); break;          \
+        default: RUN(MAXT, false, C_, F_); break;        \
+    }
+#define WAVE_SWITCH(k_, RUN)                                            \
+    do {                                                                \
+        const WaveK wk_ = (k_);                                         \
+        if (wk_.ex) {                                                   \
+            if (wk_.A == 12) {                                          \
+                if (wk_.cur) RUN(12, true, true, false);                \
+                else RUN(12, true, false, false);                       \
+            } else {                                                    \
+                if (wk_.cur) RUN(24, true, true, false);                \
+                else RUN(24, true, false, false);                       \
+            }                                                           \
+        } else if (wk_.flex) {                                          \
+            if (wk_.cur) WAVE_SWITCH_A(true, true, wk_, RUN)            \
+            else WAVE_SWITCH_A(false, true, wk_, RUN)                   \
+        } else {                                                        \
+            if (wk_.cur) WAVE_SWITCH_A(true, false, wk_, RUN)           \
+            else WAVE_SWITCH_A(false, false, wk_, RUN)                  \
+        }                                                               \
+    } while (0)
 
 // Rows 0 and ny-1 (rollerlatbnd, wave_CPU.cpp:830-871): the post-Euler
 // ee/rr of rows 1 / ny-2 times the cell's wet flag, then the cell's own
 // energy..dissipation, and finally ee after dissipation copied again from
 // rows 1 / ny-2.
-template <int NT, bool CUR>
+template <int A, bool EX, bool CUR>
 XDEV void wave_rows_body(const KP& p, const SP& s, const Fld& f, BI bi) {
-    constexpr int A = NT > 0 ? NT : MAXT;
-    const int nt = NT > 0 ? NT : p.nt;
+    const int nt = EX ? A : p.nt;
     int x = bi.x * 256 + threadIdx.x;
     int side = bi.y;
     if (x >= p.nx) return;
@@ -932,22 +1037,13 @@ XDEV void wave_rows_body(const KP& p, const SP& s, const Fld& f, BI bi) {
         efin[th] = G(f.ee_out)[is + (size_t)th * N] * wet;
     }
     float Rv, DRv;
-    dissip_cell<NT, CUR>(p, s, f, i, e, r, Rv, DRv);
-    finish_cell<NT>(p, s, f, i, efin, r, Rv, DRv);
+    dissip_cell<A, EX, CUR, false>(p, s, f, f.dirs, i, e, r, Rv, DRv);
+    finish_cell<A, EX, false>(p, s, f, f.dirs, i, efin, r, Rv, DRv);
 }
-template <int NT, bool CUR>
+template <int A, bool EX, bool CUR>
 __global__ __launch_bounds__(256) void k_wave_rows(KP p, SP s, Fld f) {
-    wave_rows_body<NT, CUR>(p, s, f, BI{(int)blockIdx.x, (int)blockIdx.y});
+    wave_rows_body<A, EX, CUR>(p, s, f, BI{(int)blockIdx.x, (int)blockIdx.y});
 }
-
-// Values needed in registers at this point.  Stencils that read their
-// operands under data-dependent branches, or after stores the compiler
-// cannot prove independent, would issue each load after the branch or store
-// above it: one round trip to memory per level.  Their operands are loaded
-// into locals and named here, ahead of the first branch and store, so all
-// loads are in flight together.  The asm emits no instruction.
-XDEV void need(float a, float b, float c, float d) { asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d)); }
-XDEV void need(int a, int b, int c, int d) { asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d)); }
 
 // Operands of wavforceCPU (wave_CPU.cpp:1159-1223) at (x, y).
 struct WfOps {
@@ -2600,14 +2696,6 @@ const char kFieldNames[] =
 
 // defer_force: the flow step follows and forms the wave forces in its first
 // launch
-template <int NT, bool CUR>
-int launch_k_wave(xbg_ctx* c, const SP& s, bool rq, dim3 gw, dim3 bw, int offshore = 0) {
-    if (offshore) gw.x += 1;
-    if (rq) LAUNCH(c, "k_wave", (k_wave<NT, CUR, true>), gw, bw, c->kp, s, c->f, offshore);
-    else LAUNCH(c, "k_wave", (k_wave<NT, CUR, false>), gw, bw, c->kp, s, c->f, offshore);
-    return 0;
-}
-
 int launch_wave(xbg_ctx* c, const SP& s, int offshore = 0, int defer_force = 0) {
     KP& p = c->kp;
     dim3 g = grid2(p);
@@ -2621,34 +2709,15 @@ int launch_wave(xbg_ctx* c, const SP& s, int offshore = 0, int defer_force = 0) 
     const int off_w = c->pre_disp && offshore && !cur ? 1 : 0;
     if (c->pre_disp && offshore && cur)
         LAUNCH(c, "k_bnd_offshore", k_bnd_offshore, dim3(1), dim3(1024), p, s, c->f, 1);
-    dim3 gr((p.nx + 255) / 256, 2, 1);
-    dim3 gw(p.wtiles_x * p.wtiles_y, 1, 1), bw(BX, WTY, 1);
-    // wci == 0 (the reference default): the current-free kernel
-    const bool rq = s.sigm_recip && p.dth_recip;
-    int rc = 0;
-    switch (p.nt) {
-        case 12:
-            rc = cur ? launch_k_wave<12, true>(c, s, rq, gw, bw) : launch_k_wave<12, false>(c, s, rq, gw, bw, off_w);
-            if (rc) return rc;
-            if (!p.fold_rows) {
-                if (cur) LAUNCH(c, "k_wave_rows", (k_wave_rows<12, true>), gr, dim3(256), p, s, c->f);
-                else LAUNCH(c, "k_wave_rows", (k_wave_rows<12, false>), gr, dim3(256), p, s, c->f);
-            }
-            break;
-        case 24:
-            rc = cur ? launch_k_wave<24, true>(c, s, rq, gw, bw) : launch_k_wave<24, false>(c, s, rq, gw, bw, off_w);
-            if (rc) return rc;
-            if (!p.fold_rows) {
-                if (cur) LAUNCH(c, "k_wave_rows", (k_wave_rows<24, true>), gr, dim3(256), p, s, c->f);
-                else LAUNCH(c, "k_wave_rows", (k_wave_rows<24, false>), gr, dim3(256), p, s, c->f);
-            }
-            break;
-        default:
-            rc = cur ? launch_k_wave<0, true>(c, s, rq, gw, bw) : launch_k_wave<0, false>(c, s, rq, gw, bw, off_w);
-            if (rc) return rc;
-            if (cur) LAUNCH(c, "k_wave_rows", (k_wave_rows<0, true>), gr, dim3(256), p, s, c->f);
-            else LAUNCH(c, "k_wave_rows", (k_wave_rows<0, false>), gr, dim3(256), p, s, c->f);
-            break;
+    const dim3 gr((p.nx + 255) / 256, 2, 1), gw(p.wtiles_x * p.wtiles_y + off_w, 1, 1), bw(BX, WTY, 1);
+    const WaveK k = wave_kernel(p.nt, cur, wave_flex(p, s));
+#define RUN(A_, EX_, C_, F_) LAUNCH(c, "k_wave", (k_wave<A_, EX_, C_, F_>), gw, bw, p, s, c->f, off_w)
+    WAVE_SWITCH(k, RUN);
+#undef RUN
+    if (!p.fold_rows) {
+#define RUN(A_, EX_, C_, F_) LAUNCH(c, "k_wave_rows", (k_wave_rows<A_, EX_, C_>), gr, dim3(256), p, s, c->f)
+        WAVE_SWITCH(rows_kernel(k), RUN);
+#undef RUN
     }
     if (!defer_force) LAUNCH(c, "k_wave_force", k_wave_force, g, blk2, p, c->f);
     c->cur = 1 - c->cur;
@@ -3591,20 +3660,23 @@ __global__ __launch_bounds__(256) void kb_dispersion(DTab tab, TMap map, int nti
 // single-domain launch gives the tile) and are skipped.  One tile per
 // workgroup: the wave kernel sits at the 128-VGPR limit of its two
 // workgroups per CU, and a tile loop around it spills.
-template <int NT, bool CUR, bool RQ>
-__global__ __launch_bounds__(WTHREADS, 4) void kb_wave(DTab tab, TMap map, int ntiles) {
+template <int A, bool EX, bool CUR, bool FLEX>
+__global__ __launch_bounds__(WTHREADS, wave_occ(A)) void kb_wave(DTab tab, TMap map, int ntiles) {
     const TileEnt e = map[blockIdx.x];
     if (e.bx < 0) return;
     const DomDesc& D = tab[e.dom];
-    if (D.status == ENS_ACTIVE) wave_body<NT, CUR, RQ>(D.p, D.s, D.f[D.par][PH_START], BI{e.bx, 0});
+    if (D.status == ENS_ACTIVE) {
+        __shared__ WaveLds<A, CUR> lds;
+        wave_body<A, EX, CUR, FLEX>(D.p, D.s, D.f[D.par][PH_START], BI{e.bx, 0}, lds);
+    }
 }
 
-template <int NT, bool CUR>
+template <int A, bool EX, bool CUR>
 __global__ __launch_bounds__(256) void kb_wave_rows(DTab tab, TMap map, int ntiles) {
     ENS_FOR_TILES(map, ntiles) {
         const TileEnt e = map[t_];
         const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) wave_rows_body<NT, CUR>(D.p, D.s, D.f[D.par][PH_START], BI{e.bx, e.by});
+        if (D.status == ENS_ACTIVE) wave_rows_body<A, EX, CUR>(D.p, D.s, D.f[D.par][PH_START], BI{e.bx, e.by});
     }
 }
 
@@ -3927,8 +3999,7 @@ struct TileMap {
 };
 
 struct WaveGroup {
-    int nt;
-    bool cur, rq;
+    WaveK k;
     TileMap map;
 };
 
@@ -4016,13 +4087,6 @@ int grid_of(const xbg_ens* e, int k, int ntiles) {
     return g < ntiles ? g : ntiles;
 }
 
-template <int NT, bool CUR>
-void launch_wave_group(xbg_ens* e, const WaveGroup& w, int grid) {
-    grid = w.map.n;  // one workgroup per tile (kb_wave has no tile loop)
-    if (w.rq) kb_wave<NT, CUR, true><<<dim3(grid), dim3(BX, WTY), 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-    else kb_wave<NT, CUR, false><<<dim3(grid), dim3(BX, WTY), 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-}
-
 void ens_ev(xbg_ens* e, int slot) {
     if (e->prof) hipEventRecord(e->ev[slot], e->stream);
 }
@@ -4051,33 +4115,20 @@ int ens_launch_step(xbg_ens* e) {
     }
     ens_ev(e, 2 * EK_WAVE);
     for (const WaveGroup& w : e->waves) {
-        int g = grid_of(e, EK_WAVE, w.map.n);
-        if (w.nt == 12) {
-            if (w.cur) launch_wave_group<12, true>(e, w, g);
-            else launch_wave_group<12, false>(e, w, g);
-        } else if (w.nt == 24) {
-            if (w.cur) launch_wave_group<24, true>(e, w, g);
-            else launch_wave_group<24, false>(e, w, g);
-        } else {
-            if (w.cur) launch_wave_group<0, true>(e, w, g);
-            else launch_wave_group<0, false>(e, w, g);
-        }
+        // one workgroup per tile (kb_wave has no tile loop)
+#define RUN(A_, EX_, C_, F_) \
+    kb_wave<A_, EX_, C_, F_><<<dim3(w.map.n), dim3(BX, WTY), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
+        WAVE_SWITCH(w.k, RUN);
+#undef RUN
     }
     ens_ev(e, 2 * EK_WAVE + 1);
     ens_ev(e, 2 * EK_ROWS);
     for (const WaveGroup& w : e->rows) {
-        int g = grid_of(e, EK_ROWS, w.map.n);
-        dim3 b(256);
-        if (w.nt == 12) {
-            if (w.cur) kb_wave_rows<12, true><<<dim3(g), b, 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-            else kb_wave_rows<12, false><<<dim3(g), b, 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-        } else if (w.nt == 24) {
-            if (w.cur) kb_wave_rows<24, true><<<dim3(g), b, 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-            else kb_wave_rows<24, false><<<dim3(g), b, 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-        } else {
-            if (w.cur) kb_wave_rows<0, true><<<dim3(g), b, 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-            else kb_wave_rows<0, false><<<dim3(g), b, 0, e->stream>>>(e->dtab, w.map.d, w.map.n);
-        }
+        const int g = grid_of(e, EK_ROWS, w.map.n);
+#define RUN(A_, EX_, C_, F_) \
+    kb_wave_rows<A_, EX_, C_><<<dim3(g), dim3(256), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
+        WAVE_SWITCH(w.k, RUN);
+#undef RUN
     }
     ens_ev(e, 2 * EK_ROWS + 1);
     const TileMap& m2 = e->m_2d;
@@ -4158,7 +4209,7 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
     for (int k = 0; k < EK_N; k++) e->grid_sel[k] = 0;
     std::vector<int> doms_all, gx2, gy2, gxc, gyc, gxcfl, gycfl;
     std::vector<TileEnt> cfl;
-    std::map<std::tuple<int, bool, bool>, std::vector<TileEnt>> wave_tiles, row_tiles;
+    std::map<WaveK, std::vector<TileEnt>> wave_tiles, row_tiles;
     e->h.resize(ndom);
     for (int d = 0; d < ndom; d++) {
         xbg_ctx* c = ctxs[d];
@@ -4222,19 +4273,19 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
         D.cfl_first = (int)cfl.size();
         D.cfl_count = ncfl;
         for (int k = 0; k < ncfl; k++) cfl.push_back(TileEnt{d, k, 0, 0});
-        const int nt = (p.nt == 12 || p.nt == 24) ? p.nt : 0;
-        const bool cur = p.wci != 0.0f;
-        float sigm = (float)(2 * PI_ / (double)(float)r.Trep);
-        const bool rq = (sigm > 0.0f && sigm < 2.0f) && p.dth_recip;
+        SP sp{};
+        sp.sigm = (float)(2 * PI_ / (double)(float)r.Trep);
+        sp.sigm_recip = sp.sigm > 0.0f && sp.sigm < 2.0f ? 1 : 0;
+        const WaveK wk = wave_kernel(p.nt, p.wci != 0.0f, wave_flex(p, sp));
         // wave tiles in the XCD order of the single-domain launch: the
         // domain's run starts on a multiple of 8 entries, padded with
         // entries of an idle domain slot (-1 -> skipped below)
-        auto& wv = wave_tiles[std::make_tuple(nt, cur, rq)];
+        auto& wv = wave_tiles[wk];
         while (wv.size() % 8) wv.push_back(TileEnt{d, -1, 0, 0});
         const int ntw = p.wtiles_x * p.wtiles_y;
         for (int b = 0; b < ntw; b++) wv.push_back(TileEnt{d, xcd_tile(b, ntw), 0, 0});
-        if (!p.fold_rows || nt == 0) {
-            auto& rv = row_tiles[std::make_tuple(nt, cur, false)];
+        if (!p.fold_rows) {
+            auto& rv = row_tiles[rows_kernel(wk)];
             for (int side = 0; side < 2; side++)
                 for (int bx = 0; bx < (p.nx + 255) / 256; bx++) rv.push_back(TileEnt{d, bx, side, 0});
         }
@@ -4263,12 +4314,12 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
         if ((rc = upload_map(e, e->m_conc[sh], cv))) return bail(rc);
     }
     for (auto& kv : wave_tiles) {
-        WaveGroup w{std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first), TileMap{}};
+        WaveGroup w{kv.first, TileMap{}};
         if ((rc = upload_map(e, w.map, kv.second))) return bail(rc);
         e->waves.push_back(w);
     }
     for (auto& kv : row_tiles) {
-        WaveGroup w{std::get<0>(kv.first), std::get<1>(kv.first), false, TileMap{}};
+        WaveGroup w{kv.first, TileMap{}};
         if ((rc = upload_map(e, w.map, kv.second))) return bail(rc);
         e->rows.push_back(w);
     }
