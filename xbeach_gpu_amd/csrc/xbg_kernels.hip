@@ -41,6 +41,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <string>
 #include <vector>
 
@@ -351,6 +352,30 @@ XDEV float face_flux(float cg, float lo, float lo2, float hi, float hi2) {
     return upw2d(pos ? lo : hi, pos ? lo2 : hi2) * cg;
 }
 
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+// A directional plane as a buffer: an access takes the plane's base from scalar
+// registers and one 32-bit byte offset per lane.
+XDEV rsrc_t plane_rsrc(const float* base, uint32_t N) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(N * 4u), 0x00027000);
+}
+XDEV float buf_load(rsrc_t r, int off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+// a pointer that is the same in every lane, in scalar registers
+template <class T>
+XDEV T* uniform_ptr(T* q) {
+    const uint64_t b = (uint64_t)q;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    return (T*)(((uint64_t)hi << 32) | lo);
+}
+// the next plane of a directional field (plane 0: q itself); opaque, so that
+// the addresses of every plane are not formed (and held) ahead of the bin loop
+template <class T>
+XDEV T* plane_next(T* q, int th, uint32_t N) {
+    uint64_t b = (uint64_t)q + (th ? (uint64_t)N * 4 : 0);
+    asm volatile("" : "+s"(b));
+    return (T*)b;
+}
 // roelvinkCPU (wave_CPU.cpp:932-985): Qb and D in double as written.
 XDEV float roelvink_cell(const KP& p, float Trep, float E, float h, float k, float fw) {
     float fac = (float)(8.0 / (double)p.rho / (double)p.g);
@@ -379,17 +404,35 @@ XDEV float baldock_cell(const KP& p, float Trep, float Ht, float h, float k, flo
 // (wave_CPU.cpp:873-1089) at cell i: e (action after Euler) -> ee after
 // dissipation, r (roller after Euler) -> rr after dissipation.
 // A bins at most: p.nt of them, A itself when EX.
-template <int A, bool EX, bool CUR, bool L>
-XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, float* e, float* r,
+// The ee bins are an array of the thread, or a column of LDS (stride STRIDE
+// floats): in the wave kernel they stay there, 24 registers that its sweep and
+// this routine do not have to find.
+struct RegBins {
+    float* a;
+    XDEV float get(int th) const { return a[th]; }
+    XDEV void set(int th, float v) const { a[th] = v; }
+};
+template <int STRIDE>
+struct LdsBins {
+    float* a;
+    XDEV float get(int th) const { return a[th * STRIDE]; }
+    XDEV void set(int th, float v) const { a[th * STRIDE] = v; }
+};
+template <int A, bool EX, bool CUR, bool L, class B>
+XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const B e, float* r,
                       float& Rout, float& DRout) {
     const int nt = EX ? A : p.nt;
     float h = G(f.hh)[i];
     float Et = 0.0f;
+    uint32_t m = 0xffffffffu;
 #pragma unroll
     for (int th = 0; th < A; th++) {
         if (th >= nt) break;
-        e[th] = fmx(e[th] * s.sigm, 0.0f);
-        Et = Et + e[th];
+        const float v = fmx(e.get(th) * s.sigm, 0.0f);
+        e.set(th, v);
+        Et = Et + v;
+        // smallest magnitude that is not zero (zero wraps to the largest)
+        if (!CUR) m = min(m, min((__float_as_uint(v) << 1) - 1u, (__float_as_uint(r[th]) << 1) - 1u));
     }
     Et = Et * p.dtheta;
     float Ht = sqrtf(Et / (p.rho * p.g / 8.0f));
@@ -415,32 +458,52 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
 #pragma unroll
         for (int th = 0; th < A; th++) {
             if (th >= nt) break;
-            e[th] = e[th] / idiv;
+            e.set(th, e.get(th) / idiv);
         }
     }
+    // The two divisions and the square root of a bin: E is the divisor of
+    // every bin of the cell, and without the current the square root is the
+    // cell's c times sqrt(cos^2 + sin^2) of the bin, which rounds near c; so
+    // the IEEE results come from a few double operations on per-cell
+    // reciprocals (20 instead of 36 instructions a bin), where no quotient
+    // can be subnormal: in the wavefronts whose cells have c in range, no
+    // bin between zero and 2^-90 (before energint's cap), and factors of at
+    // least 2^-30.  The wave kernel at 2048 x 1024 x 24: 366 -> 353 us with the
+    // ee bins left in LDS; asking each quotient instead cost more than it
+    // saved (376 us).
+    const float gb = 2.0f * p.g * p.beta;
+    const bool fast = !CUR && cc > 1e-10f && cc < 1e10f && !(Dv != 0.0f && Dv < 9.3e-10f * Emx) &&
+                      (gb == 0.0f || gb >= 1e-5f * cc) && idiv < 1e6f && m >= (__float_as_uint(8.1e-28f) << 1);
+    auto bins = [&](auto near_c) {
+        constexpr bool NEAR = decltype(near_c)::value;
+        const double rE = 1.0 / (double)Emx, c0 = (double)cc, rc = 1.0 / c0, hc = 0.5 * rc;
 #pragma unroll
-    for (int th = 0; th < A; th++) {
-        if (th >= nt) break;
-        float eet = e[th];
-        float cx = CUR ? cc * dtab<L>(dirs, 1, th) + uui : cc * dtab<L>(dirs, 1, th);
-        float cy = CUR ? cc * dtab<L>(dirs, 2, th) + vvi : cc * dtab<L>(dirs, 2, th);
-        float dd = eet * Dv / Emx;
-        float rrt;
-        if (wetc) {
-            rrt = r[th];
-            float rrd = 2.0f * p.g * p.beta * rrt / sqrtf(cx * cx + cy * cy);
-            eet = fmx(eet - s.dt * dd, 0.0f);
-            rrt = fmx(rrt + s.dt * (dd - rrd), 0.0f);
-            drr = drr + rrd;
-        } else {
-            eet = 0.0f;
-            rrt = 0.0f;
-            drr = 0.0f;
+        for (int th = 0; th < A; th++) {
+            if (th >= nt) break;
+            float eet = e.get(th);
+            float cx = CUR ? cc * dtab<L>(dirs, 1, th) + uui : cc * dtab<L>(dirs, 1, th);
+            float cy = CUR ? cc * dtab<L>(dirs, 2, th) + vvi : cc * dtab<L>(dirs, 2, th);
+            float dd = NEAR ? xm::div_by(eet * Dv, rE) : eet * Dv / Emx;
+            float rrt;
+            if (wetc) {
+                rrt = r[th];
+                const float num = gb * rrt, s2 = cx * cx + cy * cy;
+                const float rrd = NEAR ? xm::div_near(num, xm::sqrt_near(s2, c0, hc), rc) : num / sqrtf(s2);
+                eet = fmx(eet - s.dt * dd, 0.0f);
+                rrt = fmx(rrt + s.dt * (dd - rrd), 0.0f);
+                drr = drr + rrd;
+            } else {
+                eet = 0.0f;
+                rrt = 0.0f;
+                drr = 0.0f;
+            }
+            RR = RR + rrt;
+            e.set(th, eet);
+            r[th] = rrt;
         }
-        RR = RR + rrt;
-        e[th] = eet;
-        r[th] = rrt;
-    }
+    };
+    if (!CUR && __all(fast)) bins(std::true_type{});
+    else bins(std::false_type{});
     Rout = RR * p.dtheta;
     DRout = drr * p.dtheta;
 }
@@ -448,8 +511,8 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
 // meandirCPU (wave_CPU.cpp:1092-1116), radstressCPU (1118-1157) and
 // breakerdelayCPU (1334-1374, called with R) at cell i on the final ee/rr;
 // stores the directional state of the cell.
-template <int A, bool EX, bool L>
-XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const float* efin,
+template <int A, bool EX, bool L, class B>
+XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const B efin,
                       const float* r, float Rv, float DRv) {
     const int nt = EX ? A : p.nt;
     const size_t N = p.N;
@@ -459,7 +522,7 @@ XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
 #pragma unroll
     for (int th = 0; th < A; th++) {
         if (th >= nt) break;
-        float ev = efin[th], rv = r[th];
+        float ev = efin.get(th), rv = r[th];
         sume = sume + ev;
         sumethet = sumethet + ev * dtab<L>(dirs, 0, th);
         txx = txx + (dtab<L>(dirs, 3, th) * ev);   // (1 + cs*cs) * ev
@@ -538,31 +601,6 @@ constexpr int NSLOT = (PN + WTHREADS - 1) / WTHREADS;
 static_assert(NSLOT == 2, "two slots: one per thread, the rest on the last wavefronts");
 XDEV int slot_of(int it, int tid) { return it == 0 ? tid : 2 * WTHREADS - 1 - tid; }
 
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-XDEV rsrc_t plane_rsrc(const float* base, uint32_t N) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(N * 4u), 0x00027000);
-}
-XDEV float buf_load(rsrc_t r, int off) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-XDEV void buf_store(rsrc_t r, int off, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, off, 0, 0);
-}
-// a pointer that is the same in every lane, in scalar registers
-template <class T>
-XDEV T* uniform_ptr(T* q) {
-    const uint64_t b = (uint64_t)q;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-    return (T*)(((uint64_t)hi << 32) | lo);
-}
-// plane th of a directional field; the bin index is opaque, so that the
-// addresses of every plane are not formed (and held) ahead of the bin loop
-XDEV rsrc_t plane_of(const float* field, int th, uint32_t N) {
-    int thv = th;
-    asm volatile("" : "+s"(thv));
-    return plane_rsrc(field + (size_t)(uint32_t)thv * N, N);
-}
-
 // The value of the lane to the left; lane 0 gets first.
 XDEV float from_left(float v, float first) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, first), __builtin_bit_cast(int, v),
@@ -609,10 +647,10 @@ struct WaveLds {
 // lane to the left and its bottom face through LDS, one bin later, behind the
 // bin's barrier.
 //
-// Bound by VALU issue: at 2048 x 1024 x 24 the whole kernel takes 392 us, and
-// took 460 with a sweep per field, each behind its own barriers, the face
-// operands read from LDS behind the upwind test and the staged elements
-// addressed with 64-bit arithmetic in every lane.
+// Bound by VALU issue: at 2048 x 1024 x 24 the whole kernel took 460 us with a
+// sweep per field, each behind its own barriers, the face operands read from
+// LDS behind the upwind test and the staged elements addressed with 64-bit
+// arithmetic in every lane, and 392 us as one sweep.
 //
 // A, EX: at most A bins, p.nt of them (A exactly when EX).  FLEX: the roller
 // switch and the divisions by sigm and dtheta decided at run time; otherwise
@@ -655,7 +693,8 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
     }
     float re[NSLOT], rs[NSLOT] = {}, rr[NSLOT] = {};
     auto load = [&](int th) {
-        const rsrc_t qe = plane_of(pe, th, N);
+        pe = plane_next(pe, th, N);
+        const rsrc_t qe = plane_rsrc(pe, N);
 #pragma unroll
         for (int it = 0; it < NSLOT; it++) re[it] = buf_load(qe, off[it]);
         if (first) {
@@ -663,7 +702,8 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
             for (int it = 0; it < NSLOT; it++) rs[it] = gload(f.St + (uint32_t)(sto[it] + th * ny));
         }
         if (rol) {
-            const rsrc_t qr = plane_of(pr, th, N);
+            pr = plane_next(pr, th, N);
+            const rsrc_t qr = plane_rsrc(pr, N);
 #pragma unroll
             for (int it = 0; it < NSLOT; it++) rr[it] = buf_load(qr, off[it]);
         }
@@ -676,7 +716,10 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
             const int l = slot_of(it, tid);
             if (it == 0 || l < PN) {
                 float v = re[it];
-                if (first) v = offs[it] ? rs[it] * s.taper : v;
+                if (first) {
+                    asm volatile("");  // a branch: few tiles hold the offshore column
+                    v = offs[it] ? rs[it] * s.taper : v;
+                }
                 v = fmx(v, 0.000f);  // sanity + action (wave_CPU.cpp:58-82, 289-309)
                 de[l] = div(v, s.rsigm, s.sigm, s.sigm_recip);
                 if (rol) dr[l] = rr[it];
@@ -853,7 +896,8 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
     const bool rol = FLEX ? p.roller == 1 : true;
     for (int l = tid; l < 8 * MAXT; l += WTHREADS) L.dirs[l] = G(f.dirs)[l];
     __syncthreads();
-    float ra[A], ea[A];
+    float ra[A];
+    const LdsBins<WTHREADS> ee{&L.stash[0][tid]};
     // WAVEDT (Wave_kernel.cu:232-249): min over bins of CFL*dtheta/|ctheta|.
     // Rounded division is monotonic in the divisor, so this equals one
     // division by the largest |ctheta| (NaN speeds ignored as fminf does).
@@ -877,8 +921,19 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
     const int bsrc = !ftile || !valid ? 0 : (y == 0 ? BX : (y == ny - 1 ? -BX : 0));
     const bool bsink = valid && ((y0 == 0 && cy == 1) || y == ny - 2);
     float* rx = L.work;  // A x BX, the planes are no longer needed
-    static_assert(sizeof(L.work) / sizeof(float) >= (size_t)A * BX || A > 64, "roller exchange");
+    static_assert(sizeof(L.work) / sizeof(float) >= (size_t)A * BX, "roller exchange");
     float wetb = 1.0f;
+    if (!p.fold_rows) {
+        const int side = (y == 1) ? 0 : (y == ny - 2 ? 1 : -1);
+        if (valid && side >= 0) {
+#pragma unroll
+            for (int th = 0; th < A; th++) {
+                if (th >= nt) break;
+                G(f.bnd_e1)[((uint32_t)side * nt + th) * nx + x] = ee.get(th);
+                if (rol) G(f.bnd_r1)[((uint32_t)side * nt + th) * nx + x] = ra[th];
+            }
+        }
+    }
     if (ftile) {
         lds_barrier();  // the last plane and face reads are done, every row of the stash is written
         if (rol && bsink) {
@@ -888,55 +943,37 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
                 rx[th * BX + cx] = ra[th];
             }
         }
-        lds_barrier();
-        if (bsrc != 0) wetb = G(f.hh)[i] > p.eps ? 1.0f : 0.0f;
-    }
-#pragma unroll
-    for (int th = 0; th < A; th++) {
-        if (th >= nt) break;
-        ea[th] = L.stash[th][tid + bsrc];
-    }
-    if (!p.fold_rows) {
-        const int side = (y == 1) ? 0 : (y == ny - 2 ? 1 : -1);
-        if (valid && side >= 0) {
+        if (bsrc != 0) {
+            wetb = G(f.hh)[i] > p.eps ? 1.0f : 0.0f;
 #pragma unroll
             for (int th = 0; th < A; th++) {
                 if (th >= nt) break;
-                G(f.bnd_e1)[((uint32_t)side * nt + th) * nx + x] = ea[th];
-                if (rol) G(f.bnd_r1)[((uint32_t)side * nt + th) * nx + x] = ra[th];
+                ee.set(th, L.stash[th][tid + bsrc] * wetb);
             }
         }
-    }
-    if (bsrc != 0) {
+        lds_barrier();
+        if (rol && bsrc != 0) {
 #pragma unroll
-        for (int th = 0; th < A; th++) {
-            if (th >= nt) break;
-            ea[th] = ea[th] * wetb;
-            if (rol) ra[th] = rx[th * BX + cx] * wetb;
+            for (int th = 0; th < A; th++) {
+                if (th >= nt) break;
+                ra[th] = rx[th * BX + cx] * wetb;
+            }
         }
     }
     float Rv = 0.0f, DRv = 0.0f;
-    if (valid) dissip_cell<A, EX, CUR, true>(p, s, f, L.dirs, i, ea, ra, Rv, DRv);
+    if (valid) dissip_cell<A, EX, CUR, true>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
     if (ftile) {
-        lds_barrier();  // every thread has read its row of the stash
-        if (bsink) {
-#pragma unroll
-            for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
-                L.stash[th][tid] = ea[th];
-            }
-        }
-        lds_barrier();
+        lds_barrier();  // the source rows' bins after dissipation are in the stash
         if (bsrc != 0) {
 #pragma unroll
             for (int th = 0; th < A; th++) {
                 if (th >= nt) break;
-                ea[th] = L.stash[th][tid + bsrc] * wetb;
+                ee.set(th, L.stash[th][tid + bsrc] * wetb);
             }
         }
     }
     if (valid) {
-        finish_cell<A, EX, true>(p, s, f, L.dirs, i, ea, ra, Rv, DRv);
+        finish_cell<A, EX, true>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
     } else {
         wmin = 9999999.9f;
     }
@@ -1037,8 +1074,8 @@ XDEV void wave_rows_body(const KP& p, const SP& s, const Fld& f, BI bi) {
         efin[th] = G(f.ee_out)[is + (size_t)th * N] * wet;
     }
     float Rv, DRv;
-    dissip_cell<A, EX, CUR, false>(p, s, f, f.dirs, i, e, r, Rv, DRv);
-    finish_cell<A, EX, false>(p, s, f, f.dirs, i, efin, r, Rv, DRv);
+    dissip_cell<A, EX, CUR, false>(p, s, f, f.dirs, i, RegBins{e}, r, Rv, DRv);
+    finish_cell<A, EX, false>(p, s, f, f.dirs, i, RegBins{efin}, r, Rv, DRv);
 }
 template <int A, bool EX, bool CUR>
 __global__ __launch_bounds__(256) void k_wave_rows(KP p, SP s, Fld f) {

@@ -276,6 +276,30 @@ XM_FN double pow(double x, double y) {
     return sign * exp(y * log(a));
 }
 
+// ---- correctly rounded float operations through double ----
+// With a in double exactly, a few double operations that leave a relative
+// error below 2^-51 give the IEEE float result, since no exact result that is
+// not itself a float lies that near to a midpoint between floats: a square
+// root of a float no nearer than 2^-51 (relative), a normal quotient of two
+// floats no nearer than 2^-49.  A subnormal quotient can be an exact midpoint:
+// subnormal results of div_by and div_near are to be formed by a division.
+
+// sqrt(s) for a float s within a factor 1 +- 2^-20 of c*c, c a float in
+// [1e-10, 1e10], hc = 0.5 / (double)c: with s = c^2 + d and t = d / (2c),
+// sqrt(s) = c + t - t^2/(2c) + ..., the next term below 2^-62 of c; d is exact.
+XM_FN float sqrt_near(float s, double c, double hc) {
+    const double d = __builtin_fma(-c, c, (double)s), t = d * hc;
+    return (float)__builtin_fma(t, __builtin_fma(-t, hc, 1.0), c);
+}
+// a / q for a float q within a factor 1 +- 2^-20 of c, rc = 1 / (double)c:
+// 1/q = rc (1 + e + e^2 + ..), e = 1 - q rc.
+XM_FN float div_near(float a, float q, double rc) {
+    const double e = __builtin_fma(-(double)q, rc, 1.0);
+    return (float)((double)a * __builtin_fma(rc, __builtin_fma(e, e, e), rc));
+}
+// a / b with rb = 1 / (double)b
+XM_FN float div_by(float a, double rb) { return (float)((double)a * rb); }
+
 // ---- float entry points: one rounding of the double result ----
 XM_FN float expf(float x) { return (float)exp((double)x); }
 XM_FN float logf(float x) { return (float)log((double)x); }
