@@ -1845,8 +1845,10 @@ XDEV void calcuvvu_ops(const CuOps& q, float* o) {
     float wu = (float)(q.w_i & 1), wv = (float)((q.w_i >> 1) & 1);
     float vu = 0.25f * (q.v_b + q.v_i + q.v_rb + q.v_r) * wu;
     float uv = 0.25f * (q.u_l + q.u_i + q.u_lt + q.u_t) * wv;
-    float si = xm::sinf(q.tm_i), ci = xm::cosf(q.tm_i), sr = xm::sinf(q.tm_r), cr = xm::cosf(q.tm_r);
-    float st = xm::sinf(q.tm_t), ctt = xm::cosf(q.tm_t);
+    float si, ci, sr, cr, st, ctt;
+    xm::sincosf(q.tm_i, si, ci);
+    xm::sincosf(q.tm_r, sr, cr);
+    xm::sincosf(q.tm_t, st, ctt);
     float usi = q.us_i, usr = q.us_r, ust_t = q.us_t;
     float vsu = 0.5f * (usi * si + usr * sr) * wu;
     float usu = 0.5f * (usi * ci + usr * cr) * wu;
@@ -1909,16 +1911,13 @@ __global__ __launch_bounds__(256) void k_flow_uvvu(KP p, SP s, Fld f, int want_u
 // ---------------------------------------------------------------------------
 
 // xm::powf(x, y) for a base x > 0 (finite or +inf) whose double log lx =
-// xm::log((double)x) is given: the special cases in xm::pow's order, then
-// its exp(y * log(x)); two powers of one base share the log.
+// xm::log((double)x) is given: xm::pow's cases, then its exp(y * log(x)); two
+// powers of one base share the log.
 XDEV float powf_pos(float x, float y, double lx) {
     const double a = (double)x, yy = (double)y;
-    if (yy == 0.0 || a == 1.0) return 1.0f;
-    if (yy != yy) return (float)xm::nan_();
-    if (yy == 2.0) return (float)(a * a);
-    if (yy == 3.0) return (float)(a * a * a);
-    if (a == xm::inf_()) return yy > 0.0 ? (float)xm::inf_() : 0.0f;
-    return (float)(1.0 * xm::exp(yy * lx));
+    if (yy == 0.0 || yy == 2.0 || yy == 3.0 || yy == 4.0 || yy == 8.0 || yy - yy != 0.0 || a == xm::inf_())
+        return xm::powf(x, y);
+    return (float)xm::exp(yy * lx);
 }
 
 // Rvr (Sediment_kernel.cu:477-510) at cell i
@@ -1936,8 +1935,10 @@ XDEV float rvr_ops(const KP& p, const SP& s, float c, float H, float h, float ur
         const double lu = xm::log((double)Ur);
         float Bm = m1c + (m2c - m1c) / (1.0f + bet * powf_pos(Ur, alph, lu));
         float B1 = (float)((double)(-90.0f + 90.0f * xm::tanhf(m5c / powf_pos(Ur, m6c, lu))) * PI_ / 180.0);
-        float Sk = Bm * xm::cosf(B1);
-        float As = Bm * xm::sinf(B1);
+        float sB, cB;
+        xm::sincosf(B1, sB, cB);
+        float Sk = Bm * cB;
+        float As = Bm * sB;
         return (p.facsk * Sk - p.facas * As) * urms;
     }
     float Bm = m1c + (m2c - m1c) / (1.0f + bet * xm::powf(Ur, alph));
@@ -2004,7 +2005,8 @@ XDEV void sed_flux_body(const KP& p, const SP& s, const Fld& f, int ua_ready, BI
     need(hv, hh_i, DR_i, hv);
     float rol = rol_i + s.dt * (fabsf(dzsdt_i) - p.beta * c_i);
     G(f.rolthick)[i] = fmx(rol, 0.0f);
-    float ctm = xm::cosf(tm), stm = xm::sinf(tm);
+    float ctm, stm;
+    xm::sincosf(tm, stm, ctm);
     float uau = (float)(0.5 * (double)ctm * (double)(uai + uar));
     float uav = (float)(0.5 * (double)stm * (double)(uar + uai));
     float urep = ueu_i + uau;

@@ -7,24 +7,29 @@
 // HIP step reproduce its CPU oracle bit for bit, both use these functions.
 //
 // Every function is evaluated in double precision with only IEEE add,
-// subtract, multiply, divide and (where noted) sqrt, in a fixed operation
-// order and without FMA contraction (both sides compile with
-// -ffp-contract=off), so host and device produce identical bits.  The float
-// entry points round the double result once; they agree with a correctly
-// rounded libm except in double-rounding cases (about one input in 2^28).
+// subtract, multiply, fused multiply-add, divide and exact scaling, in a fixed
+// operation order; a multiply-add is fused where it is written so and nowhere
+// else (both sides compile with -ffp-contract=off), so host and device produce
+// identical bits.  The float entry points round the double result once; they
+// agree with a correctly rounded libm except in double-rounding cases (about
+// one input in 2^28).
 //
-// Methods (published):
-//   exp   Cody-Waite reduction by ln2 and the rational form of the remainder
-//         used by fdlibm/FreeBSD e_exp.c (Remez polynomial on [0, 0.347])
-//   log   reduction to [sqrt(1/2), sqrt(2)), s = f/(2+f), Remez series of
-//         fdlibm e_log.c
+// Methods.  The polynomials interpolate their functions at Chebyshev points
+// (relative error of the result below 2e-17, fitted in extended precision).
+//   exp   reduction by ln2 (two-part constant), 1 + r + r^2 Q(r), |r| <= ln2/2
+//   sinh  the same reduction, r in [0, ln2), even and odd polynomials, no division
+//   tanh  E / (E + 2), E = e^2a - 1 from exp's polynomial
+//   log   reduction to [sqrt(1/2), sqrt(2)), s = f/(2+f), the odd series in s
+//         and its reconstruction from f as in fdlibm e_log.c; 1/(2+f) from a
+//         cubic and three Newton orders instead of a division
 //   sin/cos  reduction by pi/2 (two-part constant, valid |x| < 2^19), kernel
 //         polynomials of fdlibm k_sin.c / k_cos.c on |r| <= pi/4
 //   expm1 fdlibm s_expm1.c rational form on |x| <= 1, exp(x)-1 outside
-//   sinh  Taylor series on |x| < 1, (e^x - e^-x)/2 otherwise
-//   tanh  expm1(2|x|) / (expm1(2|x|) + 2), +-1 beyond |x| = 22
-//   pow   exp(y * log|x|) with the integer-exponent sign rule; y = 2 and y = 3
-//         as products in double
+//   pow   exp(y * log|x|) with the integer-exponent sign rule; y = 2, 3, 4 and
+//         8 as products in double
+// A double division costs a wavefront of the GPU as much as some fifteen
+// fused multiply-adds: exp with one took 2.5 times as long, tanh with three
+// more than twice.
 #pragma once
 #include <stdint.h>
 
@@ -42,78 +47,82 @@ XM_FN bool isnan_(double x) { return x != x; }
 XM_FN double inf_() { return dbl(0x7ff0000000000000ull); }
 XM_FN double nan_() { return dbl(0x7ff8000000000000ull); }
 
-// x * 2^n for the exponent range of exp (|n| <= 1100), two exact steps.
-XM_FN double scale2(double x, int n) {
-    if (n > 1023) {
-        x = x * dbl(0x7fe0000000000000ull);  // 2^1023
-        n -= 1023;
-        if (n > 1023) n = 1023;
-    } else if (n < -1022) {
-        x = x * dbl(0x0010000000000000ull);  // 2^-1022
-        n += 1022;
-        if (n < -1022) n = -1022;
-    }
-    return x * dbl((uint64_t)(n + 1023) << 52);
+XM_FN double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// x = k ln2 + hi - lo, hi exact; k = x / ln2 + shift rounded to an integer,
+// from the low bits of a sum that rounds there (|x| < 2^20)
+XM_FN double reduce_ln2(double x, double shift, int& k, double& lo) {
+    const double ln2hi = 6.93147180369123816490e-01, ln2lo = 1.90821492927058770002e-10;
+    const double invln2 = 1.44269504088896338700e+00, magic = 6755399441055744.0;  // 1.5 * 2^52
+    const double t = shift == 0.0 ? fma_(x, invln2, magic) : fma_(x, invln2, shift) + magic, kd = t - magic;
+    k = (int)(uint32_t)bits(t);
+    lo = kd * ln2lo;
+    return fma_(-kd, ln2hi, x);
+}
+// (e^r - 1 - r) / r^2 for |r| <= ln2/2
+XM_FN double exp_q(double r) {
+    double q = 2.0913209691564269e-09;
+    q = fma_(q, r, 2.5105170644143384e-08);
+    q = fma_(q, r, 2.755727803945201e-07);
+    q = fma_(q, r, 2.7557255517955746e-06);
+    q = fma_(q, r, 2.480158732088198e-05);
+    q = fma_(q, r, 0.00019841269874720617);
+    q = fma_(q, r, 0.0013888888888885856);
+    q = fma_(q, r, 0.0083333333333261671);
+    q = fma_(q, r, 0.041666666666666664);
+    q = fma_(q, r, 0.16666666666666671);
+    return fma_(q, r, 0.5);
 }
 
-XM_FN int round_int(double v) { return (int)(v >= 0.0 ? v + 0.5 : v - 0.5); }
-
 XM_FN double exp(double x) {
-    if (isnan_(x)) return x;
-    if (x > 709.782712893383973096) return inf_();
-    if (x < -745.133219101941108420) return 0.0;
-    const double ln2hi = 6.93147180369123816490e-01, ln2lo = 1.90821492927058770002e-10;
-    const double invln2 = 1.44269504088896338700e+00;
-    int k = round_int(x * invln2);
-    double hi = x - k * ln2hi;  // exact: ln2hi has 32 significant bits
-    double lo = k * ln2lo;
-    double r = hi - lo;
-    const double P1 = 1.66666666666666019037e-01, P2 = -2.77777777770155933842e-03,
-                 P3 = 6.61375632143793436117e-05, P4 = -1.65339022054652515390e-06,
-                 P5 = 4.13813679705723846039e-08;
-    double t = r * r;
-    double c = r - t * (P1 + t * (P2 + t * (P3 + t * (P4 + t * P5))));
-    double y = 1.0 - ((lo - (r * c) / (2.0 - c)) - hi);
-    return scale2(y, k);
+    // at the ends the scaling gives inf and 0; NaN passes through
+    const double xc = x > 710.0 ? 710.0 : (x < -746.0 ? -746.0 : x);
+    int k;
+    double lo;
+    const double hi = reduce_ln2(xc, 0.0, k, lo), r = hi - lo;
+    // with the part of hi - lo that r lost
+    return __builtin_ldexp(1.0 + (r + fma_(r * r, exp_q(r), (hi - r) - lo)), k);
 }
 
 XM_FN double log(double x) {
-    if (isnan_(x)) return x;
-    if (x < 0.0) return nan_();
-    if (x == 0.0) return -inf_();
-    if (x == inf_()) return x;
     uint64_t b = bits(x);
     int k = 0;
-    if ((b >> 52) == 0) {  // subnormal
-        x = x * dbl(0x4350000000000000ull);  // 2^54
-        b = bits(x);
+    if (b - 0x0010000000000000ull >= 0x7fe0000000000000ull) {  // not a positive normal number
+        if (isnan_(x) || x == inf_()) return x;
+        if (x == 0.0) return -inf_();
+        if (x < 0.0) return nan_();
+        b = bits(x * dbl(0x4350000000000000ull));  // subnormal: 2^54
         k = -54;
     }
-    k += (int)(b >> 52) - 1023;
-    double m = dbl((b & 0x000fffffffffffffull) | 0x3ff0000000000000ull);  // [1,2)
-    if (m > 1.41421356237309504880) {
-        m = m * 0.5;
-        k += 1;
-    }
-    double f = m - 1.0;
+    // x = 2^k m, m in [sqrt(1/2), sqrt(2))
+    uint32_t hi = (uint32_t)(b >> 32);
+    const int e = (int)(hi - 0x3fe6a09eu) >> 20;
+    k += e;
+    hi -= (uint32_t)e << 20;
+    const double f = dbl((uint64_t)hi << 32 | (uint32_t)b) - 1.0, d = 2.0 + f;
+    double y = -0.057134684102826412;
+    y = fma_(y, f, 0.12813395353460683);
+    y = fma_(y, f, -0.25038631146362411);
+    y = fma_(y, f, 0.49995694014279746);
+    double g = fma_(-d, y, 1.0);
+    y = fma_(y, fma_(g, g, g), y);
+    g = fma_(-d, y, 1.0);
+    y = fma_(y, g, y);
+    const double s = f * y, w = s * s;
+    double R = 0.14616719870254904;
+    R = fma_(R, w, 0.15331699733323692);
+    R = fma_(R, w, 0.18182889783543663);
+    R = fma_(R, w, 0.22222211125751612);
+    R = fma_(R, w, 0.28571428626030954);
+    R = fma_(R, w, 0.39999999999899383);
+    R = fma_(R, w, 0.66666666666666696);
+    R = R * w;
     const double ln2hi = 6.93147180369123816490e-01, ln2lo = 1.90821492927058770002e-10;
-    const double Lg1 = 6.666666666666735130e-01, Lg2 = 3.999999999940941908e-01,
-                 Lg3 = 2.857142874366239149e-01, Lg4 = 2.222219843214978396e-01,
-                 Lg5 = 1.818357216161805012e-01, Lg6 = 1.531383769920937332e-01,
-                 Lg7 = 1.479819860511658591e-01;
-    double s = f / (2.0 + f);
-    double z = s * s;
-    double w = z * z;
-    double t1 = w * (Lg2 + w * (Lg4 + w * Lg6));
-    double t2 = z * (Lg1 + w * (Lg3 + w * (Lg5 + w * Lg7)));
-    double R = t2 + t1;
-    double hfsq = 0.5 * f * f;
-    double dk = (double)k;
-    if (k == 0) return f - (hfsq - s * (hfsq + R));
-    return dk * ln2hi - ((hfsq - (s * (hfsq + R) + dk * ln2lo)) - f);
+    const double hfsq = 0.5 * f * f, dk = (double)k;
+    return fma_(dk, ln2hi, -((hfsq - fma_(s, hfsq + R, dk * ln2lo)) - f));
 }
 
-XM_FN double log10(double x) { return log(x) / 2.30258509299404568402; }
+XM_FN double log10(double x) { return log(x) * 0.43429448190325182765; }
 
 XM_FN double expm1(double x) {
     if (isnan_(x)) return x;
@@ -156,89 +165,102 @@ XM_FN double expm1(double x) {
     return 1.0 + 2.0 * (x - e);
 }
 
+// a = k ln2 + r, 0 <= r < ln2: e^+-a = 2^+-k (cosh r +- sinh r), and every
+// term of sinh a is positive
 XM_FN double sinh(double x) {
-    if (isnan_(x)) return x;
-    double a = x < 0.0 ? -x : x;
-    if (a < 1.0) {
-        // x * sum_{k=0..11} z^k/(2k+1)!, z = x^2, coefficients rounded to double
-        const double c[12] = {1.00000000000000000e+00, 1.66666666666666657e-01, 8.33333333333333322e-03, 1.98412698412698413e-04, 2.75573192239858925e-06, 2.50521083854417202e-08, 1.60590438368216133e-10, 7.64716373181981641e-13, 2.81145725434552060e-15, 8.22063524662432950e-18, 1.95729410633912626e-20, 3.86817017063068413e-23};
-        double z = x * x;
-        double s = c[11];
-        for (int k = 10; k >= 0; k--) s = c[k] + s * z;
-        return x * s;
+    const double a = x < 0.0 ? -x : x;
+    double y;
+    if (a > 700.0) {
+        const double h = exp(0.5 * a);
+        y = 0.5 * h * h;
+    } else {
+        int k;
+        double lo;
+        const double hi = reduce_ln2(a, -0.5, k, lo), r = hi - lo, z = r * r;
+        double p = 1.1554240745674529e-11;
+        p = fma_(p, z, 2.0876182888828003e-09);
+        p = fma_(p, z, 2.755732119004969e-07);
+        p = fma_(p, z, 2.4801587298108202e-05);
+        p = fma_(p, z, 0.0013888888888891858);
+        p = fma_(p, z, 0.041666666666666657);
+        p = fma_(p, z, 0.5);
+        double q = 7.69436449999226e-13;
+        q = fma_(q, z, 1.6058738300383107e-10);
+        q = fma_(q, z, 2.5052109335427469e-08);
+        q = fma_(q, z, 2.7557319222561107e-06);
+        q = fma_(q, z, 0.00019841269841270736);
+        q = fma_(q, z, 0.0083333333333333332);
+        q = fma_(q, z, 0.16666666666666666);
+        const double e = (hi - r) - lo, s = r + fma_(q * z, r, e), c = 1.0 + fma_(p, z, e * r);
+        const double u = dbl((uint64_t)(k + 1022) << 52), v = dbl((uint64_t)(1022 - k) << 52);  // 2^(k-1), 2^(-k-1)
+        y = fma_(c, u - v, s * (u + v));
     }
-    if (a > 709.0) {
-        double h = exp(0.5 * a);
-        double r = 0.5 * h * h;
-        return x < 0.0 ? -r : r;
-    }
-    double e = exp(a);
-    double r = 0.5 * (e - 1.0 / e);
-    return x < 0.0 ? -r : r;
+    return x < 0.0 ? -y : y;
 }
 
+// E / (E + 2), E = e^2a - 1 = 2^k (e^r - 1) + (2^k - 1)
 XM_FN double tanh(double x) {
-    if (isnan_(x)) return x;
     double a = x < 0.0 ? -x : x;
-    double r;
-    if (a >= 22.0) {
-        r = 1.0;
-    } else {
-        double t = expm1(2.0 * a);
-        r = t / (t + 2.0);
-    }
-    return x < 0.0 ? -r : r;
+    a = a > 22.0 ? 22.0 : a;  // 1 from there on
+    int k;
+    double lo;
+    const double hi = reduce_ln2(2.0 * a, 0.0, k, lo), r = hi - lo;
+    const double p = r + fma_(r * r, exp_q(r), (hi - r) - lo), u = dbl((uint64_t)(k + 1023) << 52);
+    const double E = fma_(u, p, u - 1.0);
+    const double y = E / (E + 2.0);
+    return x < 0.0 ? -y : y;
 }
 
 XM_FN double ksin(double r) {
     const double S1 = -1.66666666666666324348e-01, S2 = 8.33333333332248946124e-03,
                  S3 = -1.98412698298579493134e-04, S4 = 2.75573137070700676789e-06,
                  S5 = -2.50507602534068634195e-08, S6 = 1.58969099521155010221e-10;
-    double z = r * r;
-    double v = z * r;
-    double q = S2 + z * (S3 + z * (S4 + z * (S5 + z * S6)));
-    return r + v * (S1 + z * q);
+    const double z = r * r, v = z * r;
+    double q = fma_(S6, z, S5);
+    q = fma_(q, z, S4);
+    q = fma_(q, z, S3);
+    q = fma_(q, z, S2);
+    return fma_(v, fma_(q, z, S1), r);
 }
 XM_FN double kcos(double r) {
     const double C1 = 4.16666666666666019037e-02, C2 = -1.38888888888741095749e-03,
                  C3 = 2.48015872894767294178e-05, C4 = -2.75573143513906633035e-07,
                  C5 = 2.08757232129817482790e-09, C6 = -1.13596475577881948265e-11;
-    double z = r * r;
-    double q = z * (C1 + z * (C2 + z * (C3 + z * (C4 + z * (C5 + z * C6)))));
-    double hz = 0.5 * z;
-    double w = 1.0 - hz;
-    return w + (((1.0 - w) - hz) + z * q);
+    const double z = r * r;
+    double q = fma_(C6, z, C5);
+    q = fma_(q, z, C4);
+    q = fma_(q, z, C3);
+    q = fma_(q, z, C2);
+    q = fma_(q, z, C1) * z;
+    const double hz = 0.5 * z, w = 1.0 - hz;
+    return w + fma_(z, q, (1.0 - w) - hz);
 }
 // reduce by pi/2: r in [-pi/4, pi/4], quadrant q
 XM_FN double rpio2(double x, int& q) {
-    const double invpio2 = 6.36619772367581382433e-01;
+    const double invpio2 = 6.36619772367581382433e-01, magic = 6755399441055744.0;
     const double pio2_1 = 1.57079632673412561417e+00, pio2_1t = 6.07710050650619224932e-11;
-    int k = round_int(x * invpio2);
-    double r = (x - k * pio2_1) - k * pio2_1t;
-    q = k & 3;
-    return r;
+    const double t = fma_(x, invpio2, magic), k = t - magic;
+    q = (int)(uint32_t)bits(t) & 3;
+    return fma_(-k, pio2_1t, fma_(-k, pio2_1, x));
 }
 XM_FN double sin(double x) {
-    if (isnan_(x)) return x;
     int q;
-    double r = rpio2(x, q);
-    switch (q) {
-        case 0: return ksin(r);
-        case 1: return kcos(r);
-        case 2: return -ksin(r);
-        default: return -kcos(r);
-    }
+    const double r = rpio2(x, q), v = q & 1 ? kcos(r) : ksin(r);
+    return q & 2 ? -v : v;
 }
 XM_FN double cos(double x) {
-    if (isnan_(x)) return x;
     int q;
-    double r = rpio2(x, q);
-    switch (q) {
-        case 0: return kcos(r);
-        case 1: return -ksin(r);
-        case 2: return -kcos(r);
-        default: return ksin(r);
-    }
+    const double r = rpio2(x, q), v = q & 1 ? ksin(r) : kcos(r);
+    return (q + 1) & 2 ? -v : v;
+}
+// both, from one reduction (the same values)
+XM_FN void sincos(double x, double& s, double& c) {
+    int q;
+    const double r = rpio2(x, q), ks = ksin(r), kc = kcos(r);
+    s = q & 1 ? kc : ks;
+    c = q & 1 ? ks : kc;
+    s = q & 2 ? -s : s;
+    c = (q + 1) & 2 ? -c : c;
 }
 
 XM_FN bool is_int(double y) {
@@ -257,10 +279,15 @@ XM_FN bool is_odd_int(double y) {
 
 XM_FN double pow(double x, double y) {
     if (y == 0.0) return 1.0;
-    if (x == 1.0) return 1.0;
-    if (isnan_(x) || isnan_(y)) return nan_();
     if (y == 2.0) return x * x;
     if (y == 3.0) return x * x * x;
+    if (y == 4.0 || y == 8.0) {
+        const double x2 = x * x, x4 = x2 * x2;
+        return y == 4.0 ? x4 : x4 * x4;
+    }
+    if (x > 0.0 && x < inf_() && y - y == 0.0) return exp(y * log(x));
+    if (x == 1.0) return 1.0;
+    if (isnan_(x) || isnan_(y)) return nan_();
     if (x == 0.0) {
         if (y > 0.0) return is_odd_int(y) ? x : 0.0;
         return is_odd_int(y) && bits(x) >> 63 ? -inf_() : inf_();
@@ -309,5 +336,11 @@ XM_FN float sinhf(float x) { return (float)sinh((double)x); }
 XM_FN float tanhf(float x) { return (float)tanh((double)x); }
 XM_FN float sinf(float x) { return (float)sin((double)x); }
 XM_FN float cosf(float x) { return (float)cos((double)x); }
+XM_FN void sincosf(float x, float& s, float& c) {
+    double ds, dc;
+    sincos((double)x, ds, dc);
+    s = (float)ds;
+    c = (float)dc;
+}
 
 }  // namespace xm
