@@ -368,8 +368,8 @@ int xbg_bnd_synth(int N, int nk, const int* idx, const double* gre, const double
  * Batched ensemble of independent domains (storm-scenario ensembles).  No
  * counterpart in the reference, which steps one domain per process
  * (mainloopGPU, Wave_gpu.cu:610-728, fixed 16x16 blocks at 615-619): here
- * every phase of the step is one launch over all domains (tile maps of
- * (domain, tile) entries walked by persistent workgroups), each domain's
+ * every phase of the step is one launch over all domains (one
+ * workgroup per entry of a tile map (domain, tile)), each domain's
  * time step (CFL minima, the rule of xbg_next_dt, the boundary record of
  * the new time) is chosen on the device, and a whole step is one hipGraph
  * replay.  Results equal xbg_advance_resident loops on each domain bit
@@ -403,9 +403,8 @@ int xbg_ens_sync(xbg_ens* e);
  * may be NULL); waits for the ensemble and points every context at the
  * buffers its last step wrote, so xbg_get_field reads the current state. */
 int xbg_ens_status(xbg_ens* e, double* t, double* dt, int* steps, int* status);
-/* Autotuner: times every offered launch shape (persistent grid per kernel
- * class, patch shape of the dispersion and concentration kernels) over
- * rounds x 12 whole steps, keeps the fastest of each and rebuilds the step
+/* Autotuner: times every offered launch shape (patch shape of the
+ * dispersion and concentration kernels) over rounds x 12 whole steps, keeps the fastest of each and rebuilds the step
  * graph.  The timed steps advance the ensemble (a launch shape never
  * changes a result).  report (may be NULL) receives the measured table. */
 int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n);

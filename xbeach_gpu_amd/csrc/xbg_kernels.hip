@@ -3633,9 +3633,8 @@ const char* xbg_noalloc_last_error(void) { return g_noalloc_error.c_str(); }
 //
 // The domains of a storm-scenario ensemble (uneven grids, own forcing, own
 // CFL time step) advance together: every phase of the step is ONE launch
-// over all domains, whose workgroups walk a tile map (domain, tile) with a
-// grid stride (persistent workgroups when the tuned grid is smaller than
-// the map).  Each workgroup reads its domain's constants, step scalars and
+// over all domains, one workgroup for each entry (domain, tile) of a tile
+// map.  Each workgroup reads its domain's constants, step scalars and
 // buffer pointers from a descriptor table in device memory.  The time step
 // of every domain (its CFL minima, the rule of mainloopGPU, the boundary
 // record of the new time) is chosen on the device by k_ens_dt, so whole
@@ -3678,11 +3677,11 @@ struct TileEnt {
 typedef const DomDesc* __restrict__ DTab;
 typedef const TileEnt* __restrict__ TMap;
 
-// grid-stride walk over the tile map; the barrier keeps a workgroup's next
-// tile from overwriting LDS its previous tile still reads
-#define ENS_FOR_TILES(map, ntiles)                                         \
-    for (int t_ = blockIdx.x; t_ < (ntiles); t_ += gridDim.x)
-#define ENS_TILE_END __syncthreads()
+// One workgroup per tile of the map.  A loop over the map (persistent
+// workgroups) was never faster, and the compiler moved the bodies' double
+// constants out of it into 50 to 80 registers: half the wavefronts per SIMD
+// (an ensemble of 48 domains 3.59 -> 3.40 ms per step without the loop).
+#define ENS_FOR_TILES(map, ntiles) if (const int t_ = blockIdx.x; t_ < (ntiles))
 
 template <int QW, int QH>
 __global__ __launch_bounds__(256) void kb_dispersion(DTab tab, TMap map, int ntiles) {
@@ -3690,15 +3689,12 @@ __global__ __launch_bounds__(256) void kb_dispersion(DTab tab, TMap map, int nti
         const TileEnt e = map[t_];
         const DomDesc& D = tab[e.dom];
         if (D.status == ENS_ACTIVE) dispersion_body<QW, QH>(D.p, D.s, D.f[D.par][PH_START], 1, BI{e.bx, e.by});
-        ENS_TILE_END;
     }
 }
 
 // Entries with bx < 0 pad a domain's run of tiles to a multiple of 8 (so
 // that map position modulo 8, the XCD of the workgroup, is the XCD the
-// single-domain launch gives the tile) and are skipped.  One tile per
-// workgroup: the wave kernel sits at the 128-VGPR limit of its two
-// workgroups per CU, and a tile loop around it spills.
+// single-domain launch gives the tile) and are skipped.
 template <int A, bool EX, bool CUR, bool FLEX>
 __global__ __launch_bounds__(WTHREADS, wave_occ(A)) void kb_wave(DTab tab, TMap map, int ntiles) {
     const TileEnt e = map[blockIdx.x];
@@ -3748,7 +3744,6 @@ __global__ __launch_bounds__(BX * CY) void kb_flow_uvcorr(DTab tab, TMap map, in
         const TileEnt e = map[t_];
         const DomDesc& D = tab[e.dom];
         if (D.status == ENS_ACTIVE) flow_uvcorr_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-        ENS_TILE_END;
     }
 }
 
@@ -3757,7 +3752,6 @@ __global__ __launch_bounds__(BX * CY) void kb_flow_zsall(DTab tab, TMap map, int
         const TileEnt e = map[t_];
         const DomDesc& D = tab[e.dom];
         if (D.status == ENS_ACTIVE) flow_zsall_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-        ENS_TILE_END;
     }
 }
 
@@ -3774,7 +3768,6 @@ __global__ __launch_bounds__(256) void kb_sed_flux(DTab tab, TMap map, int ntile
         const TileEnt e = map[t_];
         const DomDesc& D = tab[e.dom];
         if (D.status == ENS_ACTIVE && D.sed) sed_flux_body(D.p, D.s, D.f[D.par][PH_ZS], 1, BI{e.bx, e.by});
-        ENS_TILE_END;
     }
 }
 
@@ -3794,7 +3787,6 @@ __global__ __launch_bounds__(256) void kb_sed_morph(DTab tab, TMap map, int ntil
         const DomDesc& D = tab[e.dom];
         if (D.status == ENS_ACTIVE && D.sed && D.morph)
             sed_morph_body(D.p, D.s, D.f[D.par][PH_END], BI{e.bx, e.by});
-        ENS_TILE_END;
     }
 }
 
@@ -3839,7 +3831,6 @@ __global__ __launch_bounds__(256) void kb_cfl(DTab tab, TMap map, int ntiles, fl
                 part[t_] = (rb[0] | rb[1] | rb[2] | rb[3]) ? __builtin_nanf("") : v;
             }
         }
-        ENS_TILE_END;
     }
 }
 
@@ -4023,14 +4014,11 @@ enum EnsK { EK_CFL, EK_DISP, EK_WAVE, EK_ROWS, EK_NUH, EK_U, EK_V, EK_UVCORR, EK
 const char* const kEnsName[EK_N] = {"kb_cfl", "kb_dispersion", "kb_wave", "kb_wave_rows", "kb_flow_nuh",
                                     "kb_flow_u", "kb_flow_v", "kb_flow_uvcorr", "kb_flow_zsall", "kb_flow_uvvu",
                                     "kb_sed_flux", "kb_sed_conc", "kb_sed_morph"};
-// persistent grid sizes offered to the tuner, in workgroups per CU (0: one
-// workgroup per tile)
-const int kGridPerCU[] = {0, 2, 4, 8};
-constexpr int N_GRID = 4;
 // patch shapes (one wavefront) offered for the dispersion and concentration
 // kernels
 const int kShapeW[] = {4, 8, 16};
 constexpr int N_SHAPE = 3;
+constexpr int TUNE_REPEAT = 4;  // steps timed per shape and round
 
 struct TileMap {
     TileEnt* d = nullptr;  // device
@@ -4056,9 +4044,7 @@ struct xbg_ens {
     std::vector<WaveGroup> waves;
     std::vector<WaveGroup> rows;
     float* part = nullptr;
-    int ncu = 256;
     // launch choices (tuned)
-    int grid_sel[EK_N] = {};   // index into kGridPerCU
     int disp_shape = 0, conc_shape = 2;  // 4x16 dispersion, 16x4 concentration (the single-domain shapes)
     // graph of one step for the current choices
     hipGraph_t graph = nullptr;
@@ -4119,13 +4105,6 @@ std::vector<TileEnt> grid_map(const std::vector<int>& doms, const std::vector<in
     return v;
 }
 
-int grid_of(const xbg_ens* e, int k, int ntiles) {
-    int per = kGridPerCU[e->grid_sel[k]];
-    if (per == 0) return ntiles;
-    int g = per * e->ncu;
-    return g < ntiles ? g : ntiles;
-}
-
 void ens_ev(xbg_ens* e, int slot) {
     if (e->prof) hipEventRecord(e->ev[slot], e->stream);
 }
@@ -4136,25 +4115,22 @@ int ens_launch_step(xbg_ens* e) {
     const dim3 b2(BX, BY), bc(BX, CY);
     if (e->m_cfl.n) {
         ens_ev(e, 2 * EK_CFL);
-        kb_cfl<<<dim3(grid_of(e, EK_CFL, e->m_cfl.n)), dim3(256), 0, e->stream>>>(e->dtab, e->m_cfl.d, e->m_cfl.n,
-                                                                                 e->part);
+        kb_cfl<<<dim3(e->m_cfl.n), dim3(256), 0, e->stream>>>(e->dtab, e->m_cfl.d, e->m_cfl.n, e->part);
         ens_ev(e, 2 * EK_CFL + 1);
     }
     k_ens_dt<<<dim3(e->nd), dim3(256), 0, e->stream>>>(e->dtab, e->part);
     {
         const TileMap& m = e->m_disp[e->disp_shape];
-        int g = grid_of(e, EK_DISP, m.n);
         ens_ev(e, 2 * EK_DISP);
         switch (e->disp_shape) {
-            case 0: kb_dispersion<4, 16><<<dim3(g), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            case 1: kb_dispersion<8, 8><<<dim3(g), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            default: kb_dispersion<16, 4><<<dim3(g), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            case 0: kb_dispersion<4, 16><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            case 1: kb_dispersion<8, 8><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            default: kb_dispersion<16, 4><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
         }
         ens_ev(e, 2 * EK_DISP + 1);
     }
     ens_ev(e, 2 * EK_WAVE);
     for (const WaveGroup& w : e->waves) {
-        // one workgroup per tile (kb_wave has no tile loop)
 #define RUN(A_, EX_, C_, F_) \
     kb_wave<A_, EX_, C_, F_><<<dim3(w.map.n), dim3(BX, WTY), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
         WAVE_SWITCH(w.k, RUN);
@@ -4163,9 +4139,8 @@ int ens_launch_step(xbg_ens* e) {
     ens_ev(e, 2 * EK_WAVE + 1);
     ens_ev(e, 2 * EK_ROWS);
     for (const WaveGroup& w : e->rows) {
-        const int g = grid_of(e, EK_ROWS, w.map.n);
 #define RUN(A_, EX_, C_, F_) \
-    kb_wave_rows<A_, EX_, C_><<<dim3(g), dim3(256), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
+    kb_wave_rows<A_, EX_, C_><<<dim3(w.map.n), dim3(256), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
         WAVE_SWITCH(w.k, RUN);
 #undef RUN
     }
@@ -4175,7 +4150,7 @@ int ens_launch_step(xbg_ens* e) {
 #define EL(k, kern, blk, m)                                                                                 \
     do {                                                                                                    \
         ens_ev(e, 2 * (k));                                                                                 \
-        kern<<<dim3(grid_of(e, (k), (m).n)), blk, 0, e->stream>>>(e->dtab, (m).d, (m).n);                   \
+        kern<<<dim3((m).n), blk, 0, e->stream>>>(e->dtab, (m).d, (m).n);                                    \
         ens_ev(e, 2 * (k) + 1);                                                                             \
     } while (0)
     EL(EK_NUH, kb_flow_nuh, b2, m2);
@@ -4187,12 +4162,11 @@ int ens_launch_step(xbg_ens* e) {
     EL(EK_SFLUX, kb_sed_flux, b2, m2);
     {
         const TileMap& m = e->m_conc[e->conc_shape];
-        int g = grid_of(e, EK_SCONC, m.n);
         ens_ev(e, 2 * EK_SCONC);
         switch (e->conc_shape) {
-            case 0: kb_sed_conc<4, 16><<<dim3(g), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            case 1: kb_sed_conc<8, 8><<<dim3(g), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            default: kb_sed_conc<16, 4><<<dim3(g), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            case 0: kb_sed_conc<4, 16><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            case 1: kb_sed_conc<8, 8><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            default: kb_sed_conc<16, 4><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
         }
         ens_ev(e, 2 * EK_SCONC + 1);
     }
@@ -4239,13 +4213,6 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
         xbg_ens_destroy(e);
         return rc;
     };
-    int dev = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
-        prop.multiProcessorCount > 0)
-        e->ncu = prop.multiProcessorCount;
-    // the single-domain launch shapes by default: one workgroup per tile
-    for (int k = 0; k < EK_N; k++) e->grid_sel[k] = 0;
     std::vector<int> doms_all, gx2, gy2, gxc, gyc, gxcfl, gycfl;
     std::vector<TileEnt> cfl;
     std::map<WaveK, std::vector<TileEnt>> wave_tiles, row_tiles;
@@ -4404,12 +4371,10 @@ int xbg_ens_status(xbg_ens* e, double* t, double* dt, int* steps, int* status) {
 
 int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n) {
     if (!e || rounds < 1) return XBG_E_ARG;
-    // every candidate of every kernel class is timed over whole steps (the
-    // steps are real: a launch shape changes which thread computes which
-    // cell, never a result)
-    const int ncand_grid = N_GRID;
-    std::vector<std::vector<double>> tg(EK_N, std::vector<double>(ncand_grid, 0.0));
-    std::vector<std::vector<int>> cg(EK_N, std::vector<int>(ncand_grid, 0));
+    // every patch shape is timed over whole steps (the steps are real: a
+    // launch shape changes which thread computes which cell, never a result)
+    std::vector<double> tk(EK_N, 0.0);
+    std::vector<int> ck(EK_N, 0);
     std::vector<double> td(N_SHAPE, 0.0), tc(N_SHAPE, 0.0);
     std::vector<int> cd(N_SHAPE, 0), cc(N_SHAPE, 0);
     e->prof = true;
@@ -4417,18 +4382,17 @@ int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n) {
     // warm-up step (first-launch costs) with the current choices
     if ((rc = ens_launch_step(e))) { e->prof = false; return rc; }
     EHIP(e, hipStreamSynchronize(e->stream));
-    const int total = rounds * ncand_grid * N_SHAPE;
+    const int total = rounds * TUNE_REPEAT * N_SHAPE;
     for (int r = 0; r < total; r++) {
-        for (int k = 0; k < EK_N; k++) e->grid_sel[k] = r % ncand_grid;
-        e->disp_shape = (r / ncand_grid) % N_SHAPE;
-        e->conc_shape = (r / ncand_grid) % N_SHAPE;
+        e->disp_shape = r % N_SHAPE;
+        e->conc_shape = r % N_SHAPE;
         if ((rc = ens_launch_step(e))) { e->prof = false; return rc; }
         EHIP(e, hipStreamSynchronize(e->stream));
         for (int k = 0; k < EK_N; k++) {
             float ms = 0.0f;
             if (hipEventElapsedTime(&ms, e->ev[2 * k], e->ev[2 * k + 1]) != hipSuccess) continue;
-            tg[k][r % ncand_grid] += ms;
-            cg[k][r % ncand_grid] += 1;
+            tk[k] += ms;
+            ck[k] += 1;
             if (k == EK_DISP) { td[e->disp_shape] += ms; cd[e->disp_shape]++; }
             if (k == EK_SCONC) { tc[e->conc_shape] += ms; cc[e->conc_shape]++; }
         }
@@ -4437,16 +4401,8 @@ int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n) {
     std::string out;
     char line[256];
     for (int k = 0; k < EK_N; k++) {
-        int best = 0;
-        double bt = 1e300;
-        for (int j = 0; j < ncand_grid; j++) {
-            double a = cg[k][j] ? tg[k][j] / cg[k][j] : 1e300;
-            snprintf(line, sizeof(line), "%s grid=%s%d us=%.2f\n", kEnsName[k], kGridPerCU[j] ? "" : "tiles:",
-                     kGridPerCU[j] ? kGridPerCU[j] * e->ncu : 0, 1000.0 * a);
-            out += line;
-            if (a < bt) { bt = a; best = j; }
-        }
-        e->grid_sel[k] = best;
+        snprintf(line, sizeof(line), "%s us=%.2f\n", kEnsName[k], ck[k] ? 1000.0 * tk[k] / ck[k] : 0.0);
+        out += line;
     }
     int bd = 0, bc = 0;
     for (int s = 0; s < N_SHAPE; s++) {
@@ -4459,12 +4415,7 @@ int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n) {
     }
     e->disp_shape = bd;
     e->conc_shape = bc;
-    out += "chosen:";
-    for (int k = 0; k < EK_N; k++) {
-        snprintf(line, sizeof(line), " %s=%d", kEnsName[k], kGridPerCU[e->grid_sel[k]] * e->ncu);
-        out += line;
-    }
-    snprintf(line, sizeof(line), " dispersion_patch=%dx%d conc_patch=%dx%d\n", kShapeW[bd], 64 / kShapeW[bd],
+    snprintf(line, sizeof(line), "chosen: dispersion_patch=%dx%d conc_patch=%dx%d\n", kShapeW[bd], 64 / kShapeW[bd],
              kShapeW[bc], 64 / kShapeW[bc]);
     out += line;
     if (report && n) {
