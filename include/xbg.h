@@ -411,7 +411,7 @@ int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n);
 /* Average duration (us) of each kernel class over nsteps steps run with
  * events (these steps advance the ensemble); us has XBG_ENS_NKERNELS entries
  * named by xbg_ens_kernel_name. */
-#define XBG_ENS_NKERNELS 13
+#define XBG_ENS_NKERNELS 12
 int xbg_ens_kernel_times(xbg_ens* e, int nsteps, double* us);
 const char* xbg_ens_kernel_name(int k);
 /* Wave-group window means for surrogate training data: _enable allocates

@@ -41,7 +41,6 @@ struct KP {
     float sed_drho, sed_dester, sed_Ass, sed_ucrfac, rvr_alph, rvr_bet;
     int usesmago, breakmodel, roller, zb_accum, swave;
     int wtiles_x, wtiles_y;  // wave-kernel tile grid
-    int fold_rows;           // rows 0 / ny-1 finished inside the wave kernel
     double rdtheta;          // 1/dtheta rounded once in double (div_uniform)
     int dth_recip;           // 0 < dtheta < 2: divide through rdtheta
     float rdx;               // 1/dx, exact when dx_p2 is set

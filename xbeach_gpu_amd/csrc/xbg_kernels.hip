@@ -8,11 +8,10 @@
 //
 //   k_dispersion    dispersion -> k, c, cg; its first workgroup runs ubnd1D
 //                   (k_bnd_offshore alone when waves are off)
-//   k_wave<NT>      offshorebndWav .. breakerdelay fused per cell: the
+//   k_wave          offshorebndWav .. breakerdelay fused per cell: the
 //                   direction planes of ee and rr stream through LDS tiles,
 //                   the bins of a cell stay in registers; one read and one
-//                   write of each directional field per step (k_wave_rows
-//                   finishes rows 0 / ny-1 where a tile cannot)
+//                   write of each directional field per step
 //   k_flow_nuh      smago + wetu/wetv masks, and in a whole step the wave
 //                   forces: wavforce + twodimbnd(noix) for Fx, Fy, ust
 //                   (k_wave_force alone for the wave sub-step)
@@ -56,7 +55,13 @@ constexpr int BX = 64;  // block: 64 cells along x (one wavefront per row)
 constexpr int BY = 4;   // 4 rows -> 256 threads
 
 struct Fld {
-    const float* dirs;  // direction tables, 8 x MAXT (see tab())
+    // Direction tables, dirs[k * MAXT + th], k = 0..7: theta, cos, sin,
+    // 1 + cos^2, 1 + sin^2, sin*cos, cos^2, sin^2 (FP32 products as
+    // radstressCPU forms them, wave_CPU.cpp:1118-1157).  The wave kernel reads
+    // a copy in LDS: its lookups complete in order with the plane and face
+    // reads, where a scalar load (whose results may return out of order) makes
+    // each wait on it a wait for every outstanding LDS read.
+    const float* dirs;
     const float* St;   // ny*nt wave boundary of this step
     const float* qbo;  // 4*ny
     const float* qbn;
@@ -72,7 +77,6 @@ struct Fld {
     // wave products of the step
     float *k, *c, *cg, *H, *E, *Dw, *DR, *R, *urms, *ust_raw, *ust, *thetamean;
     float *Sxx, *Sxy, *Syy, *Fx, *Fy;
-    float *bnd_e1, *bnd_r1;  // post-Euler ee/rr of rows 1 and ny-2
     // flow intermediates
     float* nuh;
     uint8_t* wet;  // bit0 wetu, bit1 wetv (udepthmomcont / vdepthmomcont)
@@ -136,29 +140,6 @@ struct BI {
 };
 XDEV int gx(BI bi) { return bi.x * BX + threadIdx.x; }
 XDEV int gy(BI bi) { return bi.y * BY + threadIdx.y; }
-
-// Direction-table entry read
-// through an opaque scalar index: a scalar load at each use instead of
-// nTheta x 8 values held in scalar registers across the unrolled bin loop.
-// dirs[k * MAXT + th], k = 0..7: theta, cos, sin, 1 + cos^2, 1 + sin^2,
-// sin*cos, cos^2, sin^2 (FP32 products as radstressCPU forms them,
-// wave_CPU.cpp:1118-1157).
-typedef const __attribute__((address_space(4))) float* cfloat_ptr;  // constant (read-only) memory
-XDEV float tab(const float* t, int th) {
-    int k = th;
-    asm volatile("" : "+s"(k));
-    return ((cfloat_ptr)t)[k];
-}
-
-// L: t is the wave kernel's copy of the table in LDS (filled at its start):
-// its lookups complete in order with the plane and face reads, where a scalar
-// load (whose results may return out of order) makes each wait on it a wait
-// for every outstanding LDS read.
-template <bool L>
-XDEV float dtab(const float* t, int k, int th) {
-    if (L) return t[k * MAXT + th];
-    return tab(t + k * MAXT, th);
-}
 
 // ---------------------------------------------------------------------------
 // Flow boundary: ubnd1D (Flow_kernel.cu:167-242) / ubnd1Dnowaves (332-403).
@@ -253,10 +234,6 @@ XDEV void dispersion_body(const KP& p, const SP& s, const Fld& f, int offshore, 
 }
 __global__ __launch_bounds__(256) void k_dispersion(KP p, SP s, Fld f, int offshore) {
     dispersion_body(p, s, f, offshore, BI{(int)blockIdx.x, (int)blockIdx.y});
-}
-
-XDEV float act_rr(const KP& p, const Fld& f, int x, int y, int th) {
-    return G(f.rr_in)[(size_t)x + (size_t)y * p.nx + (size_t)th * p.N];
 }
 
 // Refraction speed of propagthetaCPU (wave_CPU.cpp:259-287), with the
@@ -404,21 +381,15 @@ XDEV float baldock_cell(const KP& p, float Trep, float Ht, float h, float k, flo
 // (wave_CPU.cpp:873-1089) at cell i: e (action after Euler) -> ee after
 // dissipation, r (roller after Euler) -> rr after dissipation.
 // A bins at most: p.nt of them, A itself when EX.
-// The ee bins are an array of the thread, or a column of LDS (stride STRIDE
-// floats): in the wave kernel they stay there, 24 registers that its sweep and
-// this routine do not have to find.
-struct RegBins {
-    float* a;
-    XDEV float get(int th) const { return a[th]; }
-    XDEV void set(int th, float v) const { a[th] = v; }
-};
+// The ee bins are a column of LDS (stride STRIDE floats): 24 registers that
+// the wave kernel's sweep and this routine do not have to find.
 template <int STRIDE>
 struct LdsBins {
     float* a;
     XDEV float get(int th) const { return a[th * STRIDE]; }
     XDEV void set(int th, float v) const { a[th * STRIDE] = v; }
 };
-template <int A, bool EX, bool CUR, bool L, class B>
+template <int A, bool EX, bool CUR, class B>
 XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const B e, float* r,
                       float& Rout, float& DRout) {
     const int nt = EX ? A : p.nt;
@@ -481,8 +452,8 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
         for (int th = 0; th < A; th++) {
             if (th >= nt) break;
             float eet = e.get(th);
-            float cx = CUR ? cc * dtab<L>(dirs, 1, th) + uui : cc * dtab<L>(dirs, 1, th);
-            float cy = CUR ? cc * dtab<L>(dirs, 2, th) + vvi : cc * dtab<L>(dirs, 2, th);
+            float cx = CUR ? cc * dirs[1 * MAXT + th] + uui : cc * dirs[1 * MAXT + th];
+            float cy = CUR ? cc * dirs[2 * MAXT + th] + vvi : cc * dirs[2 * MAXT + th];
             float dd = NEAR ? xm::div_by(eet * Dv, rE) : eet * Dv / Emx;
             float rrt;
             if (wetc) {
@@ -511,7 +482,7 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
 // meandirCPU (wave_CPU.cpp:1092-1116), radstressCPU (1118-1157) and
 // breakerdelayCPU (1334-1374, called with R) at cell i on the final ee/rr;
 // stores the directional state of the cell.
-template <int A, bool EX, bool L, class B>
+template <int A, bool EX, class B>
 XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const B efin,
                       const float* r, float Rv, float DRv) {
     const int nt = EX ? A : p.nt;
@@ -524,13 +495,13 @@ XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
         if (th >= nt) break;
         float ev = efin.get(th), rv = r[th];
         sume = sume + ev;
-        sumethet = sumethet + ev * dtab<L>(dirs, 0, th);
-        txx = txx + (dtab<L>(dirs, 3, th) * ev);   // (1 + cs*cs) * ev
-        tyy = tyy + (dtab<L>(dirs, 4, th) * ev);   // (1 + sn*sn) * ev
-        txy = txy + (dtab<L>(dirs, 5, th) * ev);   // sn*cs*ev
-        rxx = rxx + (dtab<L>(dirs, 6, th) * rv);   // (cs*cs) * rv
-        ryy = ryy + (dtab<L>(dirs, 7, th) * rv);   // (sn*sn) * rv
-        rxy = rxy + (dtab<L>(dirs, 5, th) * rv);   // sn*cs*rv
+        sumethet = sumethet + ev * dirs[0 * MAXT + th];
+        txx = txx + (dirs[3 * MAXT + th] * ev);   // (1 + cs*cs) * ev
+        tyy = tyy + (dirs[4 * MAXT + th] * ev);   // (1 + sn*sn) * ev
+        txy = txy + (dirs[5 * MAXT + th] * ev);   // sn*cs*ev
+        rxx = rxx + (dirs[6 * MAXT + th] * rv);   // (cs*cs) * rv
+        ryy = ryy + (dirs[7 * MAXT + th] * rv);   // (sn*sn) * rv
+        rxy = rxy + (dirs[5 * MAXT + th] * rv);   // sn*cs*rv
         gstore(f.ee_out + i + (size_t)th * N, ev);
         gstore(f.rr_out + i + (size_t)th * N, rv);
     }
@@ -752,8 +723,8 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
         float fxen = 0, gyen = 0, fxrn = 0, gyrn = 0;
         if (bin) {
             const float *q = L.pl(th, 0) + c0, *t = L.pl(th, 1) + c0;
-            cs = dtab<true>(L.dirs, 1, th);
-            sn = dtab<true>(L.dirs, 2, th);
+            cs = L.dirs[1 * MAXT + th];
+            sn = L.dirs[2 * MAXT + th];
             ec = q[0];
             const float el = q[-1], er = q[1], er2 = q[2], eb = q[-PW], et = q[PW], et2 = q[2 * PW];
             rc = t[0];
@@ -876,9 +847,9 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
 // offshorebndWav, sanity, action, x/y/theta advection + Euler of ee and rr,
 // energy, energint, roelvink/baldock, dissipation, meandir, radstress,
 // breakerdelay (Wavestep.cu:781-1125 order).  Rows 0 and ny-1
-// (rollerlatbnd copies from rows 1 and ny-2) are finished in the tile when
-// it also holds the source row (fold_rows), else by k_wave_rows from the
-// post-Euler bins this kernel saves.  Also the block minimum of WAVEDT.
+// (rollerlatbnd copies from rows 1 and ny-2) are finished in their tiles,
+// which hold the source rows too.  Also the block minimum of
+// WAVEDT.
 // Up to 24 bins: four waves per SIMD (<= 128 VGPRs) and at most 80 KB of LDS,
 // two workgroups per CU; more bins: one workgroup.
 constexpr int wave_occ(int A) { return A <= 24 ? 4 : 2; }
@@ -888,10 +859,15 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
     const int nt = EX ? A : p.nt;
     const int cx = threadIdx.x, cy = threadIdx.y, tid = cx + cy * BX;
     const int tile = bi.x;  // tile of the domain, after the XCD remap
-    const int x0 = (tile % p.wtiles_x) * BX, y0 = (tile / p.wtiles_x) * WTY;
     const int nx = p.nx, ny = p.ny;
+    // tile rows: the last one holds rows ny-2 and ny-1, so it starts one or
+    // more rows early where ny-1 is a multiple of WTY or ny <= WTY (row ny-2
+    // is then formed twice, alike), and no other one holds row ny-1
+    const int ty = tile / p.wtiles_x;
+    const bool bottom = ty == 0, top = ty == p.wtiles_y - 1;
+    const int x0 = (tile % p.wtiles_x) * BX, y0 = min(ty * WTY, ny - 2), yend = top ? ny : ny - 1;
     const int x = min(x0 + cx, nx - 1), y = min(y0 + cy, ny - 1);
-    const bool valid = (x0 + cx < nx) && (y0 + cy < ny);
+    const bool valid = (x0 + cx < nx) && (y0 + cy < yend);
     const uint32_t i = (uint32_t)x + (uint32_t)y * nx;
     const bool rol = FLEX ? p.roller == 1 : true;
     for (int l = tid; l < 8 * MAXT; l += WTHREADS) L.dirs[l] = G(f.dirs)[l];
@@ -913,27 +889,17 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
     // Rows 0 and ny-1 (rollerlatbnd, wave_CPU.cpp:830-871): the post-Euler
     // ee / rr of rows 1 / ny-2 times the cell's wet flag, the cell's own
     // dissipation, then ee after dissipation copied again from rows 1 /
-    // ny-2.  In the tiles that hold those rows (a workgroup-uniform
-    // condition: the barriers below are reached by every thread or none)
-    // the source row's values come through LDS; otherwise k_wave_rows
-    // finishes the rows after this kernel.
-    const bool ftile = p.fold_rows && (y0 == 0 || (ny - 1 >= y0 && ny - 1 < y0 + WTY));
-    const int bsrc = !ftile || !valid ? 0 : (y == 0 ? BX : (y == ny - 1 ? -BX : 0));
-    const bool bsink = valid && ((y0 == 0 && cy == 1) || y == ny - 2);
+    // ny-2.  The source row's values come through LDS in the first and the
+    // last tile row (a workgroup-uniform condition: the barriers below are
+    // reached by every thread or none).  A launch of its own for grids whose
+    // last tile row held row ny-1 alone took 38 of the 227 us of a step of 12
+    // small domains.
+    const bool ftile = bottom || top;
+    const int bsrc = !valid ? 0 : (y == 0 ? BX : (y == ny - 1 ? -BX : 0));
+    const bool bsink = valid && (bottom ? y == 1 : y == ny - 2);
     float* rx = L.work;  // A x BX, the planes are no longer needed
     static_assert(sizeof(L.work) / sizeof(float) >= (size_t)A * BX, "roller exchange");
     float wetb = 1.0f;
-    if (!p.fold_rows) {
-        const int side = (y == 1) ? 0 : (y == ny - 2 ? 1 : -1);
-        if (valid && side >= 0) {
-#pragma unroll
-            for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
-                G(f.bnd_e1)[((uint32_t)side * nt + th) * nx + x] = ee.get(th);
-                if (rol) G(f.bnd_r1)[((uint32_t)side * nt + th) * nx + x] = ra[th];
-            }
-        }
-    }
     if (ftile) {
         lds_barrier();  // the last plane and face reads are done, every row of the stash is written
         if (rol && bsink) {
@@ -961,7 +927,7 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
         }
     }
     float Rv = 0.0f, DRv = 0.0f;
-    if (valid) dissip_cell<A, EX, CUR, true>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
+    if (valid) dissip_cell<A, EX, CUR>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
     if (ftile) {
         lds_barrier();  // the source rows' bins after dissipation are in the stash
         if (bsrc != 0) {
@@ -973,7 +939,7 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
         }
     }
     if (valid) {
-        finish_cell<A, EX, true>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
+        finish_cell<A, EX>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
     } else {
         wmin = 9999999.9f;
     }
@@ -1021,8 +987,6 @@ inline WaveK wave_kernel(int nt, bool cur, bool flex) {
     const int A = nt <= 12 ? 12 : (nt <= 24 ? 24 : (nt <= 36 ? 36 : MAXT));
     return WaveK{A, !flex && (nt == 12 || nt == 24), cur, flex};
 }
-// the kernel of rows 0 / ny-1 does not depend on flex
-inline WaveK rows_kernel(WaveK k) { return WaveK{k.A, k.ex, k.cur, false}; }
 #define WAVE_SWITCH_A(C_, F_, k, RUN)                    \
     switch ((k).A) {                                     \
         case 12: RUN(12, false, C_, F_); break;          \
@@ -1049,38 +1013,6 @@ inline WaveK rows_kernel(WaveK k) { return WaveK{k.A, k.ex, k.cur, false}; }
             else WAVE_SWITCH_A(false, false, wk_, RUN)                  \
         }                                                               \
     } while (0)
-
-// Rows 0 and ny-1 (rollerlatbnd, wave_CPU.cpp:830-871): the post-Euler
-// ee/rr of rows 1 / ny-2 times the cell's wet flag, then the cell's own
-// energy..dissipation, and finally ee after dissipation copied again from
-// rows 1 / ny-2.
-template <int A, bool EX, bool CUR>
-XDEV void wave_rows_body(const KP& p, const SP& s, const Fld& f, BI bi) {
-    const int nt = EX ? A : p.nt;
-    int x = bi.x * 256 + threadIdx.x;
-    int side = bi.y;
-    if (x >= p.nx) return;
-    const int nx = p.nx, ny = p.ny;
-    const size_t N = p.N;
-    int y = side ? ny - 1 : 0, ys = side ? ny - 2 : 1;
-    size_t i = (size_t)x + (size_t)y * nx, is = (size_t)x + (size_t)ys * nx;
-    float wet = G(f.hh)[i] > p.eps ? 1.0f : 0.0f;
-    float e[A], r[A], efin[A];
-#pragma unroll
-    for (int th = 0; th < A; th++) {
-        if (th >= nt) break;
-        e[th] = G(f.bnd_e1)[((size_t)side * nt + th) * nx + x] * wet;
-        r[th] = p.roller == 1 ? G(f.bnd_r1)[((size_t)side * nt + th) * nx + x] * wet : act_rr(p, f, x, y, th);
-        efin[th] = G(f.ee_out)[is + (size_t)th * N] * wet;
-    }
-    float Rv, DRv;
-    dissip_cell<A, EX, CUR, false>(p, s, f, f.dirs, i, RegBins{e}, r, Rv, DRv);
-    finish_cell<A, EX, false>(p, s, f, f.dirs, i, RegBins{efin}, r, Rv, DRv);
-}
-template <int A, bool EX, bool CUR>
-__global__ __launch_bounds__(256) void k_wave_rows(KP p, SP s, Fld f) {
-    wave_rows_body<A, EX, CUR>(p, s, f, BI{(int)blockIdx.x, (int)blockIdx.y});
-}
 
 // Operands of wavforceCPU (wave_CPU.cpp:1159-1223) at (x, y).
 struct WfOps {
@@ -2643,11 +2575,7 @@ void make_kp(xbg_ctx* c) {
     k.rvr_alph = -1.0f * xm::log10f(xm::expf(1.0f)) / 0.3539f;
     k.rvr_bet = xm::expf(-0.6065f / 0.3539f);
     k.wtiles_x = (P.nx + BX - 1) / BX;
-    k.wtiles_y = (P.ny + WTY - 1) / WTY;
-    // rows 0 and ny-1 can be finished by the wave kernel's own tiles when
-    // rows 1 and ny-2 lie in the same tile as them and the two boundary
-    // rows lie in different tiles
-    k.fold_rows = P.ny > WTY && (P.ny - 1) % WTY != 0 ? 1 : 0;
+    k.wtiles_y = P.ny > WTY ? (P.ny + WTY - 1) / WTY : 2;  // rows 0 and ny-1 in different tiles
     k.rdtheta = 1.0 / (double)k.dtheta;
     k.dth_recip = k.dtheta > 0.0f && k.dtheta < 2.0f ? 1 : 0;
     {
@@ -2748,16 +2676,11 @@ int launch_wave(xbg_ctx* c, const SP& s, int offshore = 0, int defer_force = 0) 
     const int off_w = c->pre_disp && offshore && !cur ? 1 : 0;
     if (c->pre_disp && offshore && cur)
         LAUNCH(c, "k_bnd_offshore", k_bnd_offshore, dim3(1), dim3(1024), p, s, c->f, 1);
-    const dim3 gr((p.nx + 255) / 256, 2, 1), gw(p.wtiles_x * p.wtiles_y + off_w, 1, 1), bw(BX, WTY, 1);
+    const dim3 gw(p.wtiles_x * p.wtiles_y + off_w, 1, 1), bw(BX, WTY, 1);
     const WaveK k = wave_kernel(p.nt, cur, wave_flex(p, s));
 #define RUN(A_, EX_, C_, F_) LAUNCH(c, "k_wave", (k_wave<A_, EX_, C_, F_>), gw, bw, p, s, c->f, off_w)
     WAVE_SWITCH(k, RUN);
 #undef RUN
-    if (!p.fold_rows) {
-#define RUN(A_, EX_, C_, F_) LAUNCH(c, "k_wave_rows", (k_wave_rows<A_, EX_, C_>), gr, dim3(256), p, s, c->f)
-        WAVE_SWITCH(rows_kernel(k), RUN);
-#undef RUN
-    }
     if (!defer_force) LAUNCH(c, "k_wave_force", k_wave_force, g, blk2, p, c->f);
     c->cur = 1 - c->cur;
     sync_ptrs(c);
@@ -2853,10 +2776,9 @@ int xbg_create(const xbg_params* pin, xbg_ctx** out) {
                      &c->Hmean, &c->uumean, &c->vvmean, &c->hhmean, &c->zsmean, &c->zsmax, &c->Cmean};
     for (auto** q : two) { A(q, N); }
     A(&f.umean, ny);
-    A(&f.bnd_e1, 2 * (size_t)P.ntheta * P.nx); A(&f.bnd_r1, 2 * (size_t)P.ntheta * P.nx);
     A(&f.wet, N);
     if (P.zb_accum == 2) { A(&f.zb64, N); A(&f.zb64_b, N); }
-    c->nblk_wave = ((P.nx + BX - 1) / BX) * ((P.ny + WTY - 1) / WTY);
+    c->nblk_wave = c->kp.wtiles_x * c->kp.wtiles_y;
     c->nblk_flow = (int)((N + 255) / 256);
     c->nblk_sum = 256;
     A(&f.red_wave, c->nblk_wave); A(&f.red_flow, c->nblk_flow); A(&f.red_bad, 4); A(&f.red_acc, 8);
@@ -3706,15 +3628,6 @@ __global__ __launch_bounds__(WTHREADS, wave_occ(A)) void kb_wave(DTab tab, TMap 
     }
 }
 
-template <int A, bool EX, bool CUR>
-__global__ __launch_bounds__(256) void kb_wave_rows(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) wave_rows_body<A, EX, CUR>(D.p, D.s, D.f[D.par][PH_START], BI{e.bx, e.by});
-    }
-}
-
 __global__ __launch_bounds__(256) void kb_flow_nuh(DTab tab, TMap map, int ntiles) {
     ENS_FOR_TILES(map, ntiles) {
         const TileEnt e = map[t_];
@@ -4009,9 +3922,9 @@ __global__ __launch_bounds__(256) void kb_window_sample(DTab tab, TMap map, int 
 }
 
 // Kernels of a step whose launch shape the tuner chooses.
-enum EnsK { EK_CFL, EK_DISP, EK_WAVE, EK_ROWS, EK_NUH, EK_U, EK_V, EK_UVCORR, EK_ZSALL, EK_UVVU, EK_SFLUX, EK_SCONC,
+enum EnsK { EK_CFL, EK_DISP, EK_WAVE, EK_NUH, EK_U, EK_V, EK_UVCORR, EK_ZSALL, EK_UVVU, EK_SFLUX, EK_SCONC,
             EK_SMORPH, EK_N };
-const char* const kEnsName[EK_N] = {"kb_cfl", "kb_dispersion", "kb_wave", "kb_wave_rows", "kb_flow_nuh",
+const char* const kEnsName[EK_N] = {"kb_cfl", "kb_dispersion", "kb_wave", "kb_flow_nuh",
                                     "kb_flow_u", "kb_flow_v", "kb_flow_uvcorr", "kb_flow_zsall", "kb_flow_uvvu",
                                     "kb_sed_flux", "kb_sed_conc", "kb_sed_morph"};
 // patch shapes (one wavefront) offered for the dispersion and concentration
@@ -4039,10 +3952,9 @@ struct xbg_ens {
     std::vector<int> base_cur, base_zcur, base_ccur;
     DomDesc* dtab = nullptr;
     hipStream_t stream = nullptr;
-    TileMap m_cfl, m_2d, m_corr, m_rows[3];  // rows per nt class (12, 24, other)
+    TileMap m_cfl, m_2d, m_corr;
     TileMap m_disp[N_SHAPE], m_conc[N_SHAPE];
     std::vector<WaveGroup> waves;
-    std::vector<WaveGroup> rows;
     float* part = nullptr;
     // launch choices (tuned)
     int disp_shape = 0, conc_shape = 2;  // 4x16 dispersion, 16x4 concentration (the single-domain shapes)
@@ -4137,14 +4049,6 @@ int ens_launch_step(xbg_ens* e) {
 #undef RUN
     }
     ens_ev(e, 2 * EK_WAVE + 1);
-    ens_ev(e, 2 * EK_ROWS);
-    for (const WaveGroup& w : e->rows) {
-#define RUN(A_, EX_, C_, F_) \
-    kb_wave_rows<A_, EX_, C_><<<dim3(w.map.n), dim3(256), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
-        WAVE_SWITCH(w.k, RUN);
-#undef RUN
-    }
-    ens_ev(e, 2 * EK_ROWS + 1);
     const TileMap& m2 = e->m_2d;
     const TileMap& mc = e->m_corr;
 #define EL(k, kern, blk, m)                                                                                 \
@@ -4215,7 +4119,7 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
     };
     std::vector<int> doms_all, gx2, gy2, gxc, gyc, gxcfl, gycfl;
     std::vector<TileEnt> cfl;
-    std::map<WaveK, std::vector<TileEnt>> wave_tiles, row_tiles;
+    std::map<WaveK, std::vector<TileEnt>> wave_tiles;
     e->h.resize(ndom);
     for (int d = 0; d < ndom; d++) {
         xbg_ctx* c = ctxs[d];
@@ -4290,11 +4194,6 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
         while (wv.size() % 8) wv.push_back(TileEnt{d, -1, 0, 0});
         const int ntw = p.wtiles_x * p.wtiles_y;
         for (int b = 0; b < ntw; b++) wv.push_back(TileEnt{d, xcd_tile(b, ntw), 0, 0});
-        if (!p.fold_rows) {
-            auto& rv = row_tiles[rows_kernel(wk)];
-            for (int side = 0; side < 2; side++)
-                for (int bx = 0; bx < (p.nx + 255) / 256; bx++) rv.push_back(TileEnt{d, bx, side, 0});
-        }
     }
     int rc = 0;
     EHIP(e, hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
@@ -4323,11 +4222,6 @@ int xbg_ens_create(int ndom, xbg_ctx* const* ctxs, const xbg_ens_domain* run, xb
         WaveGroup w{kv.first, TileMap{}};
         if ((rc = upload_map(e, w.map, kv.second))) return bail(rc);
         e->waves.push_back(w);
-    }
-    for (auto& kv : row_tiles) {
-        WaveGroup w{kv.first, TileMap{}};
-        if ((rc = upload_map(e, w.map, kv.second))) return bail(rc);
-        e->rows.push_back(w);
     }
     e->ev.resize(2 * EK_N);
     for (auto& q : e->ev) EHIP(e, hipEventCreate(&q));
@@ -4501,7 +4395,6 @@ int xbg_ens_destroy(xbg_ens* e) {
         if (e->m_conc[s].d) hipFree(e->m_conc[s].d);
     }
     for (auto& w : e->waves) if (w.map.d) hipFree(w.map.d);
-    for (auto& w : e->rows) if (w.map.d) hipFree(w.map.d);
     if (e->part) hipFree(e->part);
     for (auto& D : e->h)
         if (D.win) hipFree(D.win);
