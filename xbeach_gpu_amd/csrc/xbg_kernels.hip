@@ -388,7 +388,22 @@ struct LdsBins {
     XDEV float get(int th) const { return a[th * STRIDE]; }
     XDEV void set(int th, float v) const { a[th * STRIDE] = v; }
 };
-template <int A, bool EX, bool CUR, class B>
+// The unrolled loops over the bins of a kernel whose count the compiler does
+// not know (EX false) end at the first bin past the last one, or (guarded)
+// skip each of those: where a thread's bins are more than 12 registers, the
+// early ends cost the allocation some forty more and 10 to 20 spilled (at
+// 1500 x 800: 16 bins 235 -> 197 us, 20 bins 285 -> 236; 36 bins at
+// 600 x 400 126 -> 119; 18 bins at 413 x 287 50 -> 39.5).  Not guarded: up to 12 bins, equal; 64,
+// whose bins are in scratch anyway (48 bins at 600 x 400: 165 against
+// 210 us); with currents and FLEX above 18, where the guards' conditions
+// overflow the scalar registers.
+constexpr bool wave_guard(int A, bool cur, bool flex) { return A > 12 && A <= (cur && flex ? 18 : 36); }
+#define BIN_STOP(c) \
+    if (c) {        \
+        if (GUARD) continue; \
+        break;      \
+    }
+template <int A, bool EX, bool CUR, bool GUARD, class B>
 XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const B e, float* r,
                       float& Rout, float& DRout) {
     const int nt = EX ? A : p.nt;
@@ -397,7 +412,7 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
     uint32_t m = 0xffffffffu;
 #pragma unroll
     for (int th = 0; th < A; th++) {
-        if (th >= nt) break;
+        BIN_STOP(th >= nt);
         const float v = fmx(e.get(th) * s.sigm, 0.0f);
         e.set(th, v);
         Et = Et + v;
@@ -427,7 +442,7 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
     if (idiv != 1.0f) {
 #pragma unroll
         for (int th = 0; th < A; th++) {
-            if (th >= nt) break;
+            BIN_STOP(th >= nt);
             e.set(th, e.get(th) / idiv);
         }
     }
@@ -449,7 +464,7 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
         const double rE = 1.0 / (double)Emx, c0 = (double)cc, rc = 1.0 / c0, hc = 0.5 * rc;
 #pragma unroll
         for (int th = 0; th < A; th++) {
-            if (th >= nt) break;
+            BIN_STOP(th >= nt);
             float eet = e.get(th);
             float cx = CUR ? cc * dirs[1 * MAXT + th] + uui : cc * dirs[1 * MAXT + th];
             float cy = CUR ? cc * dirs[2 * MAXT + th] + vvi : cc * dirs[2 * MAXT + th];
@@ -481,7 +496,7 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
 // meandirCPU (wave_CPU.cpp:1092-1116), radstressCPU (1118-1157) and
 // breakerdelayCPU (1334-1374, called with R) at cell i on the final ee/rr;
 // stores the directional state of the cell.
-template <int A, bool EX, class B>
+template <int A, bool EX, bool GUARD, class B>
 XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs, size_t i, const B efin,
                       const float* r, float Rv, float DRv) {
     const int nt = EX ? A : p.nt;
@@ -491,7 +506,7 @@ XDEV void finish_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
     float sume = 0.0f, sumethet = 0.0f, txx = 0.0f, tyy = 0.0f, txy = 0.0f, rxx = 0.0f, ryy = 0.0f, rxy = 0.0f;
 #pragma unroll
     for (int th = 0; th < A; th++) {
-        if (th >= nt) break;
+        BIN_STOP(th >= nt);
         float ev = efin.get(th), rv = r[th];
         sume = sume + ev;
         sumethet = sumethet + ev * dirs[0 * MAXT + th];
@@ -628,6 +643,7 @@ struct WaveLds {
 template <int A, bool EX, bool CUR, bool FLEX>
 XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f, int x0, int y0, int x, int y, int cx,
                       int cy, float* ra) {
+    constexpr bool GUARD = wave_guard(A, CUR, FLEX);
     const int nt = EX ? A : p.nt;
     const int tid = cx + cy * BX, nx = p.nx, ny = p.ny;
     const uint32_t N = p.N;
@@ -708,7 +724,7 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
     float cs1 = 0, sn1 = 0, ctl = 0, cm = 0;
 #pragma unroll
     for (int th = 0; th <= A; th++) {
-        if (!EX && th > nt) break;
+        BIN_STOP(!EX && th > nt);
         const bool bin = EX ? th < A : th < nt;
         float ec = e1, rc = r1, cs = 0, sn = 0;  // past the last bin: the clamped neighbour
         float gbe = 0, gbr = 0, lxe = 0, lxr = 0;
@@ -855,6 +871,7 @@ constexpr int wave_occ(int A) { return A <= 24 ? 4 : 2; }
 template <int A, bool EX, bool CUR, bool FLEX>
 XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CUR>& L) {
     static_assert(A > 24 || 2 * sizeof(WaveLds<A, CUR>) <= 160 * 1024, "two workgroups per CU");
+    constexpr bool GUARD = wave_guard(A, CUR, FLEX);
     const int nt = EX ? A : p.nt;
     const int cx = threadIdx.x, cy = threadIdx.y, tid = cx + cy * BX;
     const int tile = bi.x;  // tile of the domain, after the XCD remap
@@ -881,7 +898,7 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
     if (!rol) {
 #pragma unroll
         for (int th = 0; th < A; th++) {
-            if (th >= nt) break;
+            BIN_STOP(th >= nt);
             ra[th] = G(f.rr_in)[i + (uint32_t)th * p.N];
         }
     }
@@ -904,7 +921,7 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
         if (rol && bsink) {
 #pragma unroll
             for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
+                BIN_STOP(th >= nt);
                 rx[th * BX + cx] = ra[th];
             }
         }
@@ -912,7 +929,7 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
             wetb = G(f.hh)[i] > p.eps ? 1.0f : 0.0f;
 #pragma unroll
             for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
+                BIN_STOP(th >= nt);
                 ee.set(th, L.stash[th][tid + bsrc] * wetb);
             }
         }
@@ -920,25 +937,25 @@ XDEV void wave_body(const KP& p, const SP& s, const Fld& f, BI bi, WaveLds<A, CU
         if (rol && bsrc != 0) {
 #pragma unroll
             for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
+                BIN_STOP(th >= nt);
                 ra[th] = rx[th * BX + cx] * wetb;
             }
         }
     }
     float Rv = 0.0f, DRv = 0.0f;
-    if (valid) dissip_cell<A, EX, CUR>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
+    if (valid) dissip_cell<A, EX, CUR, GUARD>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
     if (ftile) {
         lds_barrier();  // the source rows' bins after dissipation are in the stash
         if (bsrc != 0) {
 #pragma unroll
             for (int th = 0; th < A; th++) {
-                if (th >= nt) break;
+                BIN_STOP(th >= nt);
                 ee.set(th, L.stash[th][tid + bsrc] * wetb);
             }
         }
     }
     if (valid) {
-        finish_cell<A, EX>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
+        finish_cell<A, EX, GUARD>(p, s, f, L.dirs, i, ee, ra, Rv, DRv);
     } else {
         wmin = 9999999.9f;
     }
@@ -969,8 +986,8 @@ __global__ __launch_bounds__(WTHREADS, wave_occ(A)) void k_wave(KP p, SP s, Fld 
 }
 
 // The wave kernel of a number of bins: 12 and 24 have one with every count
-// known to the compiler; other counts run in the smallest of 12, 24, 36 and
-// 64 bins that holds them (registers and LDS are sized by it; one kernel of
+// known to the compiler; other counts run in the smallest of 12, 18, 24, 36
+// and 64 bins that holds them (registers and LDS are sized by it; one kernel of
 // 64 bins for all, its arrays in scratch, and its boundary rows in a launch
 // of their own took 57 + 34 us at 413 x 287 x 18).  flex: the
 // roller is off, or sigm or dtheta is not below 2.
@@ -983,12 +1000,13 @@ struct WaveK {
 };
 inline bool wave_flex(const KP& p, const SP& s) { return p.roller != 1 || !(s.sigm_recip && p.dth_recip); }
 inline WaveK wave_kernel(int nt, bool cur, bool flex) {
-    const int A = nt <= 12 ? 12 : (nt <= 24 ? 24 : (nt <= 36 ? 36 : MAXT));
+    const int A = nt <= 12 ? 12 : (nt <= 18 ? 18 : (nt <= 24 ? 24 : (nt <= 36 ? 36 : MAXT)));
     return WaveK{A, !flex && (nt == 12 || nt == 24), cur, flex};
 }
 #define WAVE_SWITCH_A(C_, F_, k, RUN)                    \
     switch ((k).A) {                                     \
         case 12: RUN(12, false, C_, F_); break;          \
+        case 18: RUN(18, false, C_, F_); break;          \
         case 24: RUN(24, false, C_, F_); break;          \
         case 36: RUN(36, false, C_, F_); break;          \
         default: RUN(MAXT, false, C_, F_); break;        \
