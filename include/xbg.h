@@ -460,7 +460,8 @@ int xbg_sur_loss(xbg_sur* s, const void* x, const void* t, int n, double* loss);
 int xbg_sur_backward(xbg_sur* s, const void* x, const void* t, int n, double* loss);
 /* One Adam step (beta 0.9 / 0.999, eps 1e-8) at learning rate lr; loss is
  * the batch loss before the update.  Returns without waiting for the
- * update (xbg_sur_sync). */
+ * gradients and the update (xbg_sur_sync); x and t are no longer read then
+ * and may be refilled or freed. */
 int xbg_sur_train_step(xbg_sur* s, const void* x, const void* t, int n, double lr, double* loss);
 int xbg_sur_sync(xbg_sur* s);
 /* One convolution on caller device buffers ('same' padding, taps 9 = 3x3

@@ -771,9 +771,9 @@ struct xbg_sur {
     double* hloss = nullptr;                                       // the loss on the host (pinned)
     hipEvent_t loss_done = nullptr;
     int adam_t = 0;
-    // activations (A) and their gradients (D), by name
+    // the batch, activations (A) and their gradients (D), by name
     std::vector<void*> allocs;
-    bf16 *e0a, *e0, *p1, *e1a, *e1, *p2, *e2a, *e2, *p3, *b3a, *b3, *u2, *d2a, *d2, *u1, *d1a, *d1,
+    bf16 *x8, *e0a, *e0, *p1, *e1a, *e1, *p2, *e2a, *e2, *p3, *b3a, *b3, *u2, *d2a, *d2, *u1, *d1a, *d1,
         *u0, *d0a, *d0;
     bf16 *g_e0a, *g_e0, *g_e1a, *g_e1, *g_e2a, *g_e2, *g_b3a, *g_b3, *g_u2, *g_d2a,
         *g_d2, *g_u1, *g_d1a, *g_d1, *g_u0, *g_d0a, *g_d0;
@@ -1002,7 +1002,7 @@ int xbg_sur_create(int nmax, int H, int W, unsigned seed, xbg_sur** out) {
     struct B {
         bf16** p;
         size_t n;
-    } acts[] = {{&s->e0a, P0 * 32}, {&s->e0, P0 * 32},  {&s->p1, P1 * 32},
+    } acts[] = {{&s->x8, P0 * 8}, {&s->e0a, P0 * 32}, {&s->e0, P0 * 32},  {&s->p1, P1 * 32},
                 {&s->e1a, P1 * 64}, {&s->e1, P1 * 64},  {&s->p2, P2 * 64},  {&s->e2a, P2 * 128},
                 {&s->e2, P2 * 128}, {&s->p3, P3 * 128}, {&s->b3a, P3 * 256}, {&s->b3, P3 * 256},
                 {&s->u2, P3 * 128}, {&s->d2a, P2 * 128}, {&s->d2, P2 * 128},
@@ -1206,12 +1206,17 @@ int xbg_sur_loss(xbg_sur* s, const void* x8, const void* t5, int n, double* loss
 }  // extern "C"
 
 namespace {
-// forward, loss and every parameter gradient, queued
+// Forward, loss and every parameter gradient, queued.  The caller may refill
+// or free its batch once the loss is there, with the backward still running,
+// whose last kernel (layer 0's weight gradient) reads the inputs: that takes
+// a copy, made ahead of the loss.
 int sur_gradients(xbg_sur* s, const void* x8, const void* t5, int n) {
     if (!s || !x8 || !t5 || n < 1 || n > s->nmax) return sfail(s, XBG_E_ARG, "xbg_sur_backward: bad argument");
-    int rc = sur_forward(s, (const bf16*)x8, n, s->y);
+    SHIP(s, hipMemcpyAsync(s->x8, x8, (size_t)n * s->H * s->W * 8 * sizeof(bf16), hipMemcpyDeviceToDevice, s->st));
+    int rc = sur_forward(s, s->x8, n, s->y);
     if (!rc) rc = sur_loss_grad(s, (const bf16*)t5, n, 1);
-    if (!rc) rc = sur_backward(s, (const bf16*)x8, n);
+    if (!rc) rc = sur_backward(s, s->x8, n);
+    if (rc) hipStreamSynchronize(s->st);  // nothing queued reads the batch after an error either
     return rc;
 }
 }  // namespace
