@@ -437,7 +437,9 @@ int xbg_ens_destroy(xbg_ens* e);
  * on the matrix cores (v_mfma_f32_16x16x32_bf16), FP32 master weights and
  * Adam.  Tensors are NHWC DEVICE buffers: inputs BF16 [n][H][W][8] (the 7
  * channels and a zero), targets BF16 [n][H][W][5], outputs FP32
- * [n][H][W][5], all normalised per channel by the caller.
+ * [n][H][W][5], all normalised per channel by the caller.  The library
+ * works on a non-blocking stream of its own: buffers handed to a call are
+ * complete before it (it waits for no other stream).
  * ---------------------------------------------------------------------- */
 typedef struct xbg_sur xbg_sur;
 /* Buffers for batches of up to nmax images of H x W (H a multiple of 16,

@@ -186,6 +186,17 @@ class Dataset:
         return np.concatenate([m[7:], s[7:]]).astype(np.float32)
 
 
+def gather(X, T, idx):
+    """The batch idx of X and T, complete when this returns: the library's
+    stream does not wait for torch's, on which the batch is gathered."""
+    import torch
+
+    xb = X.index_select(0, idx).contiguous()
+    tb = T.index_select(0, idx).contiguous()
+    torch.cuda.current_stream().synchronize()
+    return xb, tb
+
+
 def train(X, T, epochs: int, batch: int = 64, lr: float = 1e-3, seed: int = 0, log=print, lr_final=None):
     """Adam on 80 % of the samples, at learning rate lr (with lr_final set,
     cosine decay from lr to lr_final over the run); returns (surrogate,
@@ -211,8 +222,7 @@ def train(X, T, epochs: int, batch: int = 64, lr: float = 1e-3, seed: int = 0, l
         nb = 0
         for k in range(0, ntr - batch + 1, batch):
             idx = order[k:k + batch]
-            xb = X.index_select(0, idx).contiguous()
-            tb = T.index_select(0, idx).contiguous()
+            xb, tb = gather(X, T, idx)
             lr_k = lr_end + 0.5 * (lr - lr_end) * (1.0 + math.cos(math.pi * nstep / max(total - 1, 1)))
             tot += sur.train_step(xb.data_ptr(), tb.data_ptr(), batch, lr_k)
             nb += 1
@@ -229,8 +239,7 @@ def evaluate(sur, X, T, idx, batch):
     tot, n = 0.0, 0
     for k in range(0, len(idx), batch):
         ii = idx[k:k + batch]
-        xb = X.index_select(0, ii).contiguous()
-        tb = T.index_select(0, ii).contiguous()
+        xb, tb = gather(X, T, ii)
         tot += sur.loss(xb.data_ptr(), tb.data_ptr(), len(ii)) * len(ii)
         n += len(ii)
     return tot / max(n, 1)

@@ -5,6 +5,8 @@ and Adam run on the device (xbeach_gpu_amd/csrc/xbg_sur.hip).
 Buffers cross as raw device pointers (e.g. ``tensor.data_ptr()`` of a
 torch tensor on the GPU): inputs BF16 [n][H][W][8], targets BF16
 [n][H][W][5], outputs FP32 [n][H][W][5], NHWC, normalised per channel.
+The library's stream waits for no other one: what torch queued to fill a
+buffer is synchronised before the call.
 """
 from __future__ import annotations
 
