@@ -416,8 +416,7 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
         const float v = fmx(e.get(th) * s.sigm, 0.0f);
         e.set(th, v);
         Et = Et + v;
-        // smallest magnitude that is not zero (zero wraps to the largest)
-        if (!CUR) m = min(m, min((__float_as_uint(v) << 1) - 1u, (__float_as_uint(r[th]) << 1) - 1u));
+        if (!CUR) m = xm::nonzero_min(xm::nonzero_min(m, v), r[th]);
     }
     Et = Et * p.dtheta;
     float Ht = sqrtf(Et / (p.rho * p.g / 8.0f));
@@ -450,15 +449,12 @@ XDEV void dissip_cell(const KP& p, const SP& s, const Fld& f, const float* dirs,
     // every bin of the cell, and without the current the square root is the
     // cell's c times sqrt(cos^2 + sin^2) of the bin, which rounds near c; so
     // the IEEE results come from a few double operations on per-cell
-    // reciprocals (20 instead of 36 instructions a bin), where no quotient
-    // can be subnormal: in the wavefronts whose cells have c in range, no
-    // bin between zero and 2^-90 (before energint's cap), and factors of at
-    // least 2^-30.  The wave kernel at 2048 x 1024 x 24: 366 -> 353 us with the
-    // ee bins left in LDS; asking each quotient instead cost more than it
-    // saved (376 us).
+    // reciprocals (20 instead of 36 instructions a bin), in the wavefronts
+    // where no quotient can be subnormal.  The wave kernel at 2048 x 1024 x
+    // 24: 366 -> 353 us with the ee bins left in LDS; asking each quotient
+    // instead cost more than it saved (376 us).
     const float gb = 2.0f * p.g * p.beta;
-    const bool fast = !CUR && cc > 1e-10f && cc < 1e10f && !(Dv != 0.0f && Dv < 9.3e-10f * Emx) &&
-                      (gb == 0.0f || gb >= 1e-5f * cc) && idiv < 1e6f && m >= (__float_as_uint(8.1e-28f) << 1);
+    const bool fast = !CUR && xm::no_subnormal(cc, Dv, Emx, gb, idiv, m);
     auto bins = [&](auto near_c) {
         constexpr bool NEAR = decltype(near_c)::value;
         const double rE = 1.0 / (double)Emx, c0 = (double)cc, rc = 1.0 / c0, hc = 0.5 * rc;

@@ -327,6 +327,21 @@ XM_FN float div_near(float a, float q, double rc) {
 // a / b with rb = 1 / (double)b
 XM_FN float div_by(float a, double rb) { return (float)((double)a * rb); }
 
+// The wave dissipation's bins take these forms where no quotient of the cell
+// can be subnormal.  The quotients are (a D) / E of the ee bins after a cap by
+// idiv >= 1, and (gb b) / q of the rr bins, q within a factor 1 +- 2^-20 of c.
+// small: nonzero_min over the ee bins before the cap and the rr bins; E >= 1e-7.
+// Bins of at least 2^-90 after the cap and factors of at least 2^-31 leave
+// quotients above 2^-122.
+XM_FN uint32_t nonzero_min(uint32_t small, float v) {
+    const uint32_t m = (__builtin_bit_cast(uint32_t, v) << 1) - 1u;  // zero wraps to the largest
+    return m < small ? m : small;
+}
+XM_FN bool no_subnormal(float c, float D, float E, float gb, float idiv, uint32_t small) {
+    return c > 1e-10f && c < 1e10f && !(D != 0.0f && D < 9.3e-10f * E) && (gb == 0.0f || gb >= 1e-5f * c) &&
+           idiv < 1e6f && small >= (__builtin_bit_cast(uint32_t, 8.1e-28f * idiv) << 1);
+}
+
 // ---- float entry points: one rounding of the double result ----
 XM_FN float expf(float x) { return (float)exp((double)x); }
 XM_FN float logf(float x) { return (float)log((double)x); }
