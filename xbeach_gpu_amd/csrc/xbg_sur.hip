@@ -335,7 +335,9 @@ __global__ __launch_bounds__(256, 2) void k_conv(CSrc X, const bf16* __restrict_
 // reductions take 1.8 ms, and took 8.2 ms before (one copy of X per shift,
 // transposed in registers, every X row read three times; bias sums in a pass
 // of their own).
-// Requires Cout % CBO == 0, Cin % CBI == 0; any W (pixels past it are zero).
+// Requires Cout % CBO == 0, Cin % CBI == 0; W % SEG == 0 unless RAGGED, whose
+// pixels past W have zero gradients; the column before them is taken out of
+// their products, where an infinite input would give NaN (0 x inf).
 // ---------------------------------------------------------------------------
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 // Lane l of a wave gets channel l % 16 at the eight pixels 8 (l / 16) + 0..7
@@ -356,7 +358,7 @@ struct WShape {
     static constexpr int RW = 2, RS = (WK / KG) * RW;                // rows per wave and per stage
 };
 
-template <int TAPS, int CBO, int CBI, int SEG>
+template <int TAPS, int CBO, int CBI, int SEG, bool RAGGED>
 __global__ __launch_bounds__(256, 2) void k_conv_wgrad(CSrc X, const bf16* __restrict__ dZ, float* __restrict__ part,
                                                        int N, int H, int W, int Cin, int Cout, int rows_per_split) {
     using S = WShape<CBO, CBI, SEG>;
@@ -452,7 +454,14 @@ __global__ __launch_bounds__(256, 2) void k_conv_wgrad(CSrc X, const bf16* __res
                     for (int dx = 0; dx < NDX; dx++) {
                         bf16x8 b[2];
 #pragma unroll
-                        for (int u = 0; u < 2; u++) b[u] = tr_frag<PX>(sX + slot * XROW + (p0 + dx) * PX + is + 16 * u, lane);
+                        for (int u = 0; u < 2; u++) {
+                            b[u] = tr_frag<PX>(sX + slot * XROW + (p0 + dx) * PX + is + 16 * u, lane);
+                            if (RAGGED && dx == 0) {
+#pragma unroll
+                                for (int e = 0; e < 8; e++)
+                                    if (x0 + p0 + 8 * s + e >= W) b[u][e] = to_bf16(0.0f);
+                            }
+                        }
 #pragma unroll
                         for (int z = 0; z < RW; z++) {
                             const int dy = xr - z;
@@ -901,15 +910,18 @@ int conv_wgrad(hipStream_t st, CSrc X, const bf16* dZ, float* dW, float* db, flo
         *used = 0;
     }
     part += *used;
-#define CW(T_, O_, I_)                                                                                                  \
-    do {                                                                                                                \
-        if (SEG == 64) k_conv_wgrad<T_, O_, I_, 64><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps);      \
-        else k_conv_wgrad<T_, O_, I_, 32><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps);                \
+#define CWK(T_, O_, I_, S_, R_) k_conv_wgrad<T_, O_, I_, S_, R_><<<g, dim3(256), 0, st>>>(X, dZ, part, n, H, W, Cin, Cout, rps)
+#define CW(T_, O_, I_)                                               \
+    do {                                                             \
+        if (SEG == 64) CWK(T_, O_, I_, 64, false);                   \
+        else if (T_ == 9 && W % 32) CWK(T_, O_, I_, 32, T_ == 9);    \
+        else CWK(T_, O_, I_, 32, false);                             \
     } while (0)
 #define CW_I(T_, O_) do { if (CBI == 64) CW(T_, O_, 64); else CW(T_, O_, 32); } while (0)
 #define CW_O(T_) do { if (CBO == 64) CW_I(T_, 64); else CW_I(T_, 32); } while (0)
     if (taps == 9) CW_O(9);
     else CW_O(1);
+#undef CWK
 #undef CW
 #undef CW_I
 #undef CW_O
