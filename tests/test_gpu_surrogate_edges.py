@@ -46,3 +46,21 @@ def test_infinite_inputs_stay_in_their_taps(need_gpu, n, H, W, cin, cout, taps):
     assert fin.any() and (~fin).any() and not np.isnan(ref).any()
     assert np.array_equal(got[~fin], ref[~fin])
     assert np.abs(got[fin] - ref[fin]).max() <= 1e-5 * np.abs(ref[fin]).max()
+
+
+@pytest.mark.parametrize("cin,cout,taps,rc", [(4096, 4096, 1, 0), (448, 4160, 9, 0), (4096, 4128, 1, -1)])
+def test_largest_weight_gradient(need_gpu, cin, cout, taps, rc):
+    """Layers of up to 2^24 weights are taken, larger ones are refused."""
+    n, H, W = 1, 2, 32
+    g = torch.Generator().manual_seed(cout)
+    X = torch.randn(n, H, W, cin, generator=g).to(torch.bfloat16)
+    dZ = torch.randn(n, H, W, cout, generator=g).to(torch.bfloat16)
+    Xd, dZd = X.cuda(), dZ.cuda()
+    dW, db = torch.empty(taps, cout, cin, device="cuda"), torch.empty(cout, device="cuda")
+    torch.cuda.synchronize()
+    got = lib().xbg_sur_conv_wgrad(Xd.data_ptr(), dZd.data_ptr(), dW.data_ptr(), db.data_ptr(), n, H, W, cin, cout, taps)
+    assert (got == 0) == (rc == 0)
+    if rc == 0:
+        for a, r in ((dW.cpu().double().numpy(), taps_gradient(X, dZ, taps)),
+                     (db.cpu().double().numpy(), dZ.double().numpy().reshape(-1, cout).sum(0))):
+            assert np.abs(a - r).max() <= 1e-5 * np.abs(r).max()

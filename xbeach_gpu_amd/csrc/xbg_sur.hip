@@ -1289,7 +1289,8 @@ int xbg_sur_conv_dgrad(const void* dZ, const void* Wt, void* dX, int n, int H, i
 
 int xbg_sur_conv_wgrad(const void* X, const void* dZ, float* dW, float* db, int n, int H, int W, int Cin, int Cout,
                        int taps) {
-    size_t np = (size_t)16 << 20;
+    // weights of up to 16 M values, with their bias sums
+    const size_t np = ((size_t)16 << 20) + (Cout > 0 ? Cout : 0);
     float* part = nullptr;
     if (hipMalloc((void**)&part, np * 4) != hipSuccess) return XBG_E_HIP;
     SumJobs J{};
