@@ -64,3 +64,29 @@ def test_largest_weight_gradient(need_gpu, cin, cout, taps, rc):
         for a, r in ((dW.cpu().double().numpy(), taps_gradient(X, dZ, taps)),
                      (db.cpu().double().numpy(), dZ.double().numpy().reshape(-1, cout).sum(0))):
             assert np.abs(a - r).max() <= 1e-5 * np.abs(r).max()
+
+
+def test_data_gradient_of_more_than_2_31_weights(need_gpu):
+    """The flipped weights are indexed beyond 2^31: a few weights set, products
+    and sums of small integers, so exact."""
+    n, H, W, cin, cout, taps = 1, 2, 32, 15456, 15456, 9
+    if torch.cuda.mem_get_info()[0] < 12 << 30:
+        pytest.skip("needs 12 GB")
+    rng = np.random.default_rng(5)
+    Wt = torch.zeros(taps * cout * cin, dtype=torch.bfloat16, device="cuda")
+    assert Wt.numel() > 1 << 31
+    at = np.concatenate([rng.integers(0, Wt.numel(), 200), rng.integers(1 << 31, Wt.numel(), 50),
+                         [0, (1 << 31) - 1, 1 << 31, Wt.numel() - 1]])
+    at = np.unique(at)
+    val = rng.integers(1, 5, at.size)
+    Wt[torch.as_tensor(at).cuda()] = torch.as_tensor(val).to(torch.bfloat16).cuda()
+    dZ = rng.integers(-3, 4, (H, W, cout))
+    dZd = torch.as_tensor(dZ).to(torch.bfloat16).cuda()
+    dX = torch.full((H, W, cin), float("nan"), dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+    assert lib().xbg_sur_conv_dgrad(dZd.data_ptr(), Wt.data_ptr(), dX.data_ptr(), n, H, W, cin, cout, taps) == 0
+    ref = np.zeros((H + 2, W + 2, cin))
+    for i, v in zip(at, val):
+        tap, co, ci = i // (cout * cin), i // cin % cout, i % cin
+        ref[tap // 3:tap // 3 + H, tap % 3:tap % 3 + W, ci] += v * dZ[:, :, co]
+    assert np.array_equal(dX.cpu().double().numpy(), ref[1:-1, 1:-1])

@@ -603,9 +603,10 @@ __global__ __launch_bounds__(256) void k_flip_weights(const bf16* __restrict__ W
     int k = 0;
     while (k + 1 < J.count && (int)blockIdx.x >= J.j[k + 1].blk0) k++;
     const FlipJob q = J.j[k];
-    const int i = (blockIdx.x - q.blk0) * 256 + threadIdx.x;
-    if (i >= q.taps * q.cout * q.cin) return;
-    const int ci = i % q.cin, co = i / q.cin % q.cout, tap = i / q.cin / q.cout;
+    const size_t i = (size_t)(blockIdx.x - q.blk0) * 256 + threadIdx.x;  // a layer may have 2^31 weights or more
+    if (i >= (size_t)q.taps * q.cout * q.cin) return;
+    const size_t r = i / q.cin;
+    const int ci = i % q.cin, co = r % q.cout, tap = r / q.cout;
     Wd[q.w + ((size_t)(q.taps - 1 - tap) * q.cin + ci) * q.cout + co] = Wt[q.w + i];
 }
 
