@@ -410,8 +410,9 @@ int xbg_ens_status(xbg_ens* e, double* t, double* dt, int* steps, int* status);
 int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n);
 /* Average duration (us) of each kernel class over nsteps steps run with
  * events (these steps advance the ensemble); us has XBG_ENS_NKERNELS entries
- * named by xbg_ens_kernel_name. */
-#define XBG_ENS_NKERNELS 12
+ * named by xbg_ens_kernel_name (0 for kb_wave_rows, whose rows are part of
+ * kb_wave). */
+#define XBG_ENS_NKERNELS 13
 int xbg_ens_kernel_times(xbg_ens* e, int nsteps, double* us);
 const char* xbg_ens_kernel_name(int k);
 /* Wave-group window means for surrogate training data: _enable allocates

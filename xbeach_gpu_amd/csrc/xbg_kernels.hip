@@ -3930,10 +3930,13 @@ __global__ __launch_bounds__(256) void kb_window_sample(DTab tab, TMap map, int 
     }
 }
 
-// Kernels of a step whose launch shape the tuner chooses.
-enum EnsK { EK_CFL, EK_DISP, EK_WAVE, EK_NUH, EK_U, EK_V, EK_UVCORR, EK_ZSALL, EK_UVVU, EK_SFLUX, EK_SCONC,
+// Kernel classes of a step, in the order of the public array of their times.
+// EK_ROWS has no launch (the boundary rows are part of kb_wave): it keeps the
+// others' places for callers, and its time is 0.
+enum EnsK { EK_CFL, EK_DISP, EK_WAVE, EK_ROWS, EK_NUH, EK_U, EK_V, EK_UVCORR, EK_ZSALL, EK_UVVU, EK_SFLUX, EK_SCONC,
             EK_SMORPH, EK_N };
-const char* const kEnsName[EK_N] = {"kb_cfl", "kb_dispersion", "kb_wave", "kb_flow_nuh",
+static_assert(EK_N == XBG_ENS_NKERNELS, "the public array");
+const char* const kEnsName[EK_N] = {"kb_cfl", "kb_dispersion", "kb_wave", "kb_wave_rows", "kb_flow_nuh",
                                     "kb_flow_u", "kb_flow_v", "kb_flow_uvcorr", "kb_flow_zsall", "kb_flow_uvvu",
                                     "kb_sed_flux", "kb_sed_conc", "kb_sed_morph"};
 // patch shapes (one wavefront) offered for the dispersion and concentration
@@ -4293,7 +4296,7 @@ int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n) {
         EHIP(e, hipStreamSynchronize(e->stream));
         for (int k = 0; k < EK_N; k++) {
             float ms = 0.0f;
-            if (hipEventElapsedTime(&ms, e->ev[2 * k], e->ev[2 * k + 1]) != hipSuccess) continue;
+            if (k == EK_ROWS || hipEventElapsedTime(&ms, e->ev[2 * k], e->ev[2 * k + 1]) != hipSuccess) continue;
             tk[k] += ms;
             ck[k] += 1;
             if (k == EK_DISP) { td[e->disp_shape] += ms; cd[e->disp_shape]++; }
@@ -4304,6 +4307,7 @@ int xbg_ens_tune(xbg_ens* e, int rounds, char* report, size_t n) {
     std::string out;
     char line[256];
     for (int k = 0; k < EK_N; k++) {
+        if (k == EK_ROWS) continue;
         snprintf(line, sizeof(line), "%s us=%.2f\n", kEnsName[k], ck[k] ? 1000.0 * tk[k] / ck[k] : 0.0);
         out += line;
     }
@@ -4339,6 +4343,7 @@ int xbg_ens_kernel_times(xbg_ens* e, int nsteps, double* us) {
         EHIP(e, hipStreamSynchronize(e->stream));
         for (int k = 0; k < EK_N; k++) {
             float ms = 0.0f;
+            if (k == EK_ROWS) continue;
             if (hipEventElapsedTime(&ms, e->ev[2 * k], e->ev[2 * k + 1]) == hipSuccess) us[k] += 1000.0 * ms / nsteps;
         }
     }

@@ -78,9 +78,9 @@ class Ensemble:
         return buf.value.decode()
 
     def kernel_times(self, nsteps: int = 5) -> dict:
-        us = np.zeros(12)
+        us = np.zeros(13)
         self._chk(self.L.xbg_ens_kernel_times(self._e, int(nsteps), us.ctypes.data_as(C.POINTER(C.c_double))))
-        return {self.L.xbg_ens_kernel_name(k).decode(): float(us[k]) for k in range(12)}
+        return {self.L.xbg_ens_kernel_name(k).decode(): float(us[k]) for k in range(13)}
 
     # -- wave-group window means (surrogate training samples) ----------------
     def window_enable(self) -> int:
