@@ -195,7 +195,7 @@ XM_FN double sinh(double x) {
         const double u = dbl((uint64_t)(k + 1022) << 52), v = dbl((uint64_t)(1022 - k) << 52);  // 2^(k-1), 2^(-k-1)
         y = fma_(c, u - v, s * (u + v));
     }
-    return x < 0.0 ? -y : y;
+    return __builtin_copysign(y, x);
 }
 
 // E / (E + 2), E = e^2a - 1 = 2^k (e^r - 1) + (2^k - 1)
@@ -208,7 +208,7 @@ XM_FN double tanh(double x) {
     const double p = r + fma_(r * r, exp_q(r), (hi - r) - lo), u = dbl((uint64_t)(k + 1023) << 52);
     const double E = fma_(u, p, u - 1.0);
     const double y = E / (E + 2.0);
-    return x < 0.0 ? -y : y;
+    return __builtin_copysign(y, x);
 }
 
 XM_FN double ksin(double r) {
