@@ -816,8 +816,9 @@ XDEV float wave_sweep(WaveLds<A, CUR>& L, const KP& p, const SP& s, const Fld& f
             asm volatile("" : "+v"(ra[th - 2]) : : "memory");
         }
         if (th >= 1 && !bin) {  // the last bin: nothing leaves through its upper face
-            const float te = div(0.0f - fle, p.rdtheta, p.dtheta, p.dth_recip);
-            const float tr = div(0.0f - flr, p.rdtheta, p.dtheta, p.dth_recip);
+            float te = div(0.0f - fle, p.rdtheta, p.dtheta, p.dth_recip);
+            float tr = div(0.0f - flr, p.rdtheta, p.dtheta, p.dth_recip);
+            if (FLEX && nt <= 1) te = tr = 0.0f;  // a single bin may have width 0
             L.stash[th - 1][tid] = e1 - dt * (xe1 + te);
             ra[th - 1] = r1 - dt * (xr1 + tr);
         }
