@@ -86,11 +86,8 @@ struct Fld {
     float *Sus, *Svs, *C_out, *hh_b, *zb_b, *stdep_b, *ceqsg;
     double* zb64_b;
     float* zbc_b;
-    // per-block partial minima of the CFL reductions
-    float *red_wave, *red_flow;
+    float* red_wave;  // CFL minima of the wave kernel's tiles
     float* ua;        // Rvr's ua of each cell, formed by k_flow_uvvu for k_sed_flux
-    int* red_bad;
-    unsigned* red_acc;  // two halves of {flow min bits, wave min bits, flag}
     double* red_sum;
 };
 
@@ -2441,7 +2438,7 @@ struct xbg_ctx {
     // xbg_state_save: a device copy of every allocation and the host-side
     // buffer parities and boundary scalars
     std::vector<void*> snap;
-    int snap_cur = 0, snap_ccur = 0, snap_zcur = 0, snap_acc = 0;
+    int snap_cur = 0, snap_ccur = 0, snap_zcur = 0;
     float snap_sc[7] = {};
     bool snap_valid = false;
     Fld f;
@@ -2465,7 +2462,7 @@ struct xbg_ctx {
     float *Hmean = nullptr, *uumean = nullptr, *vvmean = nullptr, *hhmean = nullptr, *zsmean = nullptr,
           *zsmax = nullptr, *Cmean = nullptr;
     float Trep = 10.0f, tsl = 0.0f, tnext = 1.0f, zsbndi = 0.0f, zsbndn = 0.0f, windu = 0.0f, windv = 0.0f;
-    int nblk_wave = 0, nblk_flow = 0, nblk_sum = 0, acc_cur = 0;
+    int nblk_wave = 0, nblk_sum = 0;
     bool pre_disp = false;  // the coming step's dispersion is already queued (xbg_advance_resident)
     float* host_red = nullptr;
     double* host_sum = nullptr;
@@ -2791,9 +2788,8 @@ int xbg_create(const xbg_params* pin, xbg_ctx** out) {
     A(&f.wet, N);
     if (P.zb_accum == 2) { A(&f.zb64, N); A(&f.zb64_b, N); }
     c->nblk_wave = c->kp.wtiles_x * c->kp.wtiles_y;
-    c->nblk_flow = (int)((N + 255) / 256);
     c->nblk_sum = 256;
-    A(&f.red_wave, c->nblk_wave); A(&f.red_flow, c->nblk_flow); A(&f.red_bad, 4); A(&f.red_acc, 8);
+    A(&f.red_wave, c->nblk_wave);
     A(&f.red_sum, 2 * c->nblk_sum);
 #undef A
     e = hipHostMalloc((void**)&c->host_red, 2 * CFL_PARTS * sizeof(float), hipHostMallocDefault);
@@ -2895,11 +2891,6 @@ int xbg_init_state(xbg_ctx* c, double Trep) {
     // the first step's wave CFL minimum is not used (totaltime == 0)
     dim3 g1((c->nblk_wave + 255) / 256);
     LAUNCH(c, "k_fill", k_fill, g1, dim3(256), c->f.red_wave, (size_t)c->nblk_wave, 9999999.9f);
-    {
-        unsigned h[8] = {0x7f7fffffu, 0x7f7fffffu, 0u, 0u, 0x7f7fffffu, 0x7f7fffffu, 0u, 0u};
-        HIPC(c, hipMemcpyAsync(c->f.red_acc, h, sizeof(h), hipMemcpyHostToDevice, c->stream));
-        HIPC(c, hipStreamSynchronize(c->stream));
-    }
     HIPC(c, hipStreamSynchronize(c->stream));
     return XBG_OK;
 }
@@ -2952,7 +2943,6 @@ int xbg_state_save(xbg_ctx* c) {
     c->snap_cur = c->cur;
     c->snap_ccur = c->ccur;
     c->snap_zcur = c->zcur;
-    c->snap_acc = c->acc_cur;
     const float sc[7] = {c->Trep, c->tsl, c->tnext, c->zsbndi, c->zsbndn, c->windu, c->windv};
     std::memcpy(c->snap_sc, sc, sizeof(sc));
     c->snap_f = c->f;
@@ -2968,7 +2958,6 @@ int xbg_state_restore(xbg_ctx* c) {
     c->cur = c->snap_cur;
     c->ccur = c->snap_ccur;
     c->zcur = c->snap_zcur;
-    c->acc_cur = c->snap_acc;
     c->Trep = c->snap_sc[0];
     c->tsl = c->snap_sc[1];
     c->tnext = c->snap_sc[2];
@@ -3205,7 +3194,7 @@ int xbg_step(xbg_ctx* c, double dt, double totaltime) {
 namespace {
 // The CFL partial minima, written to pinned host memory by the kernel itself
 // (a copy behind it is one more launch the host waits for: 17.2 against
-// 14.9 us from call to dt on an idle queue), queued; *nb partial pairs.
+// 15.1 us from call to dt on an idle queue), queued; *nb partial pairs.
 int cfl_launch(xbg_ctx* c, int initial, int* nb_out) {
     float cfl = initial ? 0.5f * c->kp.CFL : c->kp.CFL;
     // about 8 cells per thread, at most CFL_PARTS workgroups
@@ -3231,8 +3220,8 @@ int xbg_cfl_dt(xbg_ctx* c, int initial, double* dt_flow, double* dt_wave) {
 
 namespace {
 int cfl_collect(xbg_ctx* c, int nb, double* dt_flow, double* dt_wave) {
-    // the step cannot be launched before dt is known: poll for the copy
-    // rather than block, so the next launches go out as soon as it lands
+    // the step cannot be launched before dt is known: poll for the kernel
+    // rather than block, so the next launches go out as soon as it ends
     hipError_t q;
     while ((q = hipEventQuery(c->cfl_done)) == hipErrorNotReady) {
     }
@@ -3609,26 +3598,23 @@ struct TileEnt {
 typedef const DomDesc* __restrict__ DTab;
 typedef const TileEnt* __restrict__ TMap;
 
-// One workgroup per tile of the map.  A loop over the map (persistent
+// Each kernel takes one workgroup per tile of its map.  A loop over the map (persistent
 // workgroups) was never faster, and the compiler moved the bodies' double
 // constants out of it into 50 to 80 registers: half the wavefronts per SIMD
 // (an ensemble of 48 domains 3.59 -> 3.40 ms per step without the loop).
-#define ENS_FOR_TILES(map, ntiles) if (const int t_ = blockIdx.x; t_ < (ntiles))
 
 template <int QW, int QH>
-__global__ __launch_bounds__(256) void kb_dispersion(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) dispersion_body<QW, QH>(D.p, D.s, D.f[D.par][PH_START], 1, BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_dispersion(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) dispersion_body<QW, QH>(D.p, D.s, D.f[D.par][PH_START], 1, BI{e.bx, e.by});
 }
 
 // Entries with bx < 0 pad a domain's run of tiles to a multiple of 8 (so
 // that map position modulo 8, the XCD of the workgroup, is the XCD the
 // single-domain launch gives the tile) and are skipped.
 template <int A, bool EX, bool CUR, bool FLEX>
-__global__ __launch_bounds__(WTHREADS, wave_occ(A)) void kb_wave(DTab tab, TMap map, int ntiles) {
+__global__ __launch_bounds__(WTHREADS, wave_occ(A)) void kb_wave(DTab tab, TMap map) {
     const TileEnt e = map[blockIdx.x];
     if (e.bx < 0) return;
     const DomDesc& D = tab[e.dom];
@@ -3638,121 +3624,101 @@ __global__ __launch_bounds__(WTHREADS, wave_occ(A)) void kb_wave(DTab tab, TMap 
     }
 }
 
-__global__ __launch_bounds__(256) void kb_flow_nuh(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) flow_nuh_body(D.p, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_flow_nuh(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) flow_nuh_body(D.p, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(256) void kb_flow_u(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) flow_u_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_flow_u(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) flow_u_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(256) void kb_flow_v(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) flow_v_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_flow_v(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) flow_v_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(BX * CY) void kb_flow_uvcorr(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) flow_uvcorr_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(BX * CY) void kb_flow_uvcorr(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) flow_uvcorr_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(BX * CY) void kb_flow_zsall(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) flow_zsall_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(BX * CY) void kb_flow_zsall(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) flow_zsall_body(D.p, D.s, D.f[D.par][PH_WAVE], BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(256) void kb_flow_uvvu(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) flow_uvvu_body(D.p, D.s, D.f[D.par][PH_ZS], D.sed, BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_flow_uvvu(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) flow_uvvu_body(D.p, D.s, D.f[D.par][PH_ZS], D.sed, BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(256) void kb_sed_flux(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE && D.sed) sed_flux_body(D.p, D.s, D.f[D.par][PH_ZS], 1, BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_sed_flux(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE && D.sed) sed_flux_body(D.p, D.s, D.f[D.par][PH_ZS], 1, BI{e.bx, e.by});
 }
 
 template <int QW, int QH>
-__global__ __launch_bounds__(256) void kb_sed_conc(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE && D.sed)
-            sed_conc_body<QW, QH>(D.p, D.s, D.f[D.par][PH_ZS], D.morph, BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_sed_conc(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE && D.sed)
+        sed_conc_body<QW, QH>(D.p, D.s, D.f[D.par][PH_ZS], D.morph, BI{e.bx, e.by});
 }
 
-__global__ __launch_bounds__(256) void kb_sed_morph(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE && D.sed && D.morph)
-            sed_morph_body(D.p, D.s, D.f[D.par][PH_END], BI{e.bx, e.by});
-    }
+__global__ __launch_bounds__(256) void kb_sed_morph(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE && D.sed && D.morph)
+        sed_morph_body(D.p, D.s, D.f[D.par][PH_END], BI{e.bx, e.by});
 }
 
 // FLOWDT (Wave_kernel.cu:161-170) of the state at step start, one partial
 // minimum per tile of 2048 cells (NaN when a cell gives a non-finite or
 // zero step), written to part[tile].
 constexpr int CFL_TILE = 2048;
-__global__ __launch_bounds__(256) void kb_cfl(DTab tab, TMap map, int ntiles, float* part) {
+__global__ __launch_bounds__(256) void kb_cfl(DTab tab, TMap map, float* part) {
     __shared__ float rf[4];
     __shared__ int rb[4];
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        if (D.status == ENS_ACTIVE) {
-            const KP& p = D.p;
-            const float* hh = D.f[D.par][PH_END].hh;
-            const size_t b0 = (size_t)e.bx * CFL_TILE + threadIdx.x;
-            float h[CFL_TILE / 256];
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    if (D.status == ENS_ACTIVE) {
+        const KP& p = D.p;
+        const float* hh = D.f[D.par][PH_END].hh;
+        const size_t b0 = (size_t)e.bx * CFL_TILE + threadIdx.x;
+        float h[CFL_TILE / 256];
 #pragma unroll
-            for (int k = 0; k < CFL_TILE / 256; k++) {
-                size_t i = b0 + (size_t)k * 256;
-                h[k] = i < p.N ? hh[i] : 0.0f;
-            }
-            float v = 3.0e38f;
-            int bad = 0;
+        for (int k = 0; k < CFL_TILE / 256; k++) {
+            size_t i = b0 + (size_t)k * 256;
+            h[k] = i < p.N ? hh[i] : 0.0f;
+        }
+        float v = 3.0e38f;
+        int bad = 0;
 #pragma unroll
-            for (int k = 0; k < CFL_TILE / 256; k++) {
-                if (b0 + (size_t)k * 256 >= p.N) continue;
-                float d = p.CFL * p.dx / (sqrtf(9.81f * h[k]));
-                if (!(d == d) || d == INFINITY || d == 0.0f) bad = 1;
-                else v = fmn(v, d);
-            }
-            for (int o = 32; o > 0; o >>= 1) v = fmn(v, __shfl_xor(v, o, 64));
-            bad = __any(bad);
-            if ((threadIdx.x & 63) == 0) {
-                rf[threadIdx.x >> 6] = v;
-                rb[threadIdx.x >> 6] = bad;
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                v = fmn(fmn(rf[0], rf[1]), fmn(rf[2], rf[3]));
-                part[t_] = (rb[0] | rb[1] | rb[2] | rb[3]) ? __builtin_nanf("") : v;
-            }
+        for (int k = 0; k < CFL_TILE / 256; k++) {
+            if (b0 + (size_t)k * 256 >= p.N) continue;
+            float d = p.CFL * p.dx / (sqrtf(9.81f * h[k]));
+            if (!(d == d) || d == INFINITY || d == 0.0f) bad = 1;
+            else v = fmn(v, d);
+        }
+        for (int o = 32; o > 0; o >>= 1) v = fmn(v, __shfl_xor(v, o, 64));
+        bad = __any(bad);
+        if ((threadIdx.x & 63) == 0) {
+            rf[threadIdx.x >> 6] = v;
+            rb[threadIdx.x >> 6] = bad;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            v = fmn(fmn(rf[0], rf[1]), fmn(rf[2], rf[3]));
+            part[blockIdx.x] = (rb[0] | rb[1] | rb[2] | rb[3]) ? __builtin_nanf("") : v;
         }
     }
 }
@@ -3885,49 +3851,45 @@ __global__ __launch_bounds__(256) void k_ens_dt(DomDesc* tab, const float* part)
 // predicts (H, Dw, DR, Fx, Fy), after a step: the state after the last step
 // is the start state of the other parity.
 constexpr int WIN_F = 8;
-__global__ __launch_bounds__(256) void kb_window_add(DTab tab, TMap map, int ntiles) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        const BI bi{e.bx, e.by};
-        const int x = gx(bi), y = gy(bi);
-        if (D.win && x < D.p.nx && y < D.p.ny) {
-            const Fld& f = D.f[D.par ^ 1][PH_START];
-            const size_t i = (size_t)x + (size_t)y * D.p.nx, N = D.p.N;
-            float* w = D.win;
-            w[i] += G(f.zs)[i];
-            w[N + i] += G(f.uu)[i];
-            w[2 * N + i] += G(f.vv)[i];
-            w[3 * N + i] += G(f.H)[i];
-            w[4 * N + i] += G(f.Dw)[i];
-            w[5 * N + i] += G(f.DR)[i];
-            w[6 * N + i] += G(f.Fx)[i];
-            w[7 * N + i] += G(f.Fy)[i];
-        }
+__global__ __launch_bounds__(256) void kb_window_add(DTab tab, TMap map) {
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    const BI bi{e.bx, e.by};
+    const int x = gx(bi), y = gy(bi);
+    if (D.win && x < D.p.nx && y < D.p.ny) {
+        const Fld& f = D.f[D.par ^ 1][PH_START];
+        const size_t i = (size_t)x + (size_t)y * D.p.nx, N = D.p.N;
+        float* w = D.win;
+        w[i] += G(f.zs)[i];
+        w[N + i] += G(f.uu)[i];
+        w[2 * N + i] += G(f.vv)[i];
+        w[3 * N + i] += G(f.H)[i];
+        w[4 * N + i] += G(f.Dw)[i];
+        w[5 * N + i] += G(f.DR)[i];
+        w[6 * N + i] += G(f.Fx)[i];
+        w[7 * N + i] += G(f.Fy)[i];
     }
 }
 
 // Window means as surrogate samples: out[wout + i*12 + c] for the channels
 // zb, zs, uu, vv, Hm0, Tp, dir (from meta[3*d..]), H, Dw, DR, Fx, Fy; the
 // sums restart at zero.
-__global__ __launch_bounds__(256) void kb_window_sample(DTab tab, TMap map, int ntiles, float inv,
+__global__ __launch_bounds__(256) void kb_window_sample(DTab tab, TMap map, float inv,
                                                         const float* __restrict__ meta, float* __restrict__ out) {
-    ENS_FOR_TILES(map, ntiles) {
-        const TileEnt e = map[t_];
-        const DomDesc& D = tab[e.dom];
-        const BI bi{e.bx, e.by};
-        const int x = gx(bi), y = gy(bi);
-        if (D.win && x < D.p.nx && y < D.p.ny) {
-            const Fld& f = D.f[D.par ^ 1][PH_START];
-            const size_t i = (size_t)x + (size_t)y * D.p.nx, N = D.p.N;
-            float* w = D.win;
-            float* o = out + D.wout + i * 12;
-            o[0] = G(f.zb)[i];
-            for (int k = 0; k < 3; k++) o[1 + k] = w[k * N + i] * inv;
-            for (int k = 0; k < 3; k++) o[4 + k] = meta[3 * e.dom + k];
-            for (int k = 3; k < WIN_F; k++) o[4 + k] = w[k * N + i] * inv;
-            for (int k = 0; k < WIN_F; k++) w[k * N + i] = 0.0f;
-        }
+    const TileEnt e = map[blockIdx.x];
+    const DomDesc& D = tab[e.dom];
+    const BI bi{e.bx, e.by};
+    const int x = gx(bi), y = gy(bi);
+    if (D.win && x < D.p.nx && y < D.p.ny) {
+        const Fld& f = D.f[D.par ^ 1][PH_START];
+        const size_t i = (size_t)x + (size_t)y * D.p.nx, N = D.p.N;
+        float* w = D.win;
+        float* o = out + D.wout + i * 12;
+        o[0] = G(f.zb)[i];
+        for (int k = 0; k < 3; k++) o[1 + k] = w[k * N + i] * inv;
+        for (int k = 0; k < 3; k++) o[4 + k] = meta[3 * e.dom + k];
+        for (int k = 3; k < WIN_F; k++) o[4 + k] = w[k * N + i] * inv;
+        for (int k = 0; k < WIN_F; k++) w[k * N + i] = 0.0f;
     }
 }
 
@@ -4040,7 +4002,7 @@ int ens_launch_step(xbg_ens* e) {
     const dim3 b2(BX, BY), bc(BX, CY);
     if (e->m_cfl.n) {
         ens_ev(e, 2 * EK_CFL);
-        kb_cfl<<<dim3(e->m_cfl.n), dim3(256), 0, e->stream>>>(e->dtab, e->m_cfl.d, e->m_cfl.n, e->part);
+        kb_cfl<<<dim3(e->m_cfl.n), dim3(256), 0, e->stream>>>(e->dtab, e->m_cfl.d, e->part);
         ens_ev(e, 2 * EK_CFL + 1);
     }
     k_ens_dt<<<dim3(e->nd), dim3(256), 0, e->stream>>>(e->dtab, e->part);
@@ -4048,16 +4010,16 @@ int ens_launch_step(xbg_ens* e) {
         const TileMap& m = e->m_disp[e->disp_shape];
         ens_ev(e, 2 * EK_DISP);
         switch (e->disp_shape) {
-            case 0: kb_dispersion<4, 16><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            case 1: kb_dispersion<8, 8><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            default: kb_dispersion<16, 4><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            case 0: kb_dispersion<4, 16><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d); break;
+            case 1: kb_dispersion<8, 8><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d); break;
+            default: kb_dispersion<16, 4><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d); break;
         }
         ens_ev(e, 2 * EK_DISP + 1);
     }
     ens_ev(e, 2 * EK_WAVE);
     for (const WaveGroup& w : e->waves) {
 #define RUN(A_, EX_, C_, F_) \
-    kb_wave<A_, EX_, C_, F_><<<dim3(w.map.n), dim3(BX, WTY), 0, e->stream>>>(e->dtab, w.map.d, w.map.n)
+    kb_wave<A_, EX_, C_, F_><<<dim3(w.map.n), dim3(BX, WTY), 0, e->stream>>>(e->dtab, w.map.d)
         WAVE_SWITCH(w.k, RUN);
 #undef RUN
     }
@@ -4067,7 +4029,7 @@ int ens_launch_step(xbg_ens* e) {
 #define EL(k, kern, blk, m)                                                                                 \
     do {                                                                                                    \
         ens_ev(e, 2 * (k));                                                                                 \
-        kern<<<dim3((m).n), blk, 0, e->stream>>>(e->dtab, (m).d, (m).n);                                    \
+        kern<<<dim3((m).n), blk, 0, e->stream>>>(e->dtab, (m).d);                                           \
         ens_ev(e, 2 * (k) + 1);                                                                             \
     } while (0)
     EL(EK_NUH, kb_flow_nuh, b2, m2);
@@ -4081,9 +4043,9 @@ int ens_launch_step(xbg_ens* e) {
         const TileMap& m = e->m_conc[e->conc_shape];
         ens_ev(e, 2 * EK_SCONC);
         switch (e->conc_shape) {
-            case 0: kb_sed_conc<4, 16><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            case 1: kb_sed_conc<8, 8><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
-            default: kb_sed_conc<16, 4><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d, m.n); break;
+            case 0: kb_sed_conc<4, 16><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d); break;
+            case 1: kb_sed_conc<8, 8><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d); break;
+            default: kb_sed_conc<16, 4><<<dim3(m.n), b2, 0, e->stream>>>(e->dtab, m.d); break;
         }
         ens_ev(e, 2 * EK_SCONC + 1);
     }
@@ -4377,7 +4339,7 @@ int xbg_ens_window_enable(xbg_ens* e, size_t* sample_floats) {
 
 int xbg_ens_window_add(xbg_ens* e) {
     if (!e) return XBG_E_ARG;
-    kb_window_add<<<dim3(e->m_2d.n), dim3(BX, BY), 0, e->stream>>>(e->dtab, e->m_2d.d, e->m_2d.n);
+    kb_window_add<<<dim3(e->m_2d.n), dim3(BX, BY), 0, e->stream>>>(e->dtab, e->m_2d.d);
     EHIP(e, hipGetLastError());
     return XBG_OK;
 }
@@ -4387,7 +4349,7 @@ int xbg_ens_window_sample(xbg_ens* e, int count, const float* meta, float* out) 
     float* dm = nullptr;
     EHIP(e, hipMallocAsync((void**)&dm, 3 * sizeof(float) * e->nd, e->stream));
     EHIP(e, hipMemcpyAsync(dm, meta, 3 * sizeof(float) * e->nd, hipMemcpyHostToDevice, e->stream));
-    kb_window_sample<<<dim3(e->m_2d.n), dim3(BX, BY), 0, e->stream>>>(e->dtab, e->m_2d.d, e->m_2d.n, 1.0f / count,
+    kb_window_sample<<<dim3(e->m_2d.n), dim3(BX, BY), 0, e->stream>>>(e->dtab, e->m_2d.d, 1.0f / count,
                                                                      dm, out);
     EHIP(e, hipGetLastError());
     EHIP(e, hipFreeAsync(dm, e->stream));

@@ -71,7 +71,7 @@ constexpr int LROW = KB + 8;  // LDS row (pixel) stride in bf16: 80 B, keeps 16-
 // neighbouring pixels can be combined:
 //   E_STORE   store, 0 where mask <= 0 when a mask is given
 //   E_POOL    store, and the 2x2 average pool of the stored values
-//   E_HEAD    store (when y is given), and the output head on the stored values
+//   E_HEAD    store, and the output head on the stored values
 //   E_UPSUM   data gradient of a concatenation: channels below c1 summed over
 //             the 2x2 cells of the upsampled part, the others stored as they are
 //   E_UNPOOL  data gradient of a pooled tensor: a quarter of the value added
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256, 2) void k_conv(CSrc X, const bf16* __restrict_
     const size_t img = (size_t)n * H * W;
     auto at = [&](int px, int ch) { return *(const bf16x8*)(sm + px * LO + ch * 8); };
     auto pixel = [&](int px) { return img + (size_t)(y0 + px / TW) * W + x0 + px % TW; };
-    if (EPI == E_STORE || EPI == E_POOL || (EPI == E_HEAD && E.y)) {
+    if (EPI == E_STORE || EPI == E_POOL || EPI == E_HEAD) {
 #pragma unroll
         for (int it = 0; it < 64 * MB * CH / 256; it++) {
             const int i = tid + it * 256, px = i / CH, ch = i % CH;
