@@ -3598,10 +3598,10 @@ struct TileEnt {
 typedef const DomDesc* __restrict__ DTab;
 typedef const TileEnt* __restrict__ TMap;
 
-// Each kernel takes one workgroup per tile of its map.  A loop over the map (persistent
-// workgroups) was never faster, and the compiler moved the bodies' double
-// constants out of it into 50 to 80 registers: half the wavefronts per SIMD
-// (an ensemble of 48 domains 3.59 -> 3.40 ms per step without the loop).
+// Each kernel takes one workgroup per tile of its map.  A loop over the map
+// (persistent workgroups) was never faster, and the compiler moved the bodies'
+// double constants out of it into 50 to 80 registers: half the wavefronts per
+// SIMD (an ensemble of 48 domains 3.59 -> 3.40 ms per step without the loop).
 
 template <int QW, int QH>
 __global__ __launch_bounds__(256) void kb_dispersion(DTab tab, TMap map) {

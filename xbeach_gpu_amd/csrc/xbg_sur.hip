@@ -332,7 +332,7 @@ __global__ __launch_bounds__(256, 2) void k_conv(CSrc X, const bf16* __restrict_
 //
 // Bound by the LDS reads and the matrix rate at 64 channels, by memory at 32.
 // At 64 x 256 x 256 the 17 layers' weight and bias gradients and their
-// reductions take 1.8 ms, and took 8.2 ms before (one copy of X per shift,
+// reductions take 1.9 ms, and took 8.2 ms before (one copy of X per shift,
 // transposed in registers, every X row read three times; bias sums in a pass
 // of their own).
 // Requires Cout % CBO == 0, Cin % CBI == 0; W % SEG == 0 unless RAGGED, whose
